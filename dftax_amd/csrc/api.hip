@@ -44,6 +44,9 @@ hipError_t launch_eri_cls(int la, int lb, int lc, const int2* pairs, int npair, 
 hipError_t launch_eri_thread(int la, int lb, int lc, const int2* pairs, int npair, const int32_t* aux, int naux_l,
                              const ShellSet& A, const ShellSet& C, const double* boys, double* out, int64_t sa,
                              int64_t sb, int64_t c0, int tr, hipStream_t st);
+hipError_t launch_eri_pair(int la, int lb, int lc, const int2* pairs, int npair, const int32_t* aux, int naux_l,
+                           const ShellSet& A, const ShellSet& C, const double* boys, double* out, int64_t sa,
+                           int64_t sb, int64_t c0, int tr, hipStream_t st);
 hipError_t launch_int1e(const ShellSet& A, int natm, const double* atm, const double* boys, double* S, double* T,
                         double* V, int64_t nao, hipStream_t stream);
 hipError_t launch_becke(int64_t n, const double* pts, const double* raw, const int32_t* owner, int natm,
@@ -736,6 +739,21 @@ void setup_pairs(dfks_ctx* h, const std::vector<std::vector<int2>>& pairs, const
   sync(st);  // kept lives on the host until the copy is done
 }
 
+// One class of (mn|P): a thread per task in the low classes (registers only), a workgroup per bra pair
+// (H G on the matrix cores) in the others, and a wavefront per task where a span is cartesian with l >= 2.
+// The line between the first two is where the unrolled thread still fits its registers: on those 19 classes
+// it takes 12.7 ms for (H2O)_24 def2-TZVP against 18.4 ms by bra pair, whose 16-row tiles they leave mostly
+// empty ((ss|s): 0.5 against 1.4 ms; (pp|d): 0.82 against 0.87 ms).
+hipError_t launch_eri3(int la, int lb, int lc, const int2* pairs, int npair, const int32_t* aux, int naux_l,
+                       const ShellSet& A, const ShellSet& C, const double* boys, double* out, int64_t sa, int64_t sb,
+                       int64_t c0, int tr, hipStream_t st) {
+  if (C.spherical && eri_thread_has(la, lb, lc))
+    return launch_eri_thread(la, lb, lc, pairs, npair, aux, naux_l, A, C, boys, out, sa, sb, c0, tr, st);
+  if (C.spherical && (A.spherical || la < 2))
+    return launch_eri_pair(la, lb, lc, pairs, npair, aux, naux_l, A, C, boys, out, sa, sb, c0, tr, st);
+  return launch_eri_cls(la, lb, lc, pairs, npair, aux, naux_l, A, C, boys, out, sa, sb, c0, tr, st);
+}
+
 // Recompute mode: auxiliary slabs (runs of whole shells of at most aux_chunk
 // functions) with their per-lc shell lists, and the slab-sized buffers.
 void setup_slabs(dfks_ctx* h, hipStream_t st) {
@@ -1193,12 +1211,8 @@ void build_all(dfks_ctx* h, hipStream_t st) {
           const int cls = la * (lo + 1) + lb;
           const int2* pp = h->d_pairs3 + h->pair3_off[cls];
           const int npair = h->pair3_n[cls];
-          if (eri_thread_has(la, lb, lc) && A.spherical)
-            HIPCHK(launch_eri_thread(la, lb, lc, pp, npair, d_auxl + aux_off[lc], (int)auxl[lc].size(), O, A,
-                                     h->d_boys, d3, (int64_t)nao * naux, naux, 0, 1, st));
-          else
-            HIPCHK(launch_eri_cls(la, lb, lc, pp, npair, d_auxl + aux_off[lc], (int)auxl[lc].size(), O, A,
-                                  h->d_boys, d3, (int64_t)nao * naux, naux, 0, 1, st));
+          HIPCHK(launch_eri3(la, lb, lc, pp, npair, d_auxl + aux_off[lc], (int)auxl[lc].size(), O, A, h->d_boys, d3,
+                             (int64_t)nao * naux, naux, 0, 1, st));
         }
     sync(st);
   } else {
@@ -1262,12 +1276,8 @@ void build_all(dfks_ctx* h, hipStream_t st) {
           const int cls = la * (lo + 1) + lb;
           const int2* pp = h->d_pairs3 + h->pair3_off[cls];
           const int npair = h->pair3_n[cls];
-          if (eri_thread_has(la, lb, lc) && A.spherical)
-            HIPCHK(launch_eri_thread(la, lb, lc, pp, npair, d_auxl + aux_off[lc], (int)auxl[lc].size(), O, Aw,
-                                     h->d_boys, d3lr, (int64_t)nao * naux, naux, 0, 1, st));
-          else
-            HIPCHK(launch_eri_cls(la, lb, lc, pp, npair, d_auxl + aux_off[lc], (int)auxl[lc].size(), O, Aw,
-                                  h->d_boys, d3lr, (int64_t)nao * naux, naux, 0, 1, st));
+          HIPCHK(launch_eri3(la, lb, lc, pp, npair, d_auxl + aux_off[lc], (int)auxl[lc].size(), O, Aw, h->d_boys,
+                             d3lr, (int64_t)nao * naux, naux, 0, 1, st));
         }
     sync(st);
     eig_launch(d2lr, h->rb, st);
@@ -1376,10 +1386,7 @@ void eri_slab(dfks_ctx* h, int s, hipStream_t st) {
         const int nal = h->slab_aux_n[sl];
         if (nal == 0) continue;
         const int32_t* aa = h->d_slab_aux + h->slab_aux_off[sl];
-        if (eri_thread_has(la, lb, lc) && A.spherical)
-          HIPCHK(launch_eri_thread(la, lb, lc, pp, npair, aa, nal, O, A, h->d_boys, h->d_slab, sa, sb, p0, 1, st));
-        else
-          HIPCHK(launch_eri_cls(la, lb, lc, pp, npair, aa, nal, O, A, h->d_boys, h->d_slab, sa, sb, p0, 1, st));
+        HIPCHK(launch_eri3(la, lb, lc, pp, npair, aa, nal, O, A, h->d_boys, h->d_slab, sa, sb, p0, 1, st));
       }
     }
 }

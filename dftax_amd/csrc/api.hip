@@ -96,6 +96,15 @@ hipError_t launch_xcf_all(const XcfBin* tab, int nbins, int ztot, int ptot, int 
                           const int32_t* cols, const float* P, int64_t nao, const double* w, int xc_id, double thresh,
                           double* exc, double* part, float* coef, float* q, hipStream_t st);
 void xcf_bin_geometry(int n, int nb, int& nt, int& nks, int64_t& part_doubles, int64_t& coef_floats);
+hipError_t launch_xcb_rho(const XcBlock* blks, const int32_t* wgs, int nwg, const double* ao, const int32_t* cols,
+                          const double* P, int64_t nao, double* part, hipStream_t st);
+hipError_t launch_xcb_v(const XcBlock* blks, const int32_t* wgs, int nwg, const double* ao, const double* coef,
+                        double* q, hipStream_t st);
+hipError_t launch_xcb_point(int mode, int nblk, const XcBlock* blks, const double* part, const double* w,
+                            const double* rec, int xc_id, double thresh, double* exc, double* out, hipStream_t st);
+hipError_t launch_xcb_point_pol(int nblk, const XcBlock* blks, const double* parta, const double* partb,
+                                const double* w, int xc_id, double thresh, double* exc, double* outa, double* outb,
+                                hipStream_t st);
 hipError_t launch_xc_f32(int64_t ng, int64_t nao, const float* ao, const double* w, float* zw, int xc_id,
                          double thresh, double* exc, hipStream_t st);
 hipError_t launch_gamma_f32(int nao, int nq, int nf, const float* T, const double* Cf, const double* sgn,
@@ -138,8 +147,6 @@ hipError_t launch_gemm(int prec, const GemmArgs& g, double* C, double alpha, dou
 hipError_t launch_gemm_f32out(const GemmArgs& g, float* C, hipStream_t st);
 hipError_t launch_gemm_f32out_batched(const GemmArgs& g, float* C, int batch, int64_t bs_a, int64_t bs_b,
                                       int64_t bs_c, hipStream_t st);
-hipError_t launch_gemm_f64_batched(const GemmArgs& g, double* C, int batch, int64_t bs_a, int64_t bs_b,
-                                   int64_t bs_c, hipStream_t st);
 hipError_t launch_gemm_w8(const GemmArgs& g, double* C, const RowDot& rd, hipStream_t st);
 hipError_t launch_gemm_b3w8(const GemmArgs& g, float* C, const RowDot& rd, hipStream_t st, int depth);
 hipError_t launch_colsum(int nrows, int ncols, const double* part, double* out, int accumulate, hipStream_t st);
@@ -579,6 +586,13 @@ struct dfks_ctx {
   bool xcb = false;
   std::vector<XcBin> xbins;
   int64_t xc_npts = 0, xc_zw = 0, xc_nblk = 0, xc_qtot = 0;
+  // the blocks up to kXfMaxN wide for the one-launch FP64 kernels: descriptors (widest block first),
+  // workgroup ids, the strips' partial sums and the W coefficients (a second pair for nspin = 2)
+  int xk_nblk = 0, xk_nwg = 0;
+  int64_t xk_nparts = 0;
+  XcBlock* d_xk_blk = nullptr;
+  int32_t* d_xk_wg = nullptr;
+  double *d_xk_part[2] = {}, *d_xk_coef[2] = {};
   // the fused mixed-precision XC pass over all eligible bins at once: the bin table
   // (host copy kept for the upload), its device copy, the workspace, launch sizes
   std::vector<XcfBin> xcf_tab;
@@ -644,7 +658,8 @@ struct dfks_ctx {
                     d_fitd, d_aob, d_zwb, d_fxc, d_rho0, d_Rf, d_xc_pts, d_xc_w, d_xc_exc, d_xc_ao,
                     d_xc_zw, d_xc_q, d_xc_ao32, d_xc_cols, d_xc_vlen, d_xc_shl, d_xc_shoff, d_xc_vrow,
                     d_xc_vprow, d_xc_vpcol, d_xc_zw2, d_xc_q2, d_Vxc2, d_uP, d_uJ, d_uK, d_ug, d_xcf_tab,
-                    d_xcf_ws, d_Blr, d_Klr};
+                    d_xcf_ws, d_Blr, d_Klr, d_xk_blk, d_xk_wg, d_xk_part[0], d_xk_part[1], d_xk_coef[0],
+                    d_xk_coef[1]};
     for (void* p : ptrs) dfree(p);
     void* ptrs32[] = {d_gws, d_gpart, d_B32, d_ao32, d_zw32, t32_alias ? nullptr : d_T32, d_Cf32, d_P32, d_ws32,
                       d_eps32, d_offd32, d_slab32, d_Lt32, d_Tslab32, d_aob32, d_zwb32};
@@ -846,6 +861,12 @@ uint32_t spread3(uint32_t v) {  // 10 bits -> every third bit
 // padded count of their functions (multiples of 32). Uploads the binned points,
 // weights, column maps, shell lists and the row lists of the Vxc assembly, and
 // evaluates the compact AO values and gradients (resident).
+// Whether a bin's blocks go through the one-launch FP64 kernels (the others, and every bin with
+// gemm = rocblas, take rocBLAS batched products bin by bin)
+bool xc_one_launch(const dfks_ctx* h, const dfks_ctx::XcBin& bn) {
+  return h->opt.gemm != 1 && bn.n <= kXfMaxN && (int64_t)h->nao * h->nao <= 0x7fffffff;
+}
+
 void plan_xc_blocks(dfks_ctx* h, hipStream_t st) {
   const double tp0 = now_ms();
   const int64_t ng = h->ng;
@@ -933,10 +954,31 @@ void plan_xc_blocks(dfks_ctx* h, hipStream_t st) {
     ao_tot += 4 * bn.nblk * kXcG * bn.n;
     q_tot += bn.nblk * (int64_t)bn.n * bn.n;
     col_tot += bn.nblk * bn.n;
-    zw_max = std::max(zw_max, bn.nblk * kXcG * bn.n);
+    if (!xc_one_launch(h, bn)) zw_max = std::max(zw_max, bn.nblk * kXcG * bn.n);
     h->xbins.push_back(bn);
     i = j;
   }
+  // the one-launch kernels' descriptors, widest blocks first (the longest workgroups start first), and
+  // workgroup ids: 8 blocks at a time, strip by strip, so that a block's strips are 8 ids apart (-1: none)
+  std::vector<XcBlock> xk;
+  std::vector<int32_t> xw;
+  h->xk_nparts = 0;
+  for (auto bn = h->xbins.rbegin(); bn != h->xbins.rend(); ++bn) {
+    if (!xc_one_launch(h, *bn)) continue;
+    const int nt = (bn->n + 63) / 64;
+    for (int64_t k = 0; k < bn->nblk; ++k) {
+      xk.push_back({bn->ao_off + k * kXcG * bn->n, bn->nblk * kXcG * bn->n, bn->col_off + k * bn->n,
+                    bn->q_off + k * (int64_t)bn->n * bn->n, bn->pt0 + k * kXcG, h->xk_nparts, bn->n, 0});
+      h->xk_nparts += nt;
+    }
+  }
+  if (xk.size() > (size_t)0x7fffffff / kXcbStrips) fail(1, "compact XC grid too large for the one-launch kernels");
+  for (size_t b0 = 0; b0 < xk.size(); b0 += 8)
+    for (int t = 0; 64 * t < xk[b0].n; ++t)
+      for (size_t b = b0; b < b0 + 8; ++b)
+        xw.push_back(b < xk.size() && 64 * t < xk[b].n ? (int32_t)(b * kXcbStrips + t) : -1);
+  h->xk_nblk = (int)xk.size();
+  h->xk_nwg = (int)xw.size();
   const int64_t npts = nblk * kXcG;
   std::vector<double> pts((size_t)(3 * npts)), w((size_t)npts, 0.0);
   std::vector<int32_t> cols((size_t)col_tot, -1);
@@ -1012,7 +1054,13 @@ void plan_xc_blocks(dfks_ctx* h, hipStream_t st) {
   h->xc_zw = zw_max;
   h->xc_qtot = q_tot;
   h->d_xc_exc = dalloc<double>(npts);
-  h->d_xc_zw = dalloc<double>(zw_max);
+  if (zw_max > 0) h->d_xc_zw = dalloc<double>(zw_max);
+  if (!xk.empty()) {
+    h->d_xk_blk = up(xk);
+    h->d_xk_wg = up(xw);
+    h->d_xk_part[0] = dalloc<double>(h->xk_nparts * 4 * kXcG);
+    h->d_xk_coef[0] = dalloc<double>(4 * npts);
+  }
   h->d_xc_q = dalloc<double>(q_tot);
   h->d_xc_ao = dalloc<double>(ao_tot);
   const double tp4 = now_ms();
@@ -1447,8 +1495,6 @@ void coulomb_recompute(dfks_ctx* h, hipStream_t st) {
 // that shape. Both compute the same T to rounding.
 // Per-shape choice among the variants of a product. Tags and variants:
 //   0  FP64 exchange T = B^T C:      0 rocBLAS, 1 k_gemm, 2 k_gemm_w8
-//   1  FP64 XC Z_b = Phi_b Pg_b:     0 rocBLAS, 1 k_gemm (batched)
-//   2  FP64 XC Phi_b^T W_b:          0 rocBLAS, 1 k_gemm (batched)
 //   3  FP64 exchange K partials:     0 k_gemm, 1 k_gemm_w8, 2 k_gemm_w8 split by XCD (base 1)
 //   4  split-BF16 exchange T:        0 k_gemm, 1 k_gemm_b3w8 (base 1)
 //   5  SP2 product partials X X:     0 k_gemm, 1 k_gemm_w8   (base 1)
@@ -1676,10 +1722,11 @@ void jk_factored(dfks_ctx* h, const double* Cf, const std::vector<double>& sgn, 
   h->mark(kStCoulomb + 1, st);
 }
 
-// XC on the compact grid, bin by bin: Pg = P gathered to each block's columns,
-// Z_b = Phi_b Pg_b (batched), the pointwise kernel on the compact rows, then
-// prod_b = Phi_b^T W_b (batched, over Pg's storage) and the row assembly of
-// Vh = sum_b prod_b scattered to the blocks' columns.
+// XC on the compact grid: Z_b = Phi_b Pg_b (Pg = P at each block's columns)
+// reduced to rho and grad rho, the pointwise functional, prod_b = Phi_b^T W_b,
+// and the row assembly of Vh = sum_b prod_b scattered to the blocks' columns.
+// One launch each over all blocks (xc_blocks.hip; mixed: launch_xcf_all); with
+// gemm = rocblas, or wider than kXfMaxN, bin by bin on batched products.
 //   kXcEnergy:   k_xc, E_xc into E + DFKS_E_XC (FP64 or mixed)
 //   kXcRho:      rho0 and grad rho0 per padded point into d_rho0 (FP64, no Vh)
 //   kXcResponse: Z1 = Phi dP, the response kernel with the records in d_fxc (FP64)
@@ -1740,6 +1787,13 @@ void xc_compact(dfks_ctx* h, const double* P, double* E, int mode, hipStream_t s
                           h->d_xcf_ws, reinterpret_cast<float*>(h->d_xcf_ws + h->xcf_part),
                           reinterpret_cast<float*>(h->d_xc_q), st));
   }
+  if (!mixed && h->xk_nblk > 0) {
+    HIPCHK(launch_xcb_rho(h->d_xk_blk, h->d_xk_wg, h->xk_nwg, h->d_xc_ao, h->d_xc_cols, P, nao, h->d_xk_part[0], st));
+    HIPCHK(launch_xcb_point(mode, h->xk_nblk, h->d_xk_blk, h->d_xk_part[0], h->d_xc_w, h->d_fxc, h->xc_id, thresh,
+                            h->d_xc_exc, mode == kXcRho ? h->d_rho0 : h->d_xk_coef[0], st));
+    if (mode != kXcRho)
+      HIPCHK(launch_xcb_v(h->d_xk_blk, h->d_xk_wg, h->xk_nwg, h->d_xc_ao, h->d_xk_coef[0], h->d_xc_q, st));
+  }
   for (size_t bi = 0; bi < h->xbins.size(); ++bi) {
     if (fused && h->xcf_fused[bi]) continue;
     const auto& bn = h->xbins[bi];
@@ -1763,21 +1817,15 @@ void xc_compact(dfks_ctx* h, const double* P, double* E, int mode, hipStream_t s
                                           &zerof, q, n, (rocblas_stride)n * n, (int)nb));
       continue;
     }
+    if (xc_one_launch(h, bn)) continue;
     double* q = h->d_xc_q + bn.q_off;
     const double* ao = h->d_xc_ao + bn.ao_off;
     double* zw = h->d_xc_zw;
     HIPCHK((launch_gather_sym<double, double>(nb, n, cols, P, nao, q, st)));
     // Z_b (G x n, row-major) = Phi_b Pg_b; rocBLAS column-major: Z_b^T = Pg_b^T Phi_b^T
-    tuned_product(h, 1, n, nb, 0, 2, 0, [&](int choice) {
-      if (choice == 1) {
-        const GemmArgs g{kXcG, n, n, ao, n, true, q, n, true};
-        HIPCHK(launch_gemm_f64_batched(g, zw, (int)nb, (int64_t)kXcG * n, (int64_t)n * n, (int64_t)kXcG * n, st));
-      } else {
-        RBCHK(rocblas_dgemm_strided_batched(h->rb, rocblas_operation_transpose, rocblas_operation_none, n, kXcG, n,
-                                            &one, q, n, (rocblas_stride)n * n, ao, n, (rocblas_stride)kXcG * n, &zero,
-                                            zw, n, (rocblas_stride)kXcG * n, (int)nb));
-      }
-    }, st);
+    RBCHK(rocblas_dgemm_strided_batched(h->rb, rocblas_operation_transpose, rocblas_operation_none, n, kXcG, n, &one,
+                                        q, n, (rocblas_stride)n * n, ao, n, (rocblas_stride)kXcG * n, &zero, zw, n,
+                                        (rocblas_stride)kXcG * n, (int)nb));
     if (mode == kXcEnergy)
       HIPCHK(launch_xc(rows, n, ao, h->d_xc_w + bn.pt0, zw, h->xc_id, thresh, h->d_xc_exc + bn.pt0, nullptr, st));
     else if (mode == kXcRho)
@@ -1787,16 +1835,9 @@ void xc_compact(dfks_ctx* h, const double* P, double* E, int mode, hipStream_t s
       HIPCHK(launch_fxc(rows, n, ao, zw, h->d_fxc + 8 * bn.pt0, st));
     if (mode == kXcRho) continue;
     // prod_b[i][j] = sum_g Phi[g][i] W[g][j]; rocBLAS column-major: prod_b^T = W_b^T Phi_b
-    tuned_product(h, 2, n, nb, 0, 2, 0, [&](int choice) {
-      if (choice == 1) {
-        const GemmArgs g{n, n, kXcG, ao, n, false, zw, n, false};
-        HIPCHK(launch_gemm_f64_batched(g, q, (int)nb, (int64_t)kXcG * n, (int64_t)kXcG * n, (int64_t)n * n, st));
-      } else {
-        RBCHK(rocblas_dgemm_strided_batched(h->rb, rocblas_operation_none, rocblas_operation_transpose, n, n, kXcG,
-                                            &one, zw, n, (rocblas_stride)kXcG * n, ao, n, (rocblas_stride)kXcG * n,
-                                            &zero, q, n, (rocblas_stride)n * n, (int)nb));
-      }
-    }, st);
+    RBCHK(rocblas_dgemm_strided_batched(h->rb, rocblas_operation_none, rocblas_operation_transpose, n, n, kXcG, &one,
+                                        zw, n, (rocblas_stride)kXcG * n, ao, n, (rocblas_stride)kXcG * n, &zero, q, n,
+                                        (rocblas_stride)n * n, (int)nb));
   }
   if (mode == kXcRho) return;
   h->mark(kStXcKernel + 1, st);
@@ -1814,17 +1855,31 @@ void xc_compact(dfks_ctx* h, const double* P, double* E, int mode, hipStream_t s
   h->mark(kStXcSyr2k + 1, st);
 }
 
-// Spin-polarised XC on the compact grid (FP64): per bin both channels' Z_s =
-// Phi_b Pg_s (rocBLAS batched), the spin pointwise kernel (W_a, W_b over Z_a,
-// Z_b), Phi_b^T W_s per channel, then the row assembly of each channel's half
+// Spin-polarised XC on the compact grid (FP64), as xc_compact with both
+// channels' rho, the spin-polarised functional and Phi_b^T W_s per channel
+// (bin by bin on rocBLAS batched products with gemm = rocblas or where a block
+// is wider than kXfMaxN), then the row assembly of each channel's half
 // potential: Vh_a in d_Vxc, Vh_b in d_Vxc2; E_xc into E + DFKS_E_XC.
 void xc_compact_uks(dfks_ctx* h, const double* Pa, const double* Pb, double* E, hipStream_t st) {
   const int nao = h->nao;
   const double one = 1.0, zero = 0.0;
-  if (!h->d_xc_zw2) h->d_xc_zw2 = dalloc<double>(h->xc_zw);
+  if (!h->d_xc_zw2 && h->xc_zw > 0) h->d_xc_zw2 = dalloc<double>(h->xc_zw);
   if (!h->d_xc_q2) h->d_xc_q2 = dalloc<double>(h->xc_qtot);
   if (!h->d_Vxc2) h->d_Vxc2 = dalloc<double>((size_t)nao * nao);
+  if (h->xk_nblk > 0) {
+    if (!h->d_xk_part[1]) h->d_xk_part[1] = dalloc<double>(h->xk_nparts * 4 * kXcG);
+    if (!h->d_xk_coef[1]) h->d_xk_coef[1] = dalloc<double>(4 * h->xc_npts);
+    for (int sp = 0; sp < 2; ++sp)
+      HIPCHK(launch_xcb_rho(h->d_xk_blk, h->d_xk_wg, h->xk_nwg, h->d_xc_ao, h->d_xc_cols, sp == 0 ? Pa : Pb, nao,
+                            h->d_xk_part[sp], st));
+    HIPCHK(launch_xcb_point_pol(h->xk_nblk, h->d_xk_blk, h->d_xk_part[0], h->d_xk_part[1], h->d_xc_w, h->xc_id,
+                                h->opt.rho_thresh, h->d_xc_exc, h->d_xk_coef[0], h->d_xk_coef[1], st));
+    for (int sp = 0; sp < 2; ++sp)
+      HIPCHK(launch_xcb_v(h->d_xk_blk, h->d_xk_wg, h->xk_nwg, h->d_xc_ao, h->d_xk_coef[sp],
+                          sp == 0 ? h->d_xc_q : h->d_xc_q2, st));
+  }
   for (const auto& bn : h->xbins) {
+    if (xc_one_launch(h, bn)) continue;
     const int n = bn.n;
     const int64_t nb = bn.nblk, rows = nb * kXcG;
     const int32_t* cols = h->d_xc_cols + bn.col_off;

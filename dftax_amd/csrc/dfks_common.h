@@ -48,6 +48,14 @@ struct XcfBin {
   int64_t ao_off, col_off, q_off, pt0, part_off, coef_off;
   int32_t wz0, wp0, wv0, pad;
 };
+// One block of the compact XC grid for the FP64 kernels (xc_blocks.hip): n functions, the
+// offsets of its AO rows (first plane; planes are plane doubles apart), columns, product,
+// first point and first strip of partial sums. A workgroup id packs block * kXcbStrips + strip.
+constexpr int kXcbStrips = 32;        // strips of 64 columns: n <= kXfMaxN
+struct XcBlock {
+  int64_t ao0, plane, col0, q0, pt0, part0;
+  int32_t n, pad;
+};
 constexpr int kPanel = 32;            // pivoted Cholesky panel width
 constexpr int kLzSteps = 24;          // Lanczos steps for the SP2 spectral bounds
 constexpr int kLzParts = 4096;        // partial dot products of its matrix-vector kernel (n <= 4 kLzParts)

@@ -972,17 +972,4 @@ hipError_t launch_gemm_b3w8(const GemmArgs& g, float* C, const RowDot& rd, hipSt
   return vec ? run(k_gemm_b3w8<1, true>) : run(k_gemm_b3w8<1, false>);
 }
 
-// Batched FP64 variant (no split, FP64 accumulate): for b < batch,
-// C + b*bs_c = (A + b*bs_a)(B + b*bs_b)^T with ldc = N; 128- or 160-wide N
-// tiles, whichever pads N less (the per-block products of the compact XC grid).
-hipError_t launch_gemm_f64_batched(const GemmArgs& g, double* C, int batch, int64_t bs_a, int64_t bs_b,
-                                   int64_t bs_c, hipStream_t st) {
-  if (g.M <= 0 || g.N <= 0 || batch <= 0) return hipSuccess;
-  if (batch > 65535) return hipErrorInvalidValue;
-  const int t128 = (g.N + 127) / 128, t160 = (g.N + 159) / 160;
-  if (t160 < t128 && (int64_t)t160 * 160 - g.N < (int64_t)t128 * 128 - g.N)
-    return launch_gemm_t<kF64, double, 5>(g, C, g.N, 1, 0, st, batch, bs_a, bs_b, bs_c);
-  return launch_gemm_t<kF64, double>(g, C, g.N, 1, 0, st, batch, bs_a, bs_b, bs_c);
-}
-
 }  // namespace dfks

@@ -148,6 +148,8 @@ hipError_t launch_gemm_f32out(const GemmArgs& g, float* C, hipStream_t st);
 hipError_t launch_gemm_f32out_batched(const GemmArgs& g, float* C, int batch, int64_t bs_a, int64_t bs_b,
                                       int64_t bs_c, hipStream_t st);
 hipError_t launch_gemm_w8(const GemmArgs& g, double* C, const RowDot& rd, hipStream_t st);
+int gemm_t_rows(int N);
+hipError_t launch_gemm_t64(const GemmArgs& g, double* C, const RowDot& rd, hipStream_t st);
 hipError_t launch_gemm_b3w8(const GemmArgs& g, float* C, const RowDot& rd, hipStream_t st, int depth);
 hipError_t launch_colsum(int nrows, int ncols, const double* part, double* out, int accumulate, hipStream_t st);
 hipError_t launch_gemm_partials(int prec, const GemmArgs& g, int nsplit, int sym, void* ws, int variant,
@@ -1406,11 +1408,14 @@ void build_all(dfks_ctx* h, hipStream_t st) {
 // ---------------------------------------------------------------------------
 // energy + Fock for P = sum_i s_i c_i c_i^T (Cf column-major nao x nf)
 // ---------------------------------------------------------------------------
-// split count so a K-long product fills the chip (~2048 workgroups), k-chunks >= 512
+// split count so a K-long product fills the chip (~2048 workgroups), k-chunks >= 512; with few workgroups
+// a whole number per CU (K of (H2O)_8, 6 tiles: 42 splits in one round 164 us, 64 splits 195 us)
 int split_for(int64_t tiles, int64_t K) {
-  int64_t s = 2048 / std::max<int64_t>(tiles, 1);
-  s = std::min<int64_t>(s, std::max<int64_t>(1, K / 512));
-  return (int)std::max<int64_t>(1, std::min<int64_t>(s, 64));
+  tiles = std::max<int64_t>(tiles, 1);
+  int64_t s = 2048 / tiles;
+  s = std::min<int64_t>(std::min<int64_t>(s, std::max<int64_t>(1, K / 512)), 64);
+  if (s * tiles > 256 && s * tiles < 1024) s = s * tiles / 256 * 256 / tiles;
+  return (int)std::max<int64_t>(1, s);
 }
 
 // (mn|P) for the functions of slab s into d_slab, layout [m][n][p] with
@@ -1494,7 +1499,7 @@ void coulomb_recompute(dfks_ctx* h, hipStream_t st) {
 // with HIP events on the work stream, and the process keeps the faster one for
 // that shape. Both compute the same T to rounding.
 // Per-shape choice among the variants of a product. Tags and variants:
-//   0  FP64 exchange T = B^T C:      0 rocBLAS, 1 k_gemm, 2 k_gemm_w8
+//   0  FP64 exchange T = B^T C:      0 rocBLAS, 1 k_gemm, 2 k_gemm_w8, 3 k_gemm_t
 //   3  FP64 exchange K partials:     0 k_gemm, 1 k_gemm_w8, 2 k_gemm_w8 split by XCD (base 1)
 //   4  split-BF16 exchange T:        0 k_gemm, 1 k_gemm_b3w8 (base 1)
 //   5  SP2 product partials X X:     0 k_gemm, 1 k_gemm_w8   (base 1)
@@ -1564,10 +1569,12 @@ int tuned_product(dfks_ctx* h, int tag, int64_t d0, int64_t d1, int64_t d2, int 
 bool t_product(dfks_ctx* h, const double* C, int nc, const RowDot& rd, hipStream_t st) {
   const int nao = h->nao, nfit = h->nfit;
   const double one = 1.0, zero = 0.0;
-  const bool fuse = nc <= 160 && nfit >= 128;
-  const int v = tuned_product(h, 0, (int64_t)nao * nfit, nc, nao, 3, 0, [&](int choice) {
+  const bool fuse = nc <= 160 && nfit >= 128, fuse_t = nc <= 160 && nfit >= gemm_t_rows(nc);
+  const int v = tuned_product(h, 0, (int64_t)nao * nfit, nc, nao, 4, 0, [&](int choice) {
     const GemmArgs g{(int)((int64_t)nao * nfit), nc, nao, h->d_B, (int64_t)nao * nfit, false, C, nao, true};
-    if (choice == 2) {
+    if (choice == 3) {
+      HIPCHK(launch_gemm_t64(g, h->d_Tx, fuse_t ? rd : RowDot(), st));
+    } else if (choice == 2) {
       HIPCHK(launch_gemm_w8(g, h->d_Tx, fuse ? rd : RowDot(), st));
     } else if (choice == 1) {
       HIPCHK(launch_gemm(kF64, g, h->d_Tx, 1.0, 0.0, 1, 0, nullptr, st));
@@ -1577,7 +1584,7 @@ bool t_product(dfks_ctx* h, const double* C, int nc, const RowDot& rd, hipStream
                              nc));
     }
   }, st);
-  return fuse && v == 2;
+  return (fuse && v == 2) || (fuse_t && v == 3);
 }
 
 // Kout = sg T^T T + beta Kout in FP64 for T = d_Tx (nao rows of kd contiguous

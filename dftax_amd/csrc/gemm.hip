@@ -21,6 +21,7 @@
 // gridDim.z into a workspace of per-split partial tiles, then a deterministic
 // reduction kernel sums the splits in order (and mirrors the symmetric case).
 #include <cstdint>
+#include <type_traits>
 
 #include "dfks_common.h"
 
@@ -752,43 +753,54 @@ __global__ void k_gemm_reduce(int M, int N, int nsplit, const W* __restrict__ ws
   out[(int64_t)m * ldo + n] = (Out)v;
 }
 
-// Symmetric mode of the reduce for N x N: one workgroup per upper 64 x 64 tile
-// (ti <= tj) sums the partials of the tile's upper elements (coalesced, fixed
-// order), writes them, and writes the mirror tile through LDS, so both stores
-// are row-contiguous (the elementwise kernel read the lower half's partials
+// Symmetric mode of the reduce for N x N: a workgroup takes four rows of an
+// upper 64 x 64 tile (ti <= tj), one element a thread, sums its partials
+// (coalesced, fixed order, eight loads in flight), writes them, and writes the
+// mirror through LDS (the elementwise kernel read the lower half's partials
 // down columns). out = alpha * sum (+ beta * out) for every element, the
-// lower one from its upper partner's sum, as in the elementwise kernel.
+// lower one from its upper partner's sum, as in the elementwise kernel. The
+// loads are what it waits for: 64 partials of n = 344 take 391 us by whole tiles
+// with one load at a time (21 workgroups) and 9 us this way.
+constexpr int kRedRows = 4;
 template <typename W, typename Out>
 __global__ __launch_bounds__(256) void k_gemm_reduce_sym(int N, int nsplit, const W* __restrict__ ws,
                                                          int64_t split_stride, int64_t ldw, Out* __restrict__ out,
                                                          int64_t ldo, double alpha, double beta) {
-  __shared__ double t[64][65];
+  __shared__ double t[kRedRows][65];
   const int ntn = (N + 63) / 64;
-  int ti = 0, b = (int)blockIdx.x;
+  int ti = 0, b = (int)blockIdx.x / (64 / kRedRows);
+  const int rb = kRedRows * ((int)blockIdx.x % (64 / kRedRows));
   while (b >= ntn - ti) {
     b -= ntn - ti;
     ++ti;
   }
   const int tj = ti + b;
   if (ti >= ntn) return;
-  const int m0 = 64 * ti, n0 = 64 * tj, c = threadIdx.x & 63, r0 = threadIdx.x >> 6;
-  for (int j = 0; j < 16; ++j) {
-    const int r = r0 + 4 * j, m = m0 + r, n = n0 + c;
-    if (m < N && n < N && (ti != tj || r <= c)) {
-      double s = 0.0;
-      for (int z = 0; z < nsplit; ++z) s += (double)ws[z * split_stride + (int64_t)m * ldw + n];
-      const double v = alpha * s;
-      t[r][c] = v;
-      out[(int64_t)m * ldo + n] = (Out)(beta != 0.0 ? v + beta * (double)out[(int64_t)m * ldo + n] : v);
+  const int c = threadIdx.x & 63, rl = threadIdx.x >> 6, r = rb + rl;
+  const int m = 64 * ti + r, n = 64 * tj + c;
+  if (m < N && n < N && (ti != tj || r <= c)) {
+    const W* src = ws + (int64_t)m * ldw + n;
+    double s = 0.0;
+    int z = 0;
+    for (; z + 8 <= nsplit; z += 8) {
+      W x[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) x[k] = src[(z + k) * split_stride];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) s += (double)x[k];
     }
+    for (; z < nsplit; ++z) s += (double)src[z * split_stride];
+    const double v = alpha * s;
+    t[rl][c] = v;
+    out[(int64_t)m * ldo + n] = (Out)(beta != 0.0 ? v + beta * (double)out[(int64_t)m * ldo + n] : v);
   }
   __syncthreads();
-  for (int j = 0; j < 16; ++j) {
-    const int r = r0 + 4 * j, m = n0 + r, n = m0 + c;   // mirror element (n0 + r, m0 + c) of tile (c, r)
-    if (m < N && n < N && (ti != tj || c < r)) {
-      const double v = t[c][r];
-      out[(int64_t)m * ldo + n] = (Out)(beta != 0.0 ? v + beta * (double)out[(int64_t)m * ldo + n] : v);
-    }
+  // mirror: element (64 tj + cm, 64 ti + rm) from (rm, cm); kRedRows consecutive values of a row
+  const int rm = threadIdx.x % kRedRows, cm = threadIdx.x / kRedRows;
+  const int mm = 64 * tj + cm, mn = 64 * ti + rb + rm;
+  if (mm < N && mn < N && (ti != tj || rb + rm < cm)) {
+    const double v = t[rm][cm];
+    out[(int64_t)mm * ldo + mn] = (Out)(beta != 0.0 ? v + beta * (double)out[(int64_t)mm * ldo + mn] : v);
   }
 }
 
@@ -874,6 +886,166 @@ hipError_t launch_gemm_w8(const GemmArgs& g, double* C, const RowDot& rd, hipStr
   return launch_w8_t<4>(g, C, g.N, 1, 0, st, rd);
 }
 
+// T = A B^T for a tall M-contiguous A (the fitted tensor: M = nao nfit rows of K =
+// nao) and at most 160 columns per tile (B: the factor columns, K-contiguous).
+// Every element of A meets one wavefront only, so A goes from global memory to
+// the MFMA operand registers directly (two consecutive rows per 16-byte load,
+// 256-byte runs), each step's registers reloaded for the next 16 k as soon as
+// its products are issued; B is staged 16 k at a time in LDS in fragment order.
+// The tile is as wide as the factor (16 NJ), where the 128- and 160-wide tiles
+// of k_gemm_w8 pad: below about 64 columns the product is bound by reading A
+// once. K = 344, 40 columns ((H2O)_8 def2-TZVP): 0.26 ms = 3.4 TB/s, against
+// 0.53 (k_gemm), 0.60 (rocBLAS) and 0.65 ms; K = 1032, 48 columns: 5.2 against
+// 10.7 ms. At 120 columns rocBLAS is ahead (12.6 against 14.2 ms).
+template <int NJ>
+struct TTile {
+  static constexpr int MI = NJ <= 4 ? 4 : 2, ROWS = 64 * MI;   // 16-row blocks per wavefront, rows per workgroup
+};
+// 16 bytes of A: rows are 8-byte aligned only when M is odd
+typedef double dbl2u __attribute__((ext_vector_type(2), aligned(8)));
+
+template <int NJ>
+__global__ __launch_bounds__(256, NJ <= 1 ? 4 : 2) void k_gemm_t(int64_t M, int N, int K, const double* __restrict__ A,
+                                                                int64_t lda, const double* __restrict__ B, int64_t ldb,
+                                                                double* __restrict__ C, int64_t ldc, RowDot rd) {
+  constexpr int MI = TTile<NJ>::MI, ROWS = TTile<NJ>::ROWS, MP = MI / 2, BN = 16 * NJ;
+  __shared__ double s_b[2][4 * NJ * 64];
+  __shared__ double s_cs[2][BN];
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t m0 = (int64_t)blockIdx.x * ROWS, mw = m0 + wv * (16 * MI);
+  const int n0 = blockIdx.y * BN;
+  // gamma row terms: the tile's rows span at most two m (nq >= ROWS)
+  if (rd.out)
+    for (int x = tid; x < 2 * BN; x += 256) {
+      const int gn = x % BN;
+      const int64_t mm = m0 / rd.nq + x / BN;
+      s_cs[x / BN][gn] = gn < N && mm < rd.nao ? rd.sg[gn] * rd.cf[(int64_t)gn * rd.nao + mm] : 0.0;
+    }
+  dbl4 acc[MI][NJ];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
+  dbl2u a[4][MP];
+  double b[NJ];
+  const int bk = tid & 15, bi = tid >> 4;
+  const double* brow[NJ];      // a column past N repeats the last one and is not stored
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) brow[j] = B + (int64_t)min(n0 + 16 * j + bi, N - 1) * ldb;
+  const auto load_b = [&](int k0) __attribute__((always_inline)) {
+    const int k = min(k0 + bk, K - 1);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) b[j] = brow[j][k];
+  };
+  // FULL: all of the workgroup's rows exist
+  const auto product = [&](auto FULL) __attribute__((always_inline)) {
+    const auto load_a = [&](int s, int k0) __attribute__((always_inline)) {
+      const double* src = A + (int64_t)min(k0 + 4 * s + lk, K - 1) * lda;   // past the end: B is zero there
+#pragma unroll
+      for (int p = 0; p < MP; ++p) {
+        const int64_t m = mw + 32 * p + 2 * li;
+        if constexpr (decltype(FULL)::value) {
+          a[s][p] = *reinterpret_cast<const dbl2u*>(src + m);
+        } else {
+          a[s][p][0] = src[min(m, M - 1)];
+          a[s][p][1] = src[min(m + 1, M - 1)];
+        }
+      }
+    };
+    load_b(0);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) load_a(s, 0);
+    for (int k0 = 0, buf = 0; k0 < K; k0 += 16, buf ^= 1) {
+      double* sb = s_b[buf];
+      const bool in = k0 + bk < K;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) sb[((bk >> 2) * NJ + j) * 64 + (bk & 3) * 16 + bi] = in ? b[j] : 0.0;
+      __syncthreads();     // the other buffer's readers passed the previous barrier
+      const int kn = min(k0 + 16, K - 1);      // the last step's reloads are not used
+      load_b(kn);
+      double bf[2][NJ];
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) bf[0][j] = sb[j * 64 + lane];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        if (s < 3) {
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) bf[(s + 1) & 1][j] = sb[((s + 1) * NJ + j) * 64 + lane];
+        }
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < NJ; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s][i >> 1][i & 1], bf[s & 1][j], acc[i][j], 0, 0, 0);
+        load_a(s, kn);
+      }
+    }
+    // keeps the reloads where they are issued: unused after the last step, they would be moved to the
+    // start of the next one, with nothing to hide them
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int p = 0; p < MP; ++p) asm volatile("" ::"v"(a[s][p]));
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) asm volatile("" ::"v"(b[j]));
+  };
+  if (m0 + ROWS <= M) product(std::true_type());
+  else product(std::false_type());
+  // result register r of block i: row 32 (i / 2) + 2 (lk + 4 r) + i % 2 of the wavefront's rows, column 16 j + li
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int64_t gm = mw + 32 * (i >> 1) + 2 * (lk + 4 * r) + (i & 1);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const int gn = n0 + 16 * j + li;
+        if (gm < M && gn < N) C[gm * ldc + gn] = acc[i][j][r];
+      }
+      if (rd.out) {
+        const int which = gm < M ? (int)(gm / rd.nq - m0 / rd.nq) : 0;
+        double v = 0.0;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) v += acc[i][j][r] * s_cs[which][16 * j + li];
+        v += __shfl_xor(v, 1, 64);
+        v += __shfl_xor(v, 2, 64);
+        v += __shfl_xor(v, 4, 64);
+        v += __shfl_xor(v, 8, 64);
+        if (li == 0 && gm < M) rd.out[gm] = v;
+      }
+    }
+}
+
+// C = A B^T (ldc = N) by k_gemm_t in equal column tiles of at most 160; A M-contiguous, B K-contiguous. rd.out
+// (optional): the row terms of gamma, for one column tile and rd.nq at least gemm_t_rows(N).
+int gemm_t_rows(int N) { return (N + 15) / 16 <= 4 ? TTile<4>::ROWS : TTile<5>::ROWS; }
+
+hipError_t launch_gemm_t64(const GemmArgs& g, double* C, const RowDot& rd, hipStream_t st) {
+  if (g.M <= 0 || g.N <= 0) return hipSuccess;
+  if (g.K <= 0 || g.K > 0x7fffffff || g.a_kcontig || !g.b_kcontig) return hipErrorInvalidValue;
+  const int nt = (g.N + 159) / 160, nj = ((g.N + nt - 1) / nt + 15) / 16;
+  if (rd.out && (nt > 1 || rd.nq < gemm_t_rows(g.N))) return hipErrorInvalidValue;
+  const auto run = [&](auto kern, int rows) {
+    const int64_t nb = ((int64_t)g.M + rows - 1) / rows;
+    return launch_k(kern, dim3((unsigned)nb, (unsigned)nt), dim3(256), st, (int64_t)g.M, g.N, (int)g.K,
+                    static_cast<const double*>(g.A), g.lda, static_cast<const double*>(g.B), g.ldb, C, (int64_t)g.N,
+                    rd);
+  };
+  switch (nj) {
+    case 1: return run(k_gemm_t<1>, TTile<1>::ROWS);
+    case 2: return run(k_gemm_t<2>, TTile<2>::ROWS);
+    case 3: return run(k_gemm_t<3>, TTile<3>::ROWS);
+    case 4: return run(k_gemm_t<4>, TTile<4>::ROWS);
+    case 5: return run(k_gemm_t<5>, TTile<5>::ROWS);
+    case 6: return run(k_gemm_t<6>, TTile<6>::ROWS);
+    case 7: return run(k_gemm_t<7>, TTile<7>::ROWS);
+    case 8: return run(k_gemm_t<8>, TTile<8>::ROWS);
+    case 9: return run(k_gemm_t<9>, TTile<9>::ROWS);
+    default: return run(k_gemm_t<10>, TTile<10>::ROWS);
+  }
+}
+
 // Split-K partial tiles of A B^T into ws (nsplit x M x N, FP64 for kF64 and
 // FP32 for kBF16x3; upper tiles only in the symmetric mode). variant 1 takes
 // the 8-wavefront FP64 tile where it applies (B K-contiguous), 0 k_gemm.
@@ -896,7 +1068,7 @@ hipError_t launch_gemm_reduce(int prec, const GemmArgs& g, double* C, double alp
   const int64_t stride = (int64_t)g.M * g.N;
   if ((sym & 1) && g.M == g.N) {
     const int ntn = (g.N + 63) / 64;
-    const unsigned nt = (unsigned)((int64_t)ntn * (ntn + 1) / 2);
+    const unsigned nt = (unsigned)((int64_t)ntn * (ntn + 1) / 2 * (64 / kRedRows));
     if (prec == kF64)
       return launch_k(k_gemm_reduce_sym<double, double>, dim3(nt), dim3(256), st, g.N, nsplit,
                       static_cast<const double*>(ws), stride, (int64_t)g.N, C, (int64_t)g.N, alpha, beta);

@@ -60,7 +60,7 @@ __device__ __forceinline__ void rho_strip(const XcBlock& b, int c0, const double
   const int n = b.n;
   const int pc = tid % W, pk = tid / W;
   const int32_t cc = cols[c0 + pc];
-  const double* pcol = P + (cc >= 0 ? cc : 0);
+  const double* pcol = P + max(cc, 0);
   const double* arow = ao + (int64_t)(32 * wv + li) * n + 4 * lk;
   dbl4 acc[2][NJ];
 #pragma unroll
@@ -72,9 +72,8 @@ __device__ __forceinline__ void rho_strip(const XcBlock& b, int c0, const double
   const auto load_p = [&](int k0) __attribute__((always_inline)) {
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
-      const int32_t kc = cols[k0 + pk + STEP * e];
-      const double v = pcol[(int64_t)(kc >= 0 ? kc : 0) * nao];
-      p[e] = kc >= 0 && cc >= 0 ? v : 0.0;
+      // a padded k or column meets zero AO values: any element of P will do there
+      p[e] = pcol[(int64_t)max(cols[k0 + pk + STEP * e], 0) * nao];
     }
   };
   const auto load_a = [&](int q, int k0) __attribute__((always_inline)) {

@@ -165,6 +165,9 @@ hipError_t launch_sp2_begin(int n, const double* X, int nocc, double* st, hipStr
 hipError_t launch_sp2_update(int n, int nsplit, const double* ws, double* X, int nocc, double* st, hipStream_t s);
 int sp2_step_tiles(int n);
 hipError_t launch_sp2_step(int n, const double* X, double* Xn, int nocc, double* st, hipStream_t s);
+hipError_t launch_sp2_tile(int n, const double* X, double* Xn, int nocc, const double* st, double* stn,
+                           hipStream_t s);
+hipError_t launch_sp2_settle(int nocc, double* st, hipStream_t s);
 hipError_t launch_diag(int n, const double* R, double* d, hipStream_t s);
 hipError_t launch_pchol_panel(int n, int k0, int b, const double* R, double* d, double* L, int32_t* piv, double* st,
                               int last, hipStream_t s);
@@ -1365,7 +1368,7 @@ void build_all(dfks_ctx* h, hipStream_t st) {
   h->d_gws = dalloc<double>((size_t)64 * nao * nao);
   // purification state: fixed size, allocated once, because the purification
   // graph keeps its address (as it keeps those of d_W1 and d_gws)
-  h->d_sp2 = dalloc<double>(kSp2State);
+  h->d_sp2 = dalloc<double>(2 * kSp2State);
   h->d_lz = dalloc<double>(3 * (size_t)nao + kLzParts + 2 * kLzSteps);
   h->d_gpart = dalloc<double>((size_t)nao * h->nfit);
   if (h->opt.precision == 1) {
@@ -2572,14 +2575,26 @@ int sp2_split(int n) {
   return best;
 }
 
-// kSp2Block purification iterations, launched eagerly. Up to kSp2Groups upper 64 x 64
-// tiles (n <= 2015): one fused kernel per iteration (product, update, trace sums) that
-// alternates X between d_W1 and the split-K workspace, so the block (an even number of
+// kSp2Block purification iterations, launched eagerly. n <= kSp2TileN: one kernel per
+// iteration that also takes the decision, on tiles of 16 to 48 (k_sp2_tile); up to
+// kSp2Groups upper 64 x 64 tiles (n <= 2015): one fused kernel per iteration (product,
+// update, trace sums) and the decision; both alternate X between d_W1 and the split-K workspace, so the block (an even number of
 // iterations) leaves X in d_W1. Larger n: the split-K product's partial tiles, then the
 // update kernel.
 hipError_t sp2_block(dfks_ctx* h, hipStream_t st) {
   const int n = h->nmo;
   static_assert(kSp2Block % 2 == 0, "the fused iterations end in d_W1");
+  if (n <= kSp2TileN) {
+    for (int c = 0; c < kSp2Block; ++c) {
+      const double* X = c % 2 == 0 ? h->d_W1 : h->d_gws;
+      double* Xn = c % 2 == 0 ? h->d_gws : h->d_W1;
+      double* s0 = h->d_sp2 + (c % 2 == 0 ? 0 : kSp2State);
+      double* s1 = h->d_sp2 + (c % 2 == 0 ? kSp2State : 0);
+      const hipError_t e = launch_sp2_tile(n, X, Xn, h->nocc, s0, s1, st);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
   if (sp2_step_tiles(n) <= kSp2Groups) {
     for (int c = 0; c < kSp2Block; ++c) {
       const double* X = c % 2 == 0 ? h->d_W1 : h->d_gws;
@@ -2780,12 +2795,13 @@ bool purify_density(dfks_ctx* h, hipStream_t st) {
   HIPCHK(launch_sp2_begin(n, X, nocc, h->d_sp2, st));
   int done = 0;
   int chunk = h->sp2_guess + 1;
-  double stv[kSpHist];
+  double stv[kSpHead];
   bool frozen = false;
   while (done < kSp2MaxIter) {
     int nblocks = (chunk + kSp2Block - 1) / kSp2Block;
     nblocks = std::min(nblocks, (kSp2MaxIter - done) / kSp2Block);
     sp2_run_blocks(h, nblocks, st);
+    if (n <= kSp2TileN) HIPCHK(launch_sp2_settle(nocc, h->d_sp2, st));
     done += nblocks * kSp2Block;
     HIPCHK(hipMemcpyAsync(stv, h->d_sp2, sizeof(stv), hipMemcpyDeviceToHost, st));
     sync(st);

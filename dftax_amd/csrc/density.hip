@@ -101,6 +101,8 @@ __global__ __launch_bounds__(256) void k_sp2_start(int n, const double* __restri
     st[kSpTrace] = 0.0;
     st[kSpResid] = 0.0;
     st[kSpMinPiv] = 1e300;
+    st[kSpPend] = 0.0;
+    st[kSpNPart] = 0.0;
   }
 }
 
@@ -114,30 +116,34 @@ __global__ void k_sp2_init(int n, const double* __restrict__ F, const double* __
   X[idx] = ((i == j ? hi : 0.0) - F[idx]) / (hi - lo);
 }
 
-// The branch (or the freeze) of one iteration from t1 = tr X and t2 = tr X^2
-// (thread 0 of k_sp2_decide).
-__device__ void sp2_decide(double t1, double t2, int nocc, double* __restrict__ st) {
-  if (st[kSpFlag] < 0.0) return;  // frozen
-  const int it = (int)st[kSpIter];
-  const double e = t1 - t2;
-  if (it < kSp2MaxIter) st[kSpHist + it] = e;
-  st[kSpIter] = it + 1;
-  st[kSpErr] = e;
-  st[kSpTrace] = t1;
-  const double cnt = st[kSpCount];
-  double flag;
-  if (cnt >= 2.0) {
-    flag = -1.0;  // converged: X is final
-  } else if (cnt == 1.0) {
-    flag = 0.0;   // second forced step: 2X - X^2
-    st[kSpCount] = 2.0;
-  } else if (fabs(e) < kSp2Tol) {
-    flag = 1.0;   // first forced step: X^2
-    st[kSpCount] = 1.0;
-  } else {
-    flag = fabs(t2 - nocc) < fabs(2.0 * t1 - t2 - nocc) ? 1.0 : 0.0;
+// The branch (or the freeze) of one iteration from t1 = tr X and t2 = tr X^2, written to st (which may be old)
+__device__ void sp2_decide(double t1, double t2, int nocc, const double* old, double* st) {
+  double flag = old[kSpFlag], cnt = old[kSpCount], it = old[kSpIter], err = old[kSpErr], tr = old[kSpTrace];
+  if (flag >= 0.0) {   // else frozen
+    err = t1 - t2;
+    tr = t1;
+    it += 1.0;
+    if (cnt >= 2.0) {
+      flag = -1.0;  // converged: X is final
+    } else if (cnt == 1.0) {
+      flag = 0.0;   // second forced step: 2X - X^2
+      cnt = 2.0;
+    } else if (fabs(err) < kSp2Tol) {
+      flag = 1.0;   // first forced step: X^2
+      cnt = 1.0;
+    } else {
+      flag = fabs(t2 - nocc) < fabs(2.0 * t1 - t2 - nocc) ? 1.0 : 0.0;
+    }
   }
+  st[kSpEmin] = old[kSpEmin];
+  st[kSpEmax] = old[kSpEmax];
   st[kSpFlag] = flag;
+  st[kSpCount] = cnt;
+  st[kSpIter] = it;
+  st[kSpErr] = err;
+  st[kSpTrace] = tr;
+  st[kSpResid] = old[kSpResid];
+  st[kSpMinPiv] = old[kSpMinPiv];
 }
 
 // Per-workgroup partial sums of tr X and of sum_ij X_ij^2 (= tr X^2 for the
@@ -174,7 +180,7 @@ __global__ __launch_bounds__(256) void k_sp2_norms(int n, const double* __restri
 }
 
 // One block: t1, t2 from the kSp2Groups partial pairs (fixed order), then the branch.
-__global__ __launch_bounds__(kSp2Groups) void k_sp2_decide(int nocc, double* __restrict__ st) {
+__global__ __launch_bounds__(kSp2Groups) void k_sp2_decide(int nocc, double* st) {
   __shared__ double s_a[kSp2Groups], s_b[kSp2Groups];
   s_a[threadIdx.x] = st[kSpPart + 2 * threadIdx.x];
   s_b[threadIdx.x] = st[kSpPart + 2 * threadIdx.x + 1];
@@ -186,7 +192,7 @@ __global__ __launch_bounds__(kSp2Groups) void k_sp2_decide(int nocc, double* __r
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) sp2_decide(s_a[0], s_b[0], nocc, st);
+  if (threadIdx.x == 0) sp2_decide(s_a[0], s_b[0], nocc, st, st);
 }
 
 // X <- X^2 or 2X - X^2 by the decided branch, X^2 summed from the nsplit
@@ -213,8 +219,8 @@ __global__ __launch_bounds__(256) void k_sp2_reduce_update(int n, int nsplit, co
   sp2_partials(a, b, st);
 }
 
-// One purification iteration in one kernel, for n with at most kSp2Groups upper
-// 64 x 64 tiles (n <= 2015). Workgroup b < ntiles takes upper tile (ti, tj),
+// One purification iteration in one kernel, for n above kSp2TileN with at most
+// kSp2Groups upper 64 x 64 tiles (n <= 2015). Workgroup b < ntiles takes upper tile (ti, tj),
 // ti <= tj, of S = X X (FP64 MFMA over the full K; both operands are rows of
 // the symmetric X), applies the decided branch, Xn = S or 2X - S, writes the
 // tile and its mirror (through LDS, so both stores are row-contiguous), and
@@ -345,6 +351,230 @@ __global__ __launch_bounds__(kSqN) void k_sp2_step(int n, int ntiles, const doub
     }
   }
   sp2_partials<kSqN>(ta, tb, st);
+}
+
+// One purification iteration for n <= kSp2TileN, one kernel and no other: an upper
+// tile of 16 TB rows and columns per workgroup, TB the smallest that leaves at
+// most one tile per CU, so that small n still spread over the chip (k_sp2_step's
+// 64 x 64 tiles put n = 344 on 21 CUs). The wavefronts split K: X is symmetric,
+// so both operands are rows, contiguous in k, and go from global memory to the
+// MFMA registers directly, lane group l taking k = 4 l + s in step s (the product
+// sums over any order of k both operands share). The partial tiles are added in
+// LDS in a fixed order. The previous iteration's sums decide this one's branch:
+// every workgroup adds them (in the same order) while its product runs, the
+// first one writes the new state, so no kernel stands between two iterations;
+// states and X alternate. What bounds it is the chain of one kernel: launch, X
+// from the previous kernel through the memory side, product, LDS sum. (H2O)_8
+// def2-TZVP (n = 344) 27.5 -> 7.6 us per iteration,
+// n = 602: 37.6 -> 12.9 us, n = 60: 14.9 -> 5.0 us.
+typedef double sq2u __attribute__((ext_vector_type(2), aligned(8)));   // rows start at multiples of n
+
+// t1, t2 from np partial pairs by one wavefront, valid in lane 0
+__device__ __forceinline__ void sp2_sums(const double* __restrict__ part, int np, int lane, double& t1, double& t2) {
+  t1 = t2 = 0.0;
+  for (int t = lane; t < np; t += 64) {
+    t1 += part[2 * t];
+    t2 += part[2 * t + 1];
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    t1 += __shfl_down(t1, o);
+    t2 += __shfl_down(t2, o);
+  }
+}
+
+template <int TB, int NW>
+__global__ __launch_bounds__(NW * 64) void k_sp2_tile(int n, const double* __restrict__ X, double* __restrict__ Xn,
+                                                      int nocc, const double* __restrict__ st,
+                                                      double* __restrict__ stn) {
+  constexpr int T = 16 * TB, TT = T * T, NT = NW * 64, NE = (TT + NT - 1) / NT;
+  __shared__ double s_acc[NW * TT];
+  __shared__ double s_t[2][NW];
+  __shared__ double s_flag;
+  static_assert(T * (T + 1) <= NW * TT, "the mirror tile reuses s_acc");
+  const int ntn = (n + T - 1) / T;
+  int ti = 0, b = blockIdx.x;
+  while (b >= ntn - ti) {
+    b -= ntn - ti;
+    ++ti;
+  }
+  const int tj = ti + b, m0 = ti * T, n0 = tj * T;
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool frozen = st[kSpFlag] < 0.0;
+  // element e of the tile: MFMA block e / 256, result register (e / 64) % 4, lane e % 64
+  const auto elem = [&](int e, int& r, int& c) {
+    const int blk = e >> 8, l = e & 63;
+    r = 16 * (blk / TB) + (l >> 4) + 4 * ((e >> 6) & 3);
+    c = 16 * (blk % TB) + (l & 15);
+  };
+  double x0[NE];
+#pragma unroll
+  for (int k = 0; k < NE; ++k) {
+    int r, c;
+    elem(min(tid + k * NT, TT - 1), r, c);
+    x0[k] = X[(int64_t)min(m0 + r, n - 1) * n + min(n0 + c, n - 1)];
+  }
+  sq4 acc[TB][TB];
+#pragma unroll
+  for (int i = 0; i < TB; ++i)
+#pragma unroll
+    for (int j = 0; j < TB; ++j) acc[i][j] = sq4{0, 0, 0, 0};
+  if (!frozen) {
+    const double *pa[TB], *pb[TB];   // rows past n repeat the last one and are not stored
+#pragma unroll
+    for (int i = 0; i < TB; ++i) {
+      pa[i] = X + (int64_t)min(m0 + 16 * i + li, n - 1) * n;
+      pb[i] = X + (int64_t)min(n0 + 16 * i + li, n - 1) * n;
+    }
+    const int nfull = n / 16;
+    sq2u a[TB][2], bb[TB][2];
+    const auto load = [&](int g) __attribute__((always_inline)) {
+      const int k = 16 * g + 4 * lk;
+#pragma unroll
+      for (int i = 0; i < TB; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          a[i][h] = *reinterpret_cast<const sq2u*>(pa[i] + k + 2 * h);
+          bb[i][h] = *reinterpret_cast<const sq2u*>(pb[i] + k + 2 * h);
+        }
+    };
+    const auto mul = [&](const sq2u (&u)[TB][2], const sq2u (&v)[TB][2]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < TB; ++i)
+#pragma unroll
+          for (int j = 0; j < TB; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(u[i][s >> 1][s & 1], v[j][s >> 1][s & 1], acc[i][j], 0, 0,
+                                                             0);
+    };
+    int g = wv;
+    if (g < nfull) {
+      load(g);
+      for (; g + NW < nfull; g += NW) {
+        sq2u u[TB][2], v[TB][2];
+#pragma unroll
+        for (int i = 0; i < TB; ++i)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            u[i][h] = a[i][h];
+            v[i][h] = bb[i][h];
+          }
+        load(g + NW);
+        mul(u, v);
+      }
+      mul(a, bb);
+    }
+    if (n % 16 != 0 && nfull % NW == wv) {   // the last, partial group of k
+#pragma unroll
+      for (int i = 0; i < TB; ++i)
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          const int k = 16 * nfull + 4 * lk + h, kc = min(k, n - 1);
+          a[i][h >> 1][h & 1] = k < n ? pa[i][kc] : 0.0;
+          bb[i][h >> 1][h & 1] = pb[i][kc];
+        }
+      mul(a, bb);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < TB; ++i)
+#pragma unroll
+    for (int j = 0; j < TB; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s_acc[wv * TT + ((i * TB + j) * 4 + r) * 64 + lane] = acc[i][j][r];
+  if (wv == 0) {
+    double flag = st[kSpFlag];
+    const bool pend = st[kSpPend] != 0.0;
+    double t1 = 0.0, t2 = 0.0;
+    if (pend) sp2_sums(st + kSpPart, (int)st[kSpNPart], lane, t1, t2);
+    if (lane == 0) {
+      double s[kSpHead];
+      if (pend) {
+        sp2_decide(t1, t2, nocc, st, s);
+        flag = s[kSpFlag];
+      } else {
+#pragma unroll
+        for (int k = 0; k < kSpPend; ++k) s[k] = st[k];
+      }
+      s_flag = flag;
+      if (blockIdx.x == 0) {
+#pragma unroll
+        for (int k = 0; k < kSpPend; ++k) stn[k] = s[k];
+        stn[kSpPend] = flag < 0.0 ? 0.0 : 1.0;
+        stn[kSpNPart] = (double)gridDim.x;
+      }
+    }
+  }
+  __syncthreads();
+  const double flag = s_flag;
+  const double wsq = ti == tj ? 1.0 : 2.0;
+  double ta = 0.0, tb = 0.0, xv[NE];
+#pragma unroll
+  for (int k = 0; k < NE; ++k) {
+    const int e = tid + k * NT;
+    if (e < TT) {
+      int r, c;
+      elem(e, r, c);
+      double sq = 0.0;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) sq += s_acc[w * TT + e];
+      const int gm = m0 + r, gn = n0 + c;
+      double x = 0.0;
+      if (gm < n && gn < n) {
+        x = flag < 0.0 ? x0[k] : flag > 0.5 ? sq : 2.0 * x0[k] - sq;
+        Xn[(int64_t)gm * n + gn] = x;
+        if (gm == gn) ta += x;
+        tb += wsq * x * x;
+      }
+      xv[k] = x;
+    }
+  }
+  // this tile's share of tr Xn and sum Xn_ij^2, and the mirror tile through LDS
+  for (int o = 32; o > 0; o >>= 1) {
+    ta += __shfl_down(ta, o);
+    tb += __shfl_down(tb, o);
+  }
+  if (lane == 0) {
+    s_t[0][wv] = ta;
+    s_t[1][wv] = tb;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    double u = 0.0, v = 0.0;
+    for (int w = 0; w < NW; ++w) {
+      u += s_t[0][w];
+      v += s_t[1][w];
+    }
+    stn[kSpPart + 2 * blockIdx.x] = u;
+    stn[kSpPart + 2 * blockIdx.x + 1] = v;
+  }
+  if (ti == tj) return;
+#pragma unroll
+  for (int k = 0; k < NE; ++k) {
+    const int e = tid + k * NT;
+    if (e < TT) {
+      int r, c;
+      elem(e, r, c);
+      s_acc[r * (T + 1) + c] = xv[k];
+    }
+  }
+  __syncthreads();
+  for (int e = tid; e < TT; e += NT) {
+    const int c = e / T, r = e % T, gm = n0 + c, gn = m0 + r;
+    if (gm < n && gn < n) Xn[(int64_t)gm * n + gn] = s_acc[r * (T + 1) + c];
+  }
+}
+
+// The decision left pending by the last tiled step (before the host reads the state).
+__global__ __launch_bounds__(64) void k_sp2_settle(int nocc, double* st) {
+  if (st[kSpPend] == 0.0) return;
+  double t1, t2;
+  sp2_sums(st + kSpPart, (int)st[kSpNPart], threadIdx.x, t1, t2);
+  if (threadIdx.x == 0) {
+    sp2_decide(t1, t2, nocc, st, st);
+    st[kSpPend] = 0.0;
+  }
 }
 
 // d[i] = R_ii
@@ -718,6 +948,23 @@ hipError_t launch_sp2_step(int n, const double* X, double* Xn, int nocc, double*
   const hipError_t e = launch_k(k_sp2_step, dim3(kSp2Groups), dim3(kSqN), s, n, ntiles, X, Xn, st);
   if (e != hipSuccess) return e;
   return launch_k(k_sp2_decide, dim3(1), dim3(kSp2Groups), s, nocc, st);
+}
+
+// One tiled iteration (n <= kSp2TileN) X -> Xn, st -> stn; launch_sp2_settle once after the last of a run.
+hipError_t launch_sp2_tile(int n, const double* X, double* Xn, int nocc, const double* st, double* stn,
+                           hipStream_t s) {
+  const auto run = [&](auto kern, int t, int nt) {
+    const int ntn = (n + t - 1) / t;
+    return launch_k(kern, dim3((unsigned)(ntn * (ntn + 1) / 2)), dim3(nt), s, n, X, Xn, nocc, st, stn);
+  };
+  if (n < 1 || n > kSp2TileN) return hipErrorInvalidValue;
+  if (n <= 352) return run(k_sp2_tile<1, 16>, 16, 1024);   // 22 tiles a side at most: 253 workgroups
+  if (n <= 704) return run(k_sp2_tile<2, 16>, 32, 1024);
+  return run(k_sp2_tile<3, 8>, 48, 512);
+}
+
+hipError_t launch_sp2_settle(int nocc, double* st, hipStream_t s) {
+  return launch_k(k_sp2_settle, dim3(1), dim3(64), s, nocc, st);
 }
 
 hipError_t launch_diag(int n, const double* R, double* d, hipStream_t s) {

@@ -29,12 +29,13 @@ struct C2SList {
 // SP2 purification state vector (doubles) and limits, shared by host and kernels
 enum Sp2State {
   kSpEmin = 0, kSpEmax = 1, kSpFlag = 2, kSpCount = 3, kSpIter = 4, kSpErr = 5, kSpTrace = 6,
-  kSpResid = 7, kSpMinPiv = 8, kSpHist = 16
+  kSpResid = 7, kSpMinPiv = 8, kSpPend = 9, kSpNPart = 10, kSpHead = 16
 };
 constexpr int kSp2MaxIter = 128;
 constexpr int kSp2Groups = 512;       // workgroups of the SP2 update (partial trace sums)
-constexpr int kSpPart = kSpHist + kSp2MaxIter;  // their partial sums: 2 kSp2Groups doubles
-constexpr int kSp2State = kSpPart + 2 * kSp2Groups;
+constexpr int kSpPart = kSpHead;      // their partial sums: 2 kSp2Groups doubles
+constexpr int kSp2State = kSpPart + 2 * kSp2Groups;  // one state; the tiled steps alternate between two
+constexpr int kSp2TileN = 1056;       // widest n of the tiled steps (at most 253 tiles)
 constexpr int kSp2Block = 4;          // purification iterations per graph launch (divides kSp2MaxIter)
 // widest compact-grid block (functions) the fused mixed-precision XC kernels take
 constexpr int kXfMaxN = 2048;

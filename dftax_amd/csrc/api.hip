@@ -168,6 +168,10 @@ hipError_t launch_sp2_step(int n, const double* X, double* Xn, int nocc, double*
 hipError_t launch_sp2_tile(int n, const double* X, double* Xn, int nocc, const double* st, double* stn,
                            hipStream_t s);
 hipError_t launch_sp2_settle(int nocc, double* st, hipStream_t s);
+int pfactor_panel(int n);
+int pfactor_max_n();
+hipError_t launch_pfactor(int n, int c0, int npanel, double tol, double* R, double* d, double* L, double* st,
+                          double* part, hipStream_t s);
 hipError_t launch_diag(int n, const double* R, double* d, hipStream_t s);
 hipError_t launch_pchol_panel(int n, int k0, int b, const double* R, double* d, double* L, int32_t* piv, double* st,
                               int last, hipStream_t s);
@@ -2037,10 +2041,40 @@ void energy_fock_factored(dfks_ctx* h, const double* P, const double* Cf, const 
   h->mark(kStFock + 1, st);
 }
 
-// signed eigen-factorisation of a symmetric P (positive columns first); signs to sg
+// P = L L^T of a positive semidefinite P by pivoted Cholesky (columns to d_Cf), stopped where the residual's
+// diagonal is down to rounding, 1e-14 of P's largest diagonal element, the relative cutoff of the eigenvalues
+// below. Returns the number of columns, -1 when the residual is not down to rounding everywhere, as for an
+// indefinite or unsymmetric P (or past the kernel's size).
+int factor_psd(dfks_ctx* h, const double* P, hipStream_t st) {
+  const int nao = h->nao, pb = pfactor_panel(nao);
+  const double tol = 1e-14;
+  if (nao > pfactor_max_n()) return -1;
+  HIPCHK(hipMemcpyAsync(h->d_W1, P, sizeof(double) * nao * nao, hipMemcpyDeviceToDevice, st));
+  // as many panels as the occupied orbitals need and the column that finds the rank, then four at a time
+  int np = std::max(h->nocc, h->nocc_b) / pb + 1;
+  for (int c0 = 0; c0 < nao; c0 += np * pb, np = 4) {
+    HIPCHK(launch_pfactor(nao, c0, np, tol, h->d_W1, h->d_evals, h->d_Cf, h->d_part, h->d_gws, st));
+    double s[4];
+    HIPCHK(hipMemcpyAsync(s, h->d_part, sizeof(s), hipMemcpyDeviceToHost, st));
+    sync(st);
+    if (s[2] != 0.0) return s[3] <= 8.0 * tol * s[0] ? (int)s[1] : -1;
+  }
+  return -1;
+}
+
+// Factor of a symmetric P = sum_i s_i c_i c_i^T, signs to sg: factor_psd (all signs +1), else the signed
+// eigen-factorisation (positive columns first), whose ~1000 small kernels took most of a small system's Fock
+// build: one water def2-SVP 750 -> 230 us, 41 occupied orbitals at n = 230 (two exchange terms) 6.7 -> 2.2 ms.
+// The eigenvalues of rounding noise also became exchange columns (27 beside the 41), the pivoted Cholesky
+// stops before them.
 int factor_density(dfks_ctx* h, const double* P, std::vector<double>& sg, hipStream_t st) {
   const int nao = h->nao;
   RBCHK(rocblas_set_stream(h->rb, st));
+  const int np = factor_psd(h, P, st);
+  if (np >= 0) {
+    sg.assign(np, 1.0);
+    return np;
+  }
   HIPCHK(hipMemcpyAsync(h->d_W1, P, sizeof(double) * nao * nao, hipMemcpyDeviceToDevice, st));
   RBCHK(rocsolver_dsyevd(h->rb, rocblas_evect_original, rocblas_fill_upper, nao, h->d_W1, nao, h->d_evals, h->d_offd,
                          h->d_info));

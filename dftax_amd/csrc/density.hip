@@ -577,6 +577,168 @@ __global__ __launch_bounds__(64) void k_sp2_settle(int nocc, double* st) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Factor P = L L^T of a positive semidefinite density matrix by pivoted Cholesky
+// that stops at its rank: st = {largest diagonal of P, columns so far, done}.
+// A panel of PB columns per launch, one workgroup, NPT rows per thread; a thread
+// keeps its rows of the panel in registers, so a column is one reduction (the
+// pivot), one row of R and one broadcast of the pivot's panel row: ~2 us each.
+// The rank of an occupied density is small, where the eigendecomposition it
+// replaces runs thousands of kernels whatever the rank.
+// ---------------------------------------------------------------------------
+constexpr int kPfThreads = 512;
+
+template <int NPT, int PB>
+__global__ __launch_bounds__(kPfThreads) void k_pfactor_panel(int n, double tol, const double* __restrict__ R,
+                                                              double* __restrict__ d, double* __restrict__ L,
+                                                              double* __restrict__ st) {
+  constexpr int NW = kPfThreads / 64;
+  __shared__ double s_v[2][NW];
+  __shared__ int s_i[2][NW];
+  __shared__ double s_row[PB];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int k0 = (int)st[1];
+  if (st[2] != 0.0 || k0 >= n) return;
+  double dv[NPT], Lr[NPT][PB];
+#pragma unroll
+  for (int q = 0; q < NPT; ++q) {
+    const int i = tid + q * kPfThreads;
+    dv[q] = i < n ? (k0 == 0 ? R[(int64_t)i * n + i] : d[i]) : -1e300;
+  }
+  double dmax = st[0];
+  int done = 0, cols = 0;
+#pragma unroll
+  for (int j = 0; j < PB; ++j) {
+    // pivot: largest residual diagonal, lowest index among equals
+    double bv = -1e300;
+    int bi = n;
+#pragma unroll
+    for (int q = 0; q < NPT; ++q)
+      if (dv[q] > bv) {
+        bv = dv[q];
+        bi = tid + q * kPfThreads;
+      }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const double ov = __shfl_xor(bv, o);
+      const int oi = __shfl_xor(bi, o);
+      if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
+    }
+    if (lane == 0) {
+      s_v[j & 1][wv] = bv;
+      s_i[j & 1][wv] = bi;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const double ov = s_v[j & 1][w];
+      const int oi = s_i[j & 1][w];
+      if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
+    }
+    if (k0 == 0 && j == 0) dmax = bv;
+    if (!(bv > tol * dmax) || bi >= n || k0 + j >= n) {   // the same in every thread
+      done = 1;
+      break;
+    }
+    const int p = bi;
+    double c[NPT];
+#pragma unroll
+    for (int q = 0; q < NPT; ++q) {
+      const int i = tid + q * kPfThreads;
+      c[q] = R[(int64_t)p * n + min(i, n - 1)];
+      if (i == p) {
+#pragma unroll
+        for (int t = 0; t < PB; ++t)
+          if (t < j) s_row[t] = Lr[q][t];
+      }
+    }
+    __syncthreads();
+    const double inv = 1.0 / sqrt(bv);
+#pragma unroll
+    for (int q = 0; q < NPT; ++q) {
+      const int i = tid + q * kPfThreads;
+#pragma unroll
+      for (int t = 0; t < PB; ++t)
+        if (t < j) c[q] -= Lr[q][t] * s_row[t];
+      c[q] *= inv;
+      Lr[q][j] = c[q];
+      if (i < n) {
+        L[(int64_t)(k0 + j) * n + i] = c[q];
+        dv[q] = i == p ? -1e300 : dv[q] - c[q] * c[q];
+      }
+    }
+    ++cols;
+  }
+#pragma unroll
+  for (int q = 0; q < NPT; ++q) {
+    const int i = tid + q * kPfThreads;
+    if (i < n) d[i] = dv[q];
+  }
+  // a diagonal below zero by more than rounding: not semidefinite, no need to look for its rank
+  bool neg = false;
+#pragma unroll
+  for (int q = 0; q < NPT; ++q) neg |= dv[q] < -8.0 * tol * dmax && dv[q] > -1e299;
+  if (__syncthreads_or(neg)) done = 1;
+  if (tid == 0) {
+    st[0] = dmax;
+    st[1] = (double)(k0 + cols);
+    st[2] = done || k0 + cols >= n ? 1.0 : 0.0;
+  }
+}
+
+// R -= L_p L_p^T of the panel's columns k0 .. k0 + pb - 1 as far as they were formed, and the largest |R_ij|
+// of each 32 x 32 tile (one workgroup) into part.
+__global__ __launch_bounds__(256) void k_pfactor_update(int n, int k0, int pb, const double* __restrict__ L,
+                                                        double* __restrict__ R, const double* __restrict__ st,
+                                                        double* __restrict__ part) {
+  __shared__ double s_a[32][33], s_b[32][33];
+  __shared__ double s_m[4];
+  const int nt = (n + 31) / 32, m0 = 32 * (blockIdx.x / nt), n0 = 32 * (blockIdx.x % nt);
+  const int tid = threadIdx.x, c = tid & 31, r0 = tid >> 5;
+  const int kn = min(pb, (int)st[1] - k0);
+  for (int k = r0; k < 32; k += 8) {
+    const bool in = k < kn;
+    const double* row = L + (int64_t)(k0 + (in ? k : 0)) * n;
+    s_a[k][c] = in && m0 + c < n ? row[m0 + c] : 0.0;
+    s_b[k][c] = in && n0 + c < n ? row[n0 + c] : 0.0;
+  }
+  __syncthreads();
+  double mx = 0.0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int r = r0 + 8 * e;
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < 32; ++k) s += s_a[k][r] * s_b[k][c];
+    if (m0 + r < n && n0 + c < n) {
+      const int64_t at = (int64_t)(m0 + r) * n + n0 + c;
+      const double v = R[at] - s;
+      R[at] = v;
+      mx = v == v ? fmax(mx, fabs(v)) : 1e300;   // a NaN must not pass for small
+    }
+  }
+  for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
+  if ((tid & 63) == 0) s_m[tid >> 6] = mx;
+  __syncthreads();
+  if (tid == 0) part[blockIdx.x] = fmax(fmax(s_m[0], s_m[1]), fmax(s_m[2], s_m[3]));
+}
+
+// st[3] = the largest of the np workgroup maxima
+__global__ __launch_bounds__(256) void k_pfactor_max(int np, const double* __restrict__ part, double* __restrict__ st) {
+  __shared__ double s_m[4];
+  double mx = 0.0;
+  for (int i = threadIdx.x; i < np; i += 256) mx = fmax(mx, part[i]);
+  for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
+  if ((threadIdx.x & 63) == 0) s_m[threadIdx.x >> 6] = mx;
+  __syncthreads();
+  if (threadIdx.x == 0) st[3] = fmax(fmax(s_m[0], s_m[1]), fmax(s_m[2], s_m[3]));
+}
+
+// st = 0 (the first panel of a factorisation follows)
+__global__ void k_pfactor_reset(double* __restrict__ st) {
+  if (threadIdx.x < 4) st[threadIdx.x] = 0.0;
+}
+
 // d[i] = R_ii
 __global__ void k_diag(int n, const double* __restrict__ R, double* __restrict__ d) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -965,6 +1127,34 @@ hipError_t launch_sp2_tile(int n, const double* X, double* Xn, int nocc, const d
 
 hipError_t launch_sp2_settle(int nocc, double* st, hipStream_t s) {
   return launch_k(k_sp2_settle, dim3(1), dim3(64), s, nocc, st);
+}
+
+int pfactor_panel(int n) { return n <= 2 * kPfThreads ? 32 : 16; }   // columns per panel
+int pfactor_max_n() { return 4 * kPfThreads; }
+
+// npanel panels of the pivoted Cholesky of R (n x n, destroyed; d: n words, L: column-major, room for n
+// columns), from column c0 (a multiple of the panel; 0 starts afresh): st[0..3] = largest diagonal, columns,
+// done, largest |R_ij| left. part: at least ceil(n / 32)^2 words.
+hipError_t launch_pfactor(int n, int c0, int npanel, double tol, double* R, double* d, double* L, double* st,
+                          double* part, hipStream_t s) {
+  if (n < 1 || n > pfactor_max_n()) return hipErrorInvalidValue;
+  const int pb = pfactor_panel(n), nt = (n + 31) / 32;
+  hipError_t e = hipSuccess;
+  if (c0 == 0) e = launch_k(k_pfactor_reset, dim3(1), dim3(64), s, st);
+  for (int p = 0; p < npanel && e == hipSuccess; ++p) {
+    const int k0 = c0 + p * pb;
+    if (k0 >= n) break;
+    if (n <= kPfThreads)
+      e = launch_k(k_pfactor_panel<1, 32>, dim3(1), dim3(kPfThreads), s, n, tol, R, d, L, st);
+    else if (n <= 2 * kPfThreads)
+      e = launch_k(k_pfactor_panel<2, 32>, dim3(1), dim3(kPfThreads), s, n, tol, R, d, L, st);
+    else
+      e = launch_k(k_pfactor_panel<4, 16>, dim3(1), dim3(kPfThreads), s, n, tol, R, d, L, st);
+    if (e == hipSuccess)
+      e = launch_k(k_pfactor_update, dim3((unsigned)(nt * nt)), dim3(256), s, n, k0, pb, L, R, st, part);
+  }
+  if (e == hipSuccess) e = launch_k(k_pfactor_max, dim3(1), dim3(256), s, nt * nt, part, st);
+  return e;
 }
 
 hipError_t launch_diag(int n, const double* R, double* d, hipStream_t s) {

@@ -47,6 +47,8 @@ hipError_t launch_eri_thread(int la, int lb, int lc, const int2* pairs, int npai
 hipError_t launch_eri_pair(int la, int lb, int lc, const int2* pairs, int npair, const int32_t* aux, int naux_l,
                            const ShellSet& A, const ShellSet& C, const double* boys, double* out, int64_t sa,
                            int64_t sb, int64_t c0, int tr, hipStream_t st);
+hipError_t launch_eri2_pair(int la, int lc, const int2* pairs, int nshell, const int32_t* aux, int naux_l,
+                            const ShellSet& A, const double* boys, double* out, int64_t sa, hipStream_t st);
 hipError_t launch_int1e(const ShellSet& A, int natm, const double* atm, const double* boys, double* S, double* T,
                         double* V, int64_t nao, hipStream_t stream);
 hipError_t launch_becke(int64_t n, const double* pts, const double* raw, const int32_t* owner, int natm,
@@ -116,6 +118,11 @@ hipError_t launch_to_f64(int64_t n, const float* x, double* y, hipStream_t st);
 hipError_t launch_eri_grad(const int2* pairs, int npair, int nket, const ShellSet& A, const ShellSet& C,
                            const int32_t* atom_a, const int32_t* atom_c, int b_unit, const double* boys,
                            const double* G, int64_t nao_g, double* grad, hipStream_t st);
+bool eri_pair_grad_has(int la, const ShellSet& A, const ShellSet& C, int natom, int unit);
+hipError_t launch_eri_pair_grad(int la, int lb, int lc, const int2* pairs, int npair, const int32_t* aux, int naux_l,
+                                const ShellSet& A, const ShellSet& C, const int32_t* atom_a, const int32_t* atom_c,
+                                int natom, int unit, const double* boys, const double* G, int64_t gc, int64_t ga,
+                                int64_t gb, double* grad, hipStream_t st);
 hipError_t launch_int1e_grad(const ShellSet& A, const int32_t* atom_a, int natm, const double* atm,
                              const double* boys, const double* P, const double* W, int64_t nao, double* grad,
                              hipStream_t st);
@@ -778,6 +785,13 @@ hipError_t launch_eri3(int la, int lb, int lc, const int2* pairs, int npair, con
   return launch_eri_cls(la, lb, lc, pairs, npair, aux, naux_l, A, C, boys, out, sa, sb, c0, tr, st);
 }
 
+// One class of (P|Q) into out[P * sa + Q]: by bra shell where the span is spherical, else a wavefront per task.
+hipError_t launch_eri2(int la, int lc, const int2* shells, int nshell, const int32_t* aux, int naux_l,
+                       const ShellSet& A, const double* boys, double* out, int64_t sa, hipStream_t st) {
+  if (A.spherical) return launch_eri2_pair(la, lc, shells, nshell, aux, naux_l, A, boys, out, sa, st);
+  return launch_eri_wave(la, 0, lc, shells, nshell, aux, naux_l, A, A, 1, boys, out, sa, 0, 0, 0, st);
+}
+
 // Recompute mode: auxiliary slabs (runs of whole shells of at most aux_chunk
 // functions) with their per-lc shell lists, and the slab-sized buffers.
 void setup_slabs(dfks_ctx* h, hipStream_t st) {
@@ -1161,8 +1175,8 @@ void build_all(dfks_ctx* h, hipStream_t st) {
   h->d_int2c = dalloc<double>((size_t)naux * naux);
   for (int la = 0; la <= lx; ++la)
     for (int lc = 0; lc <= lx; ++lc)
-      HIPCHK(launch_eri_wave(la, 0, lc, d_pairs + apair_off[la], (int)apairs[la].size(), d_auxl + aux_off[lc],
-                             (int)auxl[lc].size(), A, A, 1, h->d_boys, h->d_int2c, naux, 0, 0, 0, st));
+      HIPCHK(launch_eri2(la, lc, d_pairs + apair_off[la], (int)apairs[la].size(), d_auxl + aux_off[lc],
+                         (int)auxl[lc].size(), A, h->d_boys, h->d_int2c, naux, st));
   sync(st);
   h->build_ms[1] = now_ms() - t0;
   t0 = now_ms();
@@ -1323,8 +1337,8 @@ void build_all(dfks_ctx* h, hipStream_t st) {
     double* d2lr = dalloc<double>((size_t)naux * naux);
     for (int la = 0; la <= lx; ++la)
       for (int lc = 0; lc <= lx; ++lc)
-        HIPCHK(launch_eri_wave(la, 0, lc, d_pairs + apair_off[la], (int)apairs[la].size(), d_auxl + aux_off[lc],
-                               (int)auxl[lc].size(), Aw, Aw, 1, h->d_boys, d2lr, naux, 0, 0, 0, st));
+        HIPCHK(launch_eri2(la, lc, d_pairs + apair_off[la], (int)apairs[la].size(), d_auxl + aux_off[lc],
+                           (int)auxl[lc].size(), Aw, h->d_boys, d2lr, naux, st));
     double* d3lr = dalloc<double>((size_t)nao * nao * naux);
     if (h->slab_zero) HIPCHK(hipMemsetAsync(d3lr, 0, sizeof(double) * nao * nao * naux, st));
     for (int la = 0; la <= lo; ++la)
@@ -2378,16 +2392,65 @@ void forces_run(dfks_ctx* h, const double* Co, int nocc, int64_t ng, const doubl
                                       h->d_Tx, (int64_t)nfit * nocc, nocc, Cf, nao, 0, &kZero, Aq, nocc, no2, nfit));
   double* D = alloc((size_t)naux * no2);    // [P][i][j]
   gemm(h, false, false, no2, naux, nfit, 1.0, Aq, no2, h->d_Lt, nfit, 0.0, D, no2);
-  // pairs (ia >= ib) of orbital shells, and the auxiliary shells with a unit partner
-  std::vector<int2> pr;
-  for (int a = 0; a < h->orb.n(); ++a)
-    for (int b = 0; b <= a; ++b) pr.push_back(make_int2(a, b));
-  std::vector<int2> apr;
-  for (int c = 0; c < h->aux.n(); ++c) apr.push_back(make_int2(c, c));
+  // pairs of orbital shells by class (la >= lb, ia >= ib within one l), the auxiliary shells by l, alone and
+  // with a unit partner
+  const int lo = h->orb.maxl(), lx = h->aux.maxl();
+  std::vector<int2> pr, apr;
+  std::vector<int32_t> axl;
+  std::vector<size_t> pr_off, apr_off;
+  for (int la = 0; la <= lo; ++la)
+    for (int lb = 0; lb <= la; ++lb) {
+      pr_off.push_back(pr.size());
+      for (int a = 0; a < h->orb.n(); ++a)
+        for (int b = 0; b < h->orb.n(); ++b)
+          if (h->orb.l[a] == la && h->orb.l[b] == lb && (la != lb || b <= a)) pr.push_back(make_int2(a, b));
+    }
+  pr_off.push_back(pr.size());
+  for (int lc = 0; lc <= lx; ++lc) {
+    apr_off.push_back(apr.size());
+    for (int c = 0; c < h->aux.n(); ++c)
+      if (h->aux.l[c] == lc) {
+        apr.push_back(make_int2(c, c));
+        axl.push_back(c);
+      }
+  }
+  apr_off.push_back(apr.size());
   int2* d_pr = reinterpret_cast<int2*>(alloc_i(2 * pr.size()));
   int2* d_apr = reinterpret_cast<int2*>(alloc_i(2 * apr.size()));
+  int32_t* d_axl = alloc_i(axl.size());
   up(d_pr, pr.data(), pr.size());
   up(d_apr, apr.data(), apr.size());
+  up(d_axl, axl.data(), axl.size());
+  // Gamma3 [P][m][n] and Gamma2 [P][Q] with the integral derivatives, by class (a wavefront per task where a
+  // span is cartesian with l >= 2)
+  const auto contract = [&](const double* g3, const double* g2, double* out_grad) {
+    int cls = 0;
+    for (int la = 0; la <= lo; ++la)
+      for (int lb = 0; lb <= la; ++lb, ++cls) {
+        const int2* pp = d_pr + pr_off[cls];
+        const int np = (int)(pr_off[cls + 1] - pr_off[cls]);
+        if (np == 0) continue;
+        if (!eri_pair_grad_has(la, O, X, natom, 0)) {
+          HIPCHK(launch_eri_grad(pp, np, h->aux.n(), O, X, d_at_o, d_at_x, 0, h->d_boys, g3, nao, out_grad, st));
+          continue;
+        }
+        for (int lc = 0; lc <= lx; ++lc)
+          HIPCHK(launch_eri_pair_grad(la, lb, lc, pp, np, d_axl + apr_off[lc], (int)(apr_off[lc + 1] - apr_off[lc]), O,
+                                      X, d_at_o, d_at_x, natom, 0, h->d_boys, g3, nn, nao, 1, out_grad, st));
+      }
+    for (int la = 0; la <= lx; ++la) {
+      const int2* pp = d_apr + apr_off[la];
+      const int np = (int)(apr_off[la + 1] - apr_off[la]);
+      if (np == 0) continue;
+      if (!eri_pair_grad_has(la, X, X, natom, 1)) {
+        HIPCHK(launch_eri_grad(pp, np, h->aux.n(), X, X, d_at_x, d_at_x, 1, h->d_boys, g2, naux, out_grad, st));
+        continue;
+      }
+      for (int lc = 0; lc <= lx; ++lc)
+        HIPCHK(launch_eri_pair_grad(la, 0, lc, pp, np, d_axl + apr_off[lc], (int)(apr_off[lc + 1] - apr_off[lc]), X, X,
+                                    d_at_x, d_at_x, natom, 1, h->d_boys, g2, 1, naux, 0, out_grad, st));
+    }
+  };
   double* G2 = alloc((size_t)naux * naux);
   double* G3 = alloc((size_t)naux * nn);
   // Coulomb: Gamma_P = d_P P, Gamma2 = -1/2 d d^T
@@ -2397,9 +2460,7 @@ void forces_run(dfks_ctx* h, const double* Co, int nocc, int64_t ng, const doubl
                        P, G3);
     HIPCHK(hipGetLastError());
     gemm(h, false, true, naux, naux, 1, -0.5, dvec, naux, dvec, naux, 0.0, G2, naux);
-    HIPCHK(launch_eri_grad(d_pr, (int)pr.size(), h->aux.n(), O, X, d_at_o, d_at_x, 0, h->d_boys, G3, nao, gp[1], st));
-    HIPCHK(launch_eri_grad(d_apr, (int)apr.size(), h->aux.n(), X, X, d_at_x, d_at_x, 1, h->d_boys, G2, naux, gp[1],
-                           st));
+    contract(G3, G2, gp[1]);
   }
   // exchange: Gamma_P = -a_x/2 Cf D^P Cf^T, Gamma2 = a_x/4 D D^T
   if (ax != 0.0) {
@@ -2410,9 +2471,7 @@ void forces_run(dfks_ctx* h, const double* Co, int nocc, int64_t ng, const doubl
     RBCHK(rocblas_dgemm_strided_batched(h->rb, rocblas_operation_none, rocblas_operation_transpose, nao, nao, nocc,
                                         &sk, Xp, nao, (int64_t)nao * nocc, Cf, nao, 0, &kZero, G3, nao, nn, naux));
     gemm(h, true, false, naux, naux, no2, 0.25 * ax, D, no2, D, no2, 0.0, G2, naux);
-    HIPCHK(launch_eri_grad(d_pr, (int)pr.size(), h->aux.n(), O, X, d_at_o, d_at_x, 0, h->d_boys, G3, nao, gp[2], st));
-    HIPCHK(launch_eri_grad(d_apr, (int)apr.size(), h->aux.n(), X, X, d_at_x, d_at_x, 1, h->d_boys, G2, naux, gp[2],
-                           st));
+    contract(G3, G2, gp[2]);
   }
 
   // XC on the caller's atom-centred grid (no weight cutoff), in chunks of points

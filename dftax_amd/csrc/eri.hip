@@ -477,6 +477,7 @@ hipError_t launch_schwarz(int la, int lb, const int2* pairs, int npair, const Sh
 // ---------------------------------------------------------------------------
 void upload_cls_tables(const C2SList& h, const int (&cart)[7][28][3]);
 void upload_pair_tables(const C2SList& h, const int (&cart)[7][28][3]);
+void upload_pair_grad_tables(const C2SList& h, const int (&cart)[7][28][3]);
 
 void upload_c2s_tables() {
   static C2SList h;
@@ -507,6 +508,7 @@ void upload_c2s_tables() {
   (void)hipMemcpyToSymbol(HIP_SYMBOL(g_cart), cart, sizeof(cart));
   upload_cls_tables(h, cart);
   upload_pair_tables(h, cart);
+  upload_pair_grad_tables(h, cart);
 }
 
 hipError_t launch_eri_wave(int la, int lb, int lc, const int2* pairs, int npair, const int32_t* aux, int naux_l,

@@ -33,15 +33,11 @@
 #include <algorithm>
 #include <cstdint>
 
-#include "dfks_common.h"
+#include "eri_pair.h"
 
 namespace dfks {
 
 namespace {
-
-typedef double dbl4 __attribute__((ext_vector_type(4)));
-
-__host__ __device__ constexpr int n_tet(int L) { return (L + 1) * (L + 2) * (L + 3) / 6; }
 
 // A class's sizes: AB rows and Hermite indices padded to the MFMA shape, R entries of order >= LC
 template <int LA, int LB, int LC>
@@ -58,116 +54,6 @@ struct PairCls {
   static constexpr int NPC = HSZ > 2304 ? 1 : (2304 / HSZ > 36 ? 36 : 2304 / HSZ);
   static constexpr int NW = NR * 16 > 2600 ? 2 : 4;
   static constexpr int OCC = MT * NM * 8 > 80 ? 1 : 2;
-};
-
-__constant__ C2SList g_c2s_pair;
-__constant__ int g_cart_pair[7][28][3];
-
-// E^{ij}_t of one axis into E[(i (LB+1) + j) (LAB+1) + t], zero where t > i + j
-template <int LA, int LB>
-__device__ __forceinline__ void e_axis(double xpa, double xpb, double i2p, double* __restrict__ out) {
-  constexpr int MT = LA + LB + 1;
-  double E[LA + 1][LB + 1][MT];
-#pragma unroll
-  for (int i = 0; i <= LA; ++i)
-#pragma unroll
-    for (int j = 0; j <= LB; ++j)
-#pragma unroll
-      for (int t = 0; t < MT; ++t) E[i][j][t] = 0.0;
-  E[0][0][0] = 1.0;
-#pragma unroll
-  for (int i = 0; i < LA; ++i)
-#pragma unroll
-    for (int t = 0; t <= i + 1; ++t) {
-      double v = xpa * E[i][0][t];
-      if (t > 0) v += i2p * E[i][0][t - 1];
-      if (t + 1 <= i) v += (t + 1) * E[i][0][t + 1];
-      E[i + 1][0][t] = v;
-    }
-#pragma unroll
-  for (int j = 0; j < LB; ++j)
-#pragma unroll
-    for (int i = 0; i <= LA; ++i)
-#pragma unroll
-      for (int t = 0; t <= i + j + 1; ++t) {
-        double v = xpb * E[i][j][t];
-        if (t > 0) v += i2p * E[i][j][t - 1];
-        if (t + 1 <= i + j) v += (t + 1) * E[i][j][t + 1];
-        E[i][j + 1][t] = v;
-      }
-#pragma unroll
-  for (int i = 0; i <= LA; ++i)
-#pragma unroll
-    for (int j = 0; j <= LB; ++j)
-#pragma unroll
-      for (int t = 0; t < MT; ++t) out[(i * (LB + 1) + j) * MT + t] = E[i][j][t];
-}
-
-// One plane v of R: the (t,u) triangle of order <= TOP by the in-place ladder from Z[n] = R^(n)_00v
-template <int TOP>
-__device__ __forceinline__ void r_plane(double x, double y, const double* Z, double* X) {
-  X[0] = Z[TOP];
-#pragma unroll
-  for (int m = TOP - 1; m >= 0; --m) {
-#pragma unroll
-    for (int r = TOP - m; r >= 1; --r)
-#pragma unroll
-      for (int u = 0; u <= r; ++u) {
-        const int t = r - u, e = r * (r + 1) / 2 + u;
-        if (t > 0) {
-          double v = x * X[(r - 1) * r / 2 + u];
-          if (t > 1) v += (t - 1) * X[(r - 2) * (r - 1) / 2 + u];
-          X[e] = v;
-        } else {
-          double v = y * X[(r - 1) * r / 2 + u - 1];
-          if (u > 1) v += (u - 1) * X[(r - 2) * (r - 1) / 2 + u - 2];
-          X[e] = v;
-        }
-      }
-    X[0] = Z[m];
-  }
-}
-
-// Planes v = V0 + sub of this lane, then V0 + 4 + sub, ...: ladder in registers, entries of order
-// LC .. L to Rw[index - R0][16 lanes]
-template <int L, int LC, int R0, int V0>
-__device__ __forceinline__ void r_planes(double x, double y, double z, int v, double* Zc, double* Zp,
-                                         double* __restrict__ Rw) {
-  if constexpr (V0 <= L) {
-    constexpr int TOP = L - V0;
-    double X[(TOP + 1) * (TOP + 2) / 2];
-    r_plane<TOP>(x, y, Zc, X);
-    const int vb = v * (v + 1) / 2 + v - R0;
-#pragma unroll
-    for (int r = 0; r <= TOP; ++r) {
-      const int s = r + v;
-      if (s >= LC && s <= L) {
-        double* dst = Rw + (s * (s + 1) * (s + 2) / 6 + vb) * 16;
-#pragma unroll
-        for (int u = 0; u <= r; ++u) dst[(u * (u + 1) / 2 + u * v) * 16] = X[r * (r + 1) / 2 + u];
-      }
-    }
-    if constexpr (V0 + 4 <= L) {
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const double fv = (double)(v + k);
-#pragma unroll
-        for (int n = 0; n + V0 < L; ++n) {
-          const double nz = z * Zc[n + 1] + fv * Zp[n + 1];
-          Zp[n] = Zc[n];
-          Zc[n] = nz;
-        }
-      }
-      r_planes<L, LC, R0, V0 + 4>(x, y, z, v + 4, Zc, Zp, Rw);
-    }
-  }
-}
-
-// The bra shell pair: its primitives' slices and centres
-struct BraPair {
-  const double *ea, *eb, *ca, *cb;
-  const double *xa, *xb;
-  int npb;
 };
 
 // H (rows row0 ..), P and p of the primitive pairs q0 .. q0 + n - 1 into LDS, by the whole workgroup
@@ -229,7 +115,7 @@ template <int LA, int LB, int LC>
 __global__ __launch_bounds__((PairCls<LA, LB, LC>::NW * 64), (PairCls<LA, LB, LC>::OCC)) void k_eri_pair(
     const int2* __restrict__ pairs, const int32_t* __restrict__ aux, int naux_l, ShellSet A, ShellSet C,
     const double* __restrict__ boys, double* __restrict__ out, int64_t sa, int64_t sb, int64_t c0, int tr,
-    int gper) {
+    int gper, int unit) {
   using K = PairCls<LA, LB, LC>;
   constexpr int L = K::L, LAB = K::LAB, FA = K::FA, FB = K::FB, NM = K::NM, MT = K::MT, KQ = K::KQ, NH = K::NH;
   constexpr int NT = K::NW * 64;
@@ -245,10 +131,9 @@ __global__ __launch_bounds__((PairCls<LA, LB, LC>::NW * 64), (PairCls<LA, LB, LC
   const int2 pr = pairs[blockIdx.x];
   const int row0 = blockIdx.z * (MT * 16);   // first AB row of this workgroup's tiles
   const int ia = pr.x, ib = pr.y;
-  const int npb = A.nprim[ib], npp = A.nprim[ia] * npb;
-  const BraPair bp{A.exps + A.prim0[ia], A.exps + A.prim0[ib], A.coefs + A.prim0[ia], A.coefs + A.prim0[ib],
-                   A.centre + 3 * ia, A.centre + 3 * ib, npb};
-  const int64_t ao_a = A.ao0[ia], ao_b = A.ao0[ib];
+  const BraPair bp = bra_pair(A, ia, ib, unit != 0);
+  const int npp = A.nprim[ia] * bp.npb;
+  const int64_t ao_a = A.ao0[ia], ao_b = unit ? 0 : A.ao0[ib];
 
   for (int h = tid; h < KQ * 4; h += NT) {
     int s = 0, e = h < NH ? h : 0;
@@ -385,7 +270,8 @@ __global__ __launch_bounds__((PairCls<LA, LB, LC>::NW * 64), (PairCls<LA, LB, LC
 
 template <int LA, int LB, int LC>
 hipError_t go_pair(const int2* pairs, int npair, const int32_t* aux, int naux_l, const ShellSet& A, const ShellSet& C,
-                   const double* boys, double* out, int64_t sa, int64_t sb, int64_t c0, int tr, hipStream_t st) {
+                   const double* boys, double* out, int64_t sa, int64_t sb, int64_t c0, int tr, hipStream_t st,
+                   int unit = 0) {
   using K = PairCls<LA, LB, LC>;
   const int ngrp = (naux_l + 15) / 16;
   // auxiliary segments: enough workgroups for the chip, at least one group per wavefront
@@ -394,7 +280,7 @@ hipError_t go_pair(const int2* pairs, int npair, const int32_t* aux, int naux_l,
   gper = (gper + K::NW - 1) / K::NW * K::NW;
   const dim3 grid((unsigned)npair, (unsigned)((ngrp + gper - 1) / gper), (unsigned)K::PARTS);
   hipLaunchKernelGGL((k_eri_pair<LA, LB, LC>), grid, dim3(K::NW * 64), 0, st, pairs, aux, naux_l, A, C, boys, out, sa,
-                     sb, c0, tr, gper);
+                     sb, c0, tr, gper, unit);
   return hipGetLastError();
 }
 
@@ -426,6 +312,28 @@ hipError_t launch_eri_pair(int la, int lb, int lc, const int2* pairs, int npair,
   DFKS_PAIR(0, 0) DFKS_PAIR(1, 0) DFKS_PAIR(1, 1) DFKS_PAIR(2, 0) DFKS_PAIR(2, 1) DFKS_PAIR(2, 2)
   DFKS_PAIR(3, 0) DFKS_PAIR(3, 1) DFKS_PAIR(3, 2) DFKS_PAIR(3, 3)
 #undef DFKS_PAIR
+  return hipErrorInvalidValue;
+}
+
+// Two-centre (p|c), one class: p over the nshell shells of `pairs` (x: the shell), l_p <= 4, into
+// out[p * sa + c]; spherical where l >= 2 (the caller checks).
+hipError_t launch_eri2_pair(int la, int lc, const int2* pairs, int nshell, const int32_t* aux, int naux_l,
+                            const ShellSet& A, const double* boys, double* out, int64_t sa, hipStream_t st) {
+  if (nshell == 0 || naux_l == 0) return hipSuccess;
+  if (!A.spherical) return hipErrorInvalidValue;
+#define DFKS_PAIR2(a) \
+  if (la == a) { \
+    switch (lc) { \
+      case 0: return go_pair<a, 0, 0>(pairs, nshell, aux, naux_l, A, A, boys, out, sa, 0, 0, 0, st, 1); \
+      case 1: return go_pair<a, 0, 1>(pairs, nshell, aux, naux_l, A, A, boys, out, sa, 0, 0, 0, st, 1); \
+      case 2: return go_pair<a, 0, 2>(pairs, nshell, aux, naux_l, A, A, boys, out, sa, 0, 0, 0, st, 1); \
+      case 3: return go_pair<a, 0, 3>(pairs, nshell, aux, naux_l, A, A, boys, out, sa, 0, 0, 0, st, 1); \
+      case 4: return go_pair<a, 0, 4>(pairs, nshell, aux, naux_l, A, A, boys, out, sa, 0, 0, 0, st, 1); \
+      default: return hipErrorInvalidValue; \
+    } \
+  }
+  DFKS_PAIR2(0) DFKS_PAIR2(1) DFKS_PAIR2(2) DFKS_PAIR2(3) DFKS_PAIR2(4)
+#undef DFKS_PAIR2
   return hipErrorInvalidValue;
 }
 

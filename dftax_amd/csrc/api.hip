@@ -14,6 +14,7 @@
 #include <rocsolver/rocsolver.h>
 
 #include <algorithm>
+#include <array>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -49,8 +50,8 @@ hipError_t launch_eri_pair(int la, int lb, int lc, const int2* pairs, int npair,
                            int64_t sb, int64_t c0, int tr, hipStream_t st);
 hipError_t launch_eri2_pair(int la, int lc, const int2* pairs, int nshell, const int32_t* aux, int naux_l,
                             const ShellSet& A, const double* boys, double* out, int64_t sa, hipStream_t st);
-hipError_t launch_int1e(const ShellSet& A, int natm, const double* atm, const double* boys, double* S, double* T,
-                        double* V, int64_t nao, hipStream_t stream);
+hipError_t launch_int1e(int la, int lb, const int2* pairs, int npair, const ShellSet& A, int natm, const double* atm,
+                        const double* boys, double* S, double* T, double* V, int64_t nao, hipStream_t st);
 hipError_t launch_becke(int64_t n, const double* pts, const double* raw, const int32_t* owner, int natm,
                         const double* atm, const double* invR, const double* aAB, double* w, hipStream_t st);
 hipError_t launch_ao(int64_t ng, const double* pts, const ShellSet& S, int64_t nao, double* ao, hipStream_t st);
@@ -123,9 +124,9 @@ hipError_t launch_eri_pair_grad(int la, int lb, int lc, const int2* pairs, int n
                                 const ShellSet& A, const ShellSet& C, const int32_t* atom_a, const int32_t* atom_c,
                                 int natom, int unit, const double* boys, const double* G, int64_t gc, int64_t ga,
                                 int64_t gb, double* grad, hipStream_t st);
-hipError_t launch_int1e_grad(const ShellSet& A, const int32_t* atom_a, int natm, const double* atm,
-                             const double* boys, const double* P, const double* W, int64_t nao, double* grad,
-                             hipStream_t st);
+hipError_t launch_int1e_grad(int la, int lb, const int2* pairs, int npair, const ShellSet& A, const int32_t* atom_a,
+                             int natm, const double* atm, const double* boys, const double* P,
+                             const double* const (&W)[4], int64_t nao, double* grad, int64_t part, hipStream_t st);
 hipError_t launch_ao_hess(int64_t npts, const double* pts, const ShellSet& S, int64_t nao, double* ao,
                           hipStream_t st);
 hipError_t launch_xcg_rho(int64_t npts, int64_t nao, const double* ao, const double* Z, double* rho, double* grad,
@@ -1136,13 +1137,6 @@ void build_all(dfks_ctx* h, hipStream_t st) {
   h->d_T = dalloc<double>((size_t)nao * nao);
   h->d_V = dalloc<double>((size_t)nao * nao);
   h->d_H = dalloc<double>((size_t)nao * nao);
-  HIPCHK(launch_int1e(O, h->natom, h->d_atm, h->d_boys, h->d_S, h->d_T, h->d_V, nao, st));
-  HIPCHK(hipMemcpyAsync(h->d_H, h->d_T, sizeof(double) * nao * nao, hipMemcpyDeviceToDevice, st));
-  HIPCHK(launch_axpy((int64_t)nao * nao, 1.0, h->d_V, h->d_H, 1, st));
-  sync(st);
-  h->build_ms[0] = now_ms() - t0;
-  t0 = now_ms();
-
   h->nf_chunk = std::max(1, std::min(std::min(nao, 512), std::max(h->nocc, 1)));
   // class lists
   const int lo = h->orb.maxl(), lx = h->aux.maxl();
@@ -1170,6 +1164,17 @@ void build_all(dfks_ctx* h, hipStream_t st) {
   int32_t* d_auxl = dalloc<int32_t>(all_aux.size());
   HIPCHK(hipMemcpyAsync(d_pairs, all_pairs.data(), all_pairs.size() * sizeof(int2), hipMemcpyHostToDevice, st));
   HIPCHK(hipMemcpyAsync(d_auxl, all_aux.data(), all_aux.size() * sizeof(int32_t), hipMemcpyHostToDevice, st));
+  for (int la = 0; la <= lo; ++la)
+    for (int lb = 0; lb <= la; ++lb) {
+      const int k = la * (lo + 1) + lb;
+      HIPCHK(launch_int1e(la, lb, d_pairs + pair_off[k], (int)pairs[k].size(), O, h->natom, h->d_atm, h->d_boys, h->d_S,
+                          h->d_T, h->d_V, nao, st));
+    }
+  HIPCHK(hipMemcpyAsync(h->d_H, h->d_T, sizeof(double) * nao * nao, hipMemcpyDeviceToDevice, st));
+  HIPCHK(launch_axpy((int64_t)nao * nao, 1.0, h->d_V, h->d_H, 1, st));
+  sync(st);
+  h->build_ms[0] = now_ms() - t0;
+  t0 = now_ms();
 
   // two-centre metric
   h->d_int2c = dalloc<double>((size_t)naux * naux);
@@ -2377,21 +2382,6 @@ void forces_run(dfks_ctx* h, const double* Co, int nocc, int64_t ng, const doubl
   up(d_at_x, at_x.data(), at_x.size());
   const ShellSet O = h->orb.view(), X = h->aux.view();
 
-  // one-electron and the S-derivative shares of every part
-  HIPCHK(launch_int1e_grad(O, d_at_o, natom, h->d_atm, h->d_boys, P, Wk[0], nao, gp[0], st));
-  for (int k = 1; k < 4; ++k)
-    HIPCHK(launch_int1e_grad(O, d_at_o, natom, h->d_atm, h->d_boys, zero, Wk[k], nao, gp[k], st));
-
-  // density fitting: d = L gamma', (ij|Q) of Cf, D = L (ij|Q)
-  double* dvec = alloc(naux);
-  RBCHK(rocblas_dgemv(h->rb, rocblas_operation_transpose, nfit, naux, &kOne, h->d_Lt, nfit, h->d_gamma, 1, &kZero,
-                      dvec, 1));
-  const int64_t no2 = (int64_t)nocc * nocc;
-  double* Aq = alloc((size_t)nfit * no2);   // [Q][i][j]
-  RBCHK(rocblas_dgemm_strided_batched(h->rb, rocblas_operation_none, rocblas_operation_none, nocc, nocc, nao, &kOne,
-                                      h->d_Tx, (int64_t)nfit * nocc, nocc, Cf, nao, 0, &kZero, Aq, nocc, no2, nfit));
-  double* D = alloc((size_t)naux * no2);    // [P][i][j]
-  gemm(h, false, false, no2, naux, nfit, 1.0, Aq, no2, h->d_Lt, nfit, 0.0, D, no2);
   // pairs of orbital shells by class (la >= lb, ia >= ib within one l), the auxiliary shells by l, alone and
   // with a unit partner
   const int lo = h->orb.maxl(), lx = h->aux.maxl();
@@ -2421,6 +2411,26 @@ void forces_run(dfks_ctx* h, const double* Co, int nocc, int64_t ng, const doubl
   up(d_pr, pr.data(), pr.size());
   up(d_apr, apr.data(), apr.size());
   up(d_axl, axl.data(), axl.size());
+  // one-electron and the S-derivative shares of every part
+  {
+    const double* const W[4] = {Wk[0], Wk[1], Wk[2], Wk[3]};
+    int cls = 0;
+    for (int la = 0; la <= lo; ++la)
+      for (int lb = 0; lb <= la; ++lb, ++cls)
+        HIPCHK(launch_int1e_grad(la, lb, d_pr + pr_off[cls], (int)(pr_off[cls + 1] - pr_off[cls]), O, d_at_o, natom,
+                                 h->d_atm, h->d_boys, P, W, nao, g, na3, st));
+  }
+
+  // density fitting: d = L gamma', (ij|Q) of Cf, D = L (ij|Q)
+  double* dvec = alloc(naux);
+  RBCHK(rocblas_dgemv(h->rb, rocblas_operation_transpose, nfit, naux, &kOne, h->d_Lt, nfit, h->d_gamma, 1, &kZero,
+                      dvec, 1));
+  const int64_t no2 = (int64_t)nocc * nocc;
+  double* Aq = alloc((size_t)nfit * no2);   // [Q][i][j]
+  RBCHK(rocblas_dgemm_strided_batched(h->rb, rocblas_operation_none, rocblas_operation_none, nocc, nocc, nao, &kOne,
+                                      h->d_Tx, (int64_t)nfit * nocc, nocc, Cf, nao, 0, &kZero, Aq, nocc, no2, nfit));
+  double* D = alloc((size_t)naux * no2);    // [P][i][j]
+  gemm(h, false, false, no2, naux, nfit, 1.0, Aq, no2, h->d_Lt, nfit, 0.0, D, no2);
   // Gamma3 [P][m][n] and Gamma2 [P][Q] with the integral derivatives, by class (a wavefront per task where a
   // span is cartesian with l >= 2)
   const auto contract = [&](const double* g3, const double* g2, double* out_grad) {
@@ -3452,12 +3462,28 @@ int dfks_overlap(const dfks_basis_desc* basis, double* host_out, dfks_stream str
     } rel{&b};
     const int64_t n = b.nfunc;
     double *dS = dalloc<double>(n * n), *dT = dalloc<double>(n * n), *dV = dalloc<double>(n * n);
-    double* dummy = dalloc<double>(kBoysNg * kBoysN);
     struct Free {
       std::vector<void*> p;
       ~Free() { for (void* q : p) dfree(q); }
-    } fr{{dS, dT, dV, dummy}};
-    HIPCHK(launch_int1e(b.view(), 0, dummy, dummy, dS, dT, dV, n, st));
+    } fr{{dS, dT, dV}};
+    std::vector<int2> pairs;
+    std::vector<std::array<int, 4>> cls;   // la, lb, first pair, pairs
+    for (int la = 0; la <= b.maxl(); ++la)
+      for (int lb = 0; lb <= la; ++lb) {
+        const size_t at = pairs.size();
+        for (int i = 0; i < b.n(); ++i)
+          for (int j = 0; j < b.n(); ++j)
+            if (b.l[i] == la && b.l[j] == lb && (la != lb || j <= i)) pairs.push_back(make_int2(i, j));
+        cls.push_back({la, lb, (int)at, (int)(pairs.size() - at)});
+      }
+    int2* d_pairs = dalloc<int2>(pairs.size());
+    struct FreeP {
+      int2* p;
+      ~FreeP() { dfree(p); }
+    } frp{d_pairs};
+    HIPCHK(hipMemcpyAsync(d_pairs, pairs.data(), pairs.size() * sizeof(int2), hipMemcpyHostToDevice, st));
+    for (const auto& c : cls)
+      HIPCHK(launch_int1e(c[0], c[1], d_pairs + c[2], c[3], b.view(), 0, nullptr, nullptr, dS, dT, dV, n, st));
     HIPCHK(hipMemcpyAsync(host_out, dS, n * n * sizeof(double), hipMemcpyDeviceToHost, st));
     sync(st);
   });

@@ -244,4 +244,29 @@ __device__ __forceinline__ void boys_op_rt(int nmax, double T, double rho, doubl
   }
 }
 
+// E^{ij}_t for one axis into a [(la+1)][(lb+1)][mt] LDS block (lanes 0..2 call it).
+__device__ inline void e_table_1d(int la, int lb, double al, double be, double xab, int mt, double* E) {
+  double p = al + be, i2g = 0.5 / p, xpa = -be * xab / p, xpb = al * xab / p;
+  int nb = lb + 1;
+  for (int i = 0; i <= la; ++i)
+    for (int j = 0; j <= lb; ++j)
+      for (int t = 0; t < mt; ++t) E[(i * nb + j) * mt + t] = 0.0;
+  E[0] = 1.0;
+  for (int i = 0; i < la; ++i)
+    for (int t = 0; t <= i + 1 && t < mt; ++t) {
+      double v = xpa * E[(i * nb) * mt + t];
+      if (t > 0) v += i2g * E[(i * nb) * mt + t - 1];
+      if (t + 1 < mt) v += (t + 1) * E[(i * nb) * mt + t + 1];
+      E[((i + 1) * nb) * mt + t] = v;
+    }
+  for (int j = 0; j < lb; ++j)
+    for (int i = 0; i <= la; ++i)
+      for (int t = 0; t <= i + j + 1 && t < mt; ++t) {
+        double v = xpb * E[(i * nb + j) * mt + t];
+        if (t > 0) v += i2g * E[(i * nb + j) * mt + t - 1];
+        if (t + 1 < mt) v += (t + 1) * E[(i * nb + j) * mt + t + 1];
+        E[(i * nb + j + 1) * mt + t] = v;
+      }
+}
+
 }  // namespace dfks

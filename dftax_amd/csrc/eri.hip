@@ -1,4 +1,5 @@
-// McMurchie-Davidson 1-, 2- and 3-centre integrals on gfx950 (FP64).
+// McMurchie-Davidson two-electron integrals with sizes chosen at run time (FP64): two-centre ones of
+// cartesian spans, four-centre ones and the Schwarz bounds, and the gradient of cartesian spans.
 //
 // Algorithm (dftax/integrals/eri3c_bucketed.py:290-426, 697-734):
 //   (ab|c) = K_AB 2 pi^2.5 / (p q sqrt(p+q)) *
@@ -44,31 +45,6 @@ struct Task3 {
   const int32_t* aux;    // aux shell ids of this lc
   int npair, naux_l;
 };
-
-// E^{ij}_t for one axis into a [(la+1)][(lb+1)][mt] LDS block (lanes 0..2 call it).
-__device__ void e_table_1d(int la, int lb, double al, double be, double xab, int mt, double* E) {
-  double p = al + be, i2g = 0.5 / p, xpa = -be * xab / p, xpb = al * xab / p;
-  int nb = lb + 1;
-  for (int i = 0; i <= la; ++i)
-    for (int j = 0; j <= lb; ++j)
-      for (int t = 0; t < mt; ++t) E[(i * nb + j) * mt + t] = 0.0;
-  E[0] = 1.0;
-  for (int i = 0; i < la; ++i)
-    for (int t = 0; t <= i + 1 && t < mt; ++t) {
-      double v = xpa * E[(i * nb) * mt + t];
-      if (t > 0) v += i2g * E[(i * nb) * mt + t - 1];
-      if (t + 1 < mt) v += (t + 1) * E[(i * nb) * mt + t + 1];
-      E[((i + 1) * nb) * mt + t] = v;
-    }
-  for (int j = 0; j < lb; ++j)
-    for (int i = 0; i <= la; ++i)
-      for (int t = 0; t <= i + j + 1 && t < mt; ++t) {
-        double v = xpb * E[(i * nb + j) * mt + t];
-        if (t > 0) v += i2g * E[(i * nb + j) * mt + t - 1];
-        if (t + 1 < mt) v += (t + 1) * E[(i * nb + j) * mt + t + 1];
-        E[(i * nb + j + 1) * mt + t] = v;
-      }
-}
 
 // Build R^{(0)}_{tuv}, t+u+v <= L, in LDS (compact). buf0/buf1 ping-pong.
 // Returns a pointer to the buffer that holds level 0.
@@ -272,106 +248,6 @@ __global__ __launch_bounds__(64) void k_eri_wave(
 }
 
 // ---------------------------------------------------------------------------
-// One-electron S, T, V: one wave per ordered shell pair, lanes over the
-// cartesian outputs; the nuclear R ladder per (primitive pair, atom) in LDS.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(64) void k_int1e(ShellSet A, int natm, const double* __restrict__ atm,
-                                              const double* __restrict__ boys, double* __restrict__ S,
-                                              double* __restrict__ Tm, double* __restrict__ V, int64_t nao) {
-  __shared__ double s_E[3][4 * 6 * 10];
-  __shared__ double s_F[12];
-  __shared__ double s_R[2][84];
-  __shared__ double s_cart[3][100];
-  const int lane = threadIdx.x;
-  const int ia = blockIdx.x / A.n, ib = blockIdx.x % A.n;
-  const int la = A.l[ia], lb = A.l[ib];
-  const int na = ncart(la), nb = ncart(lb);
-  const int L = la + lb;
-  const int mtS = L + 3;   // kinetic needs j + 2
-  const int nbb = lb + 3;
-  double Ax = A.centre[3 * ia], Ay = A.centre[3 * ia + 1], Az = A.centre[3 * ia + 2];
-  double Bx = A.centre[3 * ib], By = A.centre[3 * ib + 1], Bz = A.centre[3 * ib + 2];
-  double ABx = Ax - Bx, ABy = Ay - By, ABz = Az - Bz;
-  double ab2 = ABx * ABx + ABy * ABy + ABz * ABz;
-  const int nout = na * nb;
-  for (int o = lane; o < nout; o += kWave) { s_cart[0][o] = 0.0; s_cart[1][o] = 0.0; s_cart[2][o] = 0.0; }
-  for (int pa = 0; pa < A.nprim[ia]; ++pa)
-    for (int pb = 0; pb < A.nprim[ib]; ++pb) {
-      double al = A.exps[A.prim0[ia] + pa], be = A.exps[A.prim0[ib] + pb];
-      double cab = A.coefs[A.prim0[ia] + pa] * A.coefs[A.prim0[ib] + pb];
-      double p = al + be;
-      double Px = (al * Ax + be * Bx) / p, Py = (al * Ay + be * By) / p, Pz = (al * Az + be * Bz) / p;
-      double Kab = exp(-al * be / p * ab2);
-      __syncthreads();
-      if (lane < 3) {
-        double xab = lane == 0 ? ABx : (lane == 1 ? ABy : ABz);
-        e_table_1d(la, lb + 2, al, be, xab, mtS, s_E[lane]);
-      }
-      __syncthreads();
-      double s0 = pow(kPi / p, 1.5) * Kab * cab;
-      for (int o = lane; o < nout; o += kWave) {
-        int ai = o / nb, bi = o % nb;
-        double s1[3], t1[3];
-        for (int x = 0; x < 3; ++x) {
-          int i = cexp(la, ai, x), jj = cexp(lb, bi, x);
-          const double* E = s_E[x];
-          double sij = E[(i * nbb + jj) * mtS];
-          double tt = -2.0 * be * be * E[(i * nbb + jj + 2) * mtS] + be * (2 * jj + 1) * sij;
-          if (jj >= 2) tt -= 0.5 * jj * (jj - 1) * E[(i * nbb + jj - 2) * mtS];
-          s1[x] = sij;
-          t1[x] = tt;
-        }
-        s_cart[0][o] += s0 * s1[0] * s1[1] * s1[2];
-        s_cart[1][o] += s0 * (t1[0] * s1[1] * s1[2] + s1[0] * t1[1] * s1[2] + s1[0] * s1[1] * t1[2]);
-      }
-      for (int c = 0; c < natm; ++c) {
-        double pcx = Px - atm[4 * c], pcy = Py - atm[4 * c + 1], pcz = Pz - atm[4 * c + 2];
-        double Z = atm[4 * c + 3];
-        __syncthreads();
-        if (lane == 0) boys_array_rt(L, p * (pcx * pcx + pcy * pcy + pcz * pcz), s_F, boys);
-        __syncthreads();
-        const double* R = r_ladder(L, p, pcx, pcy, pcz, s_F, s_R[0], s_R[1]);
-        double pref = -Z * cab * Kab * 2.0 * kPi / p;
-        for (int o = lane; o < nout; o += kWave) {
-          int ai = o / nb, bi = o % nb;
-          int a0 = cexp(la, ai, 0), a1 = cexp(la, ai, 1), a2 = cexp(la, ai, 2);
-          int b0 = cexp(lb, bi, 0), b1 = cexp(lb, bi, 1), b2 = cexp(lb, bi, 2);
-          const double* Ex = s_E[0] + (a0 * nbb + b0) * mtS;
-          const double* Ey = s_E[1] + (a1 * nbb + b1) * mtS;
-          const double* Ez = s_E[2] + (a2 * nbb + b2) * mtS;
-          double sum = 0.0;
-          for (int t = 0; t <= a0 + b0; ++t)
-            for (int u = 0; u <= a1 + b1; ++u)
-              for (int v = 0; v <= a2 + b2; ++v) sum += Ex[t] * Ey[u] * Ez[v] * R[ridx(t, u, v)];
-          s_cart[2][o] += pref * sum;
-        }
-        __syncthreads();
-      }
-    }
-  __syncthreads();
-  const int sphA = A.spherical && la >= 2, sphB = A.spherical && lb >= 2;
-  const int fa = sphA ? nsph(la) : na, fb = sphB ? nsph(lb) : nb;
-  for (int o = lane; o < fa * fb; o += kWave) {
-    int Ai = o / fb, Bi = o % fb;
-    int nA = sphA ? g_c2s.n[la][Ai] : 1, nB = sphB ? g_c2s.n[lb][Bi] : 1;
-    double v[3] = {0, 0, 0};
-    for (int x = 0; x < nA; ++x) {
-      int ai = sphA ? g_c2s.cart[la][Ai][x] : Ai;
-      double wa = sphA ? g_c2s.coef[la][Ai][x] : 1.0;
-      for (int y = 0; y < nB; ++y) {
-        int bi = sphB ? g_c2s.cart[lb][Bi][y] : Bi;
-        double w = wa * (sphB ? g_c2s.coef[lb][Bi][y] : 1.0);
-        for (int z = 0; z < 3; ++z) v[z] += w * s_cart[z][ai * nb + bi];
-      }
-    }
-    int64_t idx = (int64_t)(A.ao0[ia] + Ai) * nao + A.ao0[ib] + Bi;
-    S[idx] = v[0];
-    Tm[idx] = v[1];
-    V[idx] = v[2];
-  }
-}
-
-// ---------------------------------------------------------------------------
 // Schwarz factors of bra shell pairs: Q_ab = max over cartesian components
 // (mu nu) of sqrt((mu nu|mu nu)) (dftax/integrals/eri4c.py:206-220, taken per
 // shell pair as in eri3c_bucketed.py:140-169). One wavefront per pair, lanes
@@ -478,6 +354,7 @@ hipError_t launch_schwarz(int la, int lb, const int2* pairs, int npair, const Sh
 void upload_cls_tables(const C2SList& h, const int (&cart)[7][28][3]);
 void upload_pair_tables(const C2SList& h, const int (&cart)[7][28][3]);
 void upload_pair_grad_tables(const C2SList& h, const int (&cart)[7][28][3]);
+void upload_int1e_tables(const C2SList& h, const int (&cart)[7][28][3]);
 
 void upload_c2s_tables() {
   static C2SList h;
@@ -509,6 +386,7 @@ void upload_c2s_tables() {
   upload_cls_tables(h, cart);
   upload_pair_tables(h, cart);
   upload_pair_grad_tables(h, cart);
+  upload_int1e_tables(h, cart);
 }
 
 hipError_t launch_eri_wave(int la, int lb, int lc, const int2* pairs, int npair, const int32_t* aux, int naux_l,
@@ -528,13 +406,6 @@ hipError_t launch_eri_wave(int la, int lb, int lc, const int2* pairs, int npair,
   }
   return hipSuccess;
 }
-
-hipError_t launch_int1e(const ShellSet& A, int natm, const double* atm, const double* boys, double* S, double* T,
-                        double* V, int64_t nao, hipStream_t stream) {
-  hipLaunchKernelGGL(k_int1e, dim3((unsigned)(A.n * A.n)), dim3(kWave), 0, stream, A, natm, atm, boys, S, T, V, nao);
-  return hipGetLastError();
-}
-
 
 // ---------------------------------------------------------------------------
 // Nuclear-coordinate derivatives of the integrals, contracted on the fly with
@@ -739,126 +610,6 @@ __global__ __launch_bounds__(64) void k_eri_grad(const int2* __restrict__ pairs,
   }
 }
 
-// One-electron part of dE/dR over every ordered shell pair (a, b), derivative in
-// the bra centre only (the ket-centre share equals it by symmetry, hence the 2):
-//   2 sum_{mn in (a,b)} [ P_mn (dT_mn + sum_C dV^C_mn) - W_mn dS_mn ]  -> atom of a,
-//   and the Hellmann-Feynman term of each nucleus C, d/dC V^C = -(d/dA + d/dB) V^C:
-//   -2 sum_{mn} P_mn dV^C_mn -> atom C.
-__global__ __launch_bounds__(64) void k_int1e_grad(ShellSet A, const int32_t* __restrict__ atom_a, int natm,
-                                                   const double* __restrict__ atm, const double* __restrict__ boys,
-                                                   const double* __restrict__ P, const double* __restrict__ W,
-                                                   int64_t nao, double* __restrict__ grad) {
-  __shared__ double s_E[3][5 * 6 * 11];
-  __shared__ double s_F[12];
-  __shared__ double s_R[2][120];
-  __shared__ double s_P[100], s_W[100];
-  const int lane = threadIdx.x;
-  const int ia = blockIdx.x / A.n, ib = blockIdx.x % A.n;
-  const int la = A.l[ia], lb = A.l[ib];
-  const int na = ncart(la), nb = ncart(lb), nout = na * nb;
-  const int L = la + lb + 1;
-  const int mt = la + lb + 4;   // E up to (la+1, lb+2)
-  const int nbb = lb + 3;
-  const int sphA = A.spherical && la >= 2, sphB = A.spherical && lb >= 2;
-  weight_to_cart(la, lb, 0, sphA, sphB, 0, P, 0, nao, 1, A.ao0[ia], A.ao0[ib], 0, s_P);
-  weight_to_cart(la, lb, 0, sphA, sphB, 0, W, 0, nao, 1, A.ao0[ia], A.ao0[ib], 0, s_W);
-  const double Ax = A.centre[3 * ia], Ay = A.centre[3 * ia + 1], Az = A.centre[3 * ia + 2];
-  const double Bx = A.centre[3 * ib], By = A.centre[3 * ib + 1], Bz = A.centre[3 * ib + 2];
-  const double ABx = Ax - Bx, ABy = Ay - By, ABz = Az - Bz, ab2 = ABx * ABx + ABy * ABy + ABz * ABz;
-  double gA[3] = {0, 0, 0};   // this lane's share of the S and T terms
-  double gV[3] = {0, 0, 0};   // the wavefront's nuclear-attraction sums (the same on every lane)
-  for (int pa = 0; pa < A.nprim[ia]; ++pa)
-    for (int pb = 0; pb < A.nprim[ib]; ++pb) {
-      const double al = A.exps[A.prim0[ia] + pa], be = A.exps[A.prim0[ib] + pb];
-      const double cab = A.coefs[A.prim0[ia] + pa] * A.coefs[A.prim0[ib] + pb];
-      const double p = al + be;
-      const double Px = (al * Ax + be * Bx) / p, Py = (al * Ay + be * By) / p, Pz = (al * Az + be * Bz) / p;
-      const double Kab = exp(-al * be / p * ab2);
-      __syncthreads();
-      if (lane < 3) {
-        const double xab = lane == 0 ? ABx : (lane == 1 ? ABy : ABz);
-        e_table_1d(la + 1, lb + 2, al, be, xab, mt, s_E[lane]);
-      }
-      __syncthreads();
-      const double s0 = pow(kPi / p, 1.5) * Kab * cab;
-      // overlap and kinetic: per-axis factors s_ij = E^{ij}_0, t_ij from E^{i,j+2}, E^{ij}, E^{i,j-2};
-      // their bra derivatives 2a f_{i+1,j} - i f_{i-1,j}
-      for (int o = lane; o < nout; o += kWave) {
-        const int ai = o / nb, bi = o % nb;
-        double s1[3], t1[3], ds[3], dt[3];
-        for (int x = 0; x < 3; ++x) {
-          const int i = cexp(la, ai, x), j = cexp(lb, bi, x);
-          const double* E = s_E[x];
-          auto sv = [&](int ii, int jj) { return E[(ii * nbb + jj) * mt]; };
-          auto tv = [&](int ii, int jj) {
-            double r = -2.0 * be * be * sv(ii, jj + 2) + be * (2 * jj + 1) * sv(ii, jj);
-            if (jj >= 2) r -= 0.5 * jj * (jj - 1) * sv(ii, jj - 2);
-            return r;
-          };
-          s1[x] = sv(i, j);
-          t1[x] = tv(i, j);
-          ds[x] = 2.0 * al * sv(i + 1, j) - (i > 0 ? i * sv(i - 1, j) : 0.0);
-          dt[x] = 2.0 * al * tv(i + 1, j) - (i > 0 ? i * tv(i - 1, j) : 0.0);
-        }
-        const double wP = s_P[o], wW = s_W[o];
-        for (int x = 0; x < 3; ++x) {
-          const int y = (x + 1) % 3, z = (x + 2) % 3;
-          const double dS = s0 * ds[x] * s1[y] * s1[z];
-          const double dT = s0 * (dt[x] * s1[y] * s1[z] + ds[x] * t1[y] * s1[z] + ds[x] * s1[y] * t1[z]);
-          gA[x] += wP * dT - wW * dS;
-        }
-      }
-      // nuclear attraction, nucleus by nucleus
-      for (int c = 0; c < natm; ++c) {
-        const double pcx = Px - atm[4 * c], pcy = Py - atm[4 * c + 1], pcz = Pz - atm[4 * c + 2];
-        __syncthreads();
-        if (lane == 0) boys_array_rt(L, p * (pcx * pcx + pcy * pcy + pcz * pcz), s_F, boys);
-        __syncthreads();
-        const double* R = r_ladder(L, p, pcx, pcy, pcz, s_F, s_R[0], s_R[1]);
-        const double pref = -atm[4 * c + 3] * cab * Kab * 2.0 * kPi / p;
-        double gc[3] = {0, 0, 0};
-        for (int o = lane; o < nout; o += kWave) {
-          const double wP = s_P[o];
-          if (wP == 0.0) continue;
-          const int ai = o / nb, bi = o % nb;
-          double Ev[3][8], DA[3][8];
-          int ij[3];
-          for (int x = 0; x < 3; ++x) {
-            const int i = cexp(la, ai, x), j = cexp(lb, bi, x);
-            const double* E = s_E[x];
-            ij[x] = i + j;
-            for (int t = 0; t <= i + j + 1; ++t) {
-              Ev[x][t] = t <= i + j ? E[(i * nbb + j) * mt + t] : 0.0;
-              double da = 2.0 * al * E[((i + 1) * nbb + j) * mt + t];
-              if (i > 0 && t <= i + j - 1) da -= i * E[((i - 1) * nbb + j) * mt + t];
-              DA[x][t] = da;
-            }
-          }
-          double d3[3] = {0, 0, 0};
-          for (int t = 0; t <= ij[0] + 1; ++t)
-            for (int u = 0; u <= ij[1] + 1; ++u)
-              for (int v = 0; v <= ij[2] + 1; ++v) {
-                const double r = R[ridx(t, u, v)];
-                d3[0] += DA[0][t] * Ev[1][u] * Ev[2][v] * r;
-                d3[1] += Ev[0][t] * DA[1][u] * Ev[2][v] * r;
-                d3[2] += Ev[0][t] * Ev[1][u] * DA[2][v] * r;
-              }
-          for (int x = 0; x < 3; ++x) gc[x] += wP * pref * d3[x];
-        }
-        for (int x = 0; x < 3; ++x) {
-          const double v = wave_sum(gc[x]);
-          gV[x] += v;
-          if (lane == 0) atomicAdd(&grad[3 * c + x], -2.0 * v);
-        }
-        __syncthreads();
-      }
-    }
-  for (int x = 0; x < 3; ++x) {
-    const double v = wave_sum(gA[x]) + gV[x];
-    if (lane == 0) atomicAdd(&grad[3 * atom_a[ia] + x], 2.0 * v);
-  }
-}
-
 hipError_t launch_eri_grad(const int2* pairs, int npair, int nket, const ShellSet& A, const ShellSet& C,
                            const int32_t* atom_a, const int32_t* atom_c, int b_unit, const double* boys,
                            const double* G, int64_t nao_g, double* grad, hipStream_t st) {
@@ -869,14 +620,6 @@ hipError_t launch_eri_grad(const int2* pairs, int npair, int nket, const ShellSe
     hipLaunchKernelGGL(k_eri_grad, dim3((unsigned)nb), dim3(kWave), 0, st, pairs, npair, nket, A, C, atom_a, atom_c,
                        b_unit, boys, G, nao_g, grad, b0);
   }
-  return hipGetLastError();
-}
-
-hipError_t launch_int1e_grad(const ShellSet& A, const int32_t* atom_a, int natm, const double* atm,
-                             const double* boys, const double* P, const double* W, int64_t nao, double* grad,
-                             hipStream_t st) {
-  hipLaunchKernelGGL(k_int1e_grad, dim3((unsigned)(A.n * A.n)), dim3(kWave), 0, st, A, atom_a, natm, atm, boys, P, W,
-                     nao, grad);
   return hipGetLastError();
 }
 

@@ -1,6 +1,6 @@
-// Three-centre (ab|c) for the higher angular-momentum classes: one 64-lane
-// wavefront per task (bra shell pair x auxiliary shell), one template instance
-// per class.
+// Three-centre (ab|c) of cartesian spans with l >= 2 (spherical ones go by bra
+// pair, eri_pair.hip): one 64-lane wavefront per task (bra shell pair x
+// auxiliary shell), one template instance per class.
 //
 // Same scheme as the generic wavefront kernel in eri.hip (E tables, R ladder
 // and the cartesian block in LDS, lanes over the cartesian outputs, sparse

@@ -11,7 +11,10 @@
 // v_mfma_f64_16x16x4f64 (rows = h, k = AB functions, columns = 16 auxiliary shells), and each lane
 // weights its rows of the products with G and its three shifts from R in LDS: no derivative of a
 // single integral is formed. Auxiliary centres collect in LDS per atom and go out once a workgroup.
-// Bound by the matrix work (4 times the integrals') and the reads of R.
+// Bound by the matrix work (4 times the integrals') and the reads of R. A tree of 6 heavy atoms,
+// def2-SVP: 6.6 ms for the Coulomb and the exchange term, 71 ms with a wavefront per task that
+// differentiated each integral (k_eri_grad in eri.hip, kept for cartesian spans with l >= 2 and for
+// more atoms than the LDS sums hold).
 // Reference: dftax/ks/forces.py:128-270 (jax.grad through eri3c_bucketed.py:290-426).
 #include <algorithm>
 #include <cstdint>

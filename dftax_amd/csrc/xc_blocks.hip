@@ -14,12 +14,13 @@
 // 3.9 ms, against 14 ms for the per-bin gathers, batched products and
 // wavefront-per-point kernels they replace. Vh is near what its AO rows read
 // and products written take at the copy rate (3 ms); rho is between its reads
-// (1.7 ms) and its matrix work (2.8 ms). An MFMA sums over any order of k as long as both operands agree, so the operand that is contiguous along k
-// (Phi in Z) is loaded straight from global memory in 32-byte runs, lane group
-// l taking k = 4 l + s in step s, and the other operand sits in LDS in
-// fragment order (64 consecutive doubles per step and 16 columns): no
-// conflicts and no transposition. In Vh the contraction runs over the points,
-// so Phi's fragments are 128-byte runs of one point's row as they lie.
+// (1.7 ms) and its matrix work (2.8 ms). An MFMA sums over any order of k as
+// long as both operands agree, so the operand that is contiguous along k (Phi
+// in Z) is loaded straight from global memory in 32-byte runs, lane group l
+// taking k = 4 l + s in step s, and the other operand sits in LDS in fragment
+// order (64 consecutive doubles per step and 16 columns): no conflicts and no
+// transposition. In Vh the contraction runs over the points, so Phi's
+// fragments are 128-byte runs of one point's row as they lie.
 #include <cstdint>
 
 #include "dfks_common.h"

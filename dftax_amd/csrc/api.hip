@@ -130,12 +130,12 @@ hipError_t launch_int1e_grad(int la, int lb, const int2* pairs, int npair, const
 hipError_t launch_ao_hess(int64_t npts, const double* pts, const ShellSet& S, int64_t nao, double* ao,
                           hipStream_t st);
 hipError_t launch_xcg_rho(int64_t npts, int64_t nao, const double* ao, const double* Z, double* rho, double* grad,
-                          double* sigma, hipStream_t st);
-hipError_t launch_xcg_gdot(int64_t npts, int64_t nao, const double* ao, const double* grad, double* Gd,
-                           hipStream_t st);
-hipError_t launch_xcg_q(int64_t npts, int64_t nao, const double* ao, const double* Z, const double* X,
-                        const double* rho, const double* grad, const double* xc, const double* w,
-                        const int32_t* owner, double thresh, double* q, double* gout, double* fm, hipStream_t st);
+                          double* sigma, double* Gd, hipStream_t st);
+int xcg_blocks(int64_t npts);
+hipError_t launch_xcg_sum(int64_t npts, int64_t nao, const double* ao, const double* Z, const double* X,
+                          const double* rho, const double* grad, const double* xc, const double* w,
+                          const int32_t* owner, double thresh, double* part, double* colsum, double* gout, double* fm,
+                          hipStream_t st);
 hipError_t launch_becke_grad(int64_t n, const double* pts, const double* raw, const int32_t* owner, const double* f,
                              int natm, const double* atm, const double* invR, const double* aAB, double* gout,
                              hipStream_t st);
@@ -2520,7 +2520,8 @@ void forces_run(dfks_ctx* h, const double* Co, int nocc, int64_t ng, const doubl
     double* ao = alloc(10 * (size_t)chunk * nao);
     double* Z = alloc((size_t)chunk * nao);
     double* Xg = alloc((size_t)chunk * nao);
-    double* q = alloc(3 * (size_t)chunk * nao);
+    double* gd = alloc((size_t)chunk * nao);
+    double* part = alloc((size_t)xcg_blocks(chunk) * 3 * nao);
     double* rho = alloc(chunk);
     double* grad = alloc(3 * (size_t)chunk);
     double* sigma = alloc(chunk);
@@ -2533,15 +2534,11 @@ void forces_run(dfks_ctx* h, const double* Co, int nocc, int64_t ng, const doubl
       HIPCHK(launch_ao_hess(nc, d_pts + 3 * g0, O, nao, ao, st));
       // Z = Phi P and X = (grad rho . grad Phi) P, row-major nc x nao
       gemm(h, false, false, nao, nc, nao, 1.0, P, nao, ao, nao, 0.0, Z, nao);
-      HIPCHK(launch_xcg_rho(nc, nao, ao, Z, rho, grad, sigma, st));
+      HIPCHK(launch_xcg_rho(nc, nao, ao, Z, rho, grad, sigma, gd, st));
       HIPCHK(launch_xc_pointwise(nc, h->xc_id, rho, sigma, xco, st));
-      HIPCHK(launch_xcg_gdot(nc, nao, ao, grad, q, st));
-      gemm(h, false, false, nao, nc, nao, 1.0, P, nao, q, nao, 0.0, Xg, nao);
-      HIPCHK(launch_xcg_q(nc, nao, ao, Z, Xg, rho, grad, xco, d_w + g0, d_own + g0, h->opt.rho_thresh, q, gp[3], fm,
-                          st));
-      for (int j = 0; j < 3; ++j)
-        RBCHK(rocblas_dgemv(h->rb, rocblas_operation_none, nao, nc, &kOne, q + (int64_t)j * nc * nao, nao, d_w + g0, 1,
-                            &kOne, Sm + (int64_t)j * nao, 1));
+      gemm(h, false, false, nao, nc, nao, 1.0, P, nao, gd, nao, 0.0, Xg, nao);
+      HIPCHK(launch_xcg_sum(nc, nao, ao, Z, Xg, rho, grad, xco, d_w + g0, d_own + g0, h->opt.rho_thresh, part, Sm,
+                            gp[3], fm, st));
       HIPCHK(launch_becke_grad(nc, d_pts + 3 * g0, d_raw + g0, d_own + g0, fm, natom, d_atm3, d_invR, d_aAB, gp[3],
                                st));
     }

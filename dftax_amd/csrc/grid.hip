@@ -14,11 +14,55 @@
 
 namespace dfks {
 
+// 16 points a wavefront, 4 lanes each: the point's distances in LDS ([natm][16] a wavefront), each lane the
+// products of every fourth atom. A tree of 20 heavy atoms: 2.0 ms, 4.0 ms with a thread a point that forms both
+// distances of every pair (k_becke_far).
 __global__ __launch_bounds__(256) void k_becke(int64_t n, const double* __restrict__ pts, const double* __restrict__ raw,
-                                                const int32_t* __restrict__ owner, int natm,
-                                                const double* __restrict__ atm /*[natm*3]*/,
-                                                const double* __restrict__ invR /*[natm*natm]*/,
-                                                const double* __restrict__ aAB /*[natm*natm]*/, double* __restrict__ w) {
+                                               const int32_t* __restrict__ owner, int natm,
+                                               const double* __restrict__ atm /*[natm*3]*/,
+                                               const double* __restrict__ invR /*[natm*natm]*/,
+                                               const double* __restrict__ aAB /*[natm*natm]*/, double* __restrict__ w) {
+  extern __shared__ double s_bw[];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, pt = lane & 15, sub = lane >> 4;
+  double* s_r = s_bw + (size_t)wave * 16 * natm + pt;
+  const int64_t g = ((int64_t)blockIdx.x * (blockDim.x >> 6) + wave) * 16 + pt, gc = min(g, n - 1);
+  const double px = pts[3 * gc], py = pts[3 * gc + 1], pz = pts[3 * gc + 2];
+  const int own = owner[gc];
+  for (int a = sub; a < natm; a += 4) {
+    const double dx = px - atm[3 * a], dy = py - atm[3 * a + 1], dz = pz - atm[3 * a + 2];
+    s_r[16 * a] = sqrt(dx * dx + dy * dy + dz * dz + 1e-30);
+  }
+  __syncthreads();
+  double total = 0.0, mine = 0.0;
+  for (int a = sub; a < natm; a += 4) {
+    const double ra = s_r[16 * a];
+    const double *iRa = invR + (int64_t)a * natm, *aa = aAB + (int64_t)a * natm;
+    double prod = 1.0;
+#pragma unroll 4
+    for (int b = 0; b < natm; ++b) {
+      const double mu = (ra - s_r[16 * b]) * iRa[b];
+      double f = mu + aa[b] * (1.0 - mu * mu);
+      f = 1.5 * f - 0.5 * f * f * f;
+      f = 1.5 * f - 0.5 * f * f * f;
+      f = 1.5 * f - 0.5 * f * f * f;
+      prod *= b == a ? 1.0 : 0.5 * (1.0 - f);
+    }
+    total += prod;
+    if (a == own) mine = prod;
+  }
+  total += __shfl_xor(total, 16);
+  total += __shfl_xor(total, 32);
+  mine += __shfl_xor(mine, 16);
+  mine += __shfl_xor(mine, 32);
+  if (sub == 0 && g < n) w[g] = raw[g] * mine / total;
+}
+
+// The same with one thread per point and no distance kept, for molecules whose distances do not fit.
+__global__ __launch_bounds__(256) void k_becke_far(int64_t n, const double* __restrict__ pts,
+                                                   const double* __restrict__ raw, const int32_t* __restrict__ owner,
+                                                   int natm, const double* __restrict__ atm,
+                                                   const double* __restrict__ invR, const double* __restrict__ aAB,
+                                                   double* __restrict__ w) {
   extern __shared__ double s_atm[];  // 3*natm
   for (int i = threadIdx.x; i < 3 * natm; i += blockDim.x) s_atm[i] = atm[i];
   __syncthreads();
@@ -307,9 +351,15 @@ template hipError_t launch_vassemble<float>(int, const int64_t*, const int64_t*,
 hipError_t launch_becke(int64_t n, const double* pts, const double* raw, const int32_t* owner, int natm,
                         const double* atm, const double* invR, const double* aAB, double* w, hipStream_t st) {
   if (n == 0) return hipSuccess;
-  const int bs = 256;
-  hipLaunchKernelGGL(k_becke, dim3((unsigned)((n + bs - 1) / bs)), dim3(bs), 3 * natm * sizeof(double), st, n, pts,
-                     raw, owner, natm, atm, invR, aAB, w);
+  // 64 KB of LDS hold the distances of 128 atoms for 4 wavefronts, of 512 for one
+  const auto lds = [&](int nw) { return (size_t)natm * 16 * nw * sizeof(double); };
+  const int nw = lds(4) <= 65536 ? 4 : 1;
+  if (lds(nw) <= 65536)
+    hipLaunchKernelGGL(k_becke, dim3((unsigned)((n + 16 * nw - 1) / (16 * nw))), dim3(64 * nw), lds(nw), st, n, pts, raw,
+                       owner, natm, atm, invR, aAB, w);
+  else
+    hipLaunchKernelGGL(k_becke_far, dim3((unsigned)((n + 255) / 256)), dim3(256), 3 * natm * sizeof(double), st, n, pts,
+                       raw, owner, natm, atm, invR, aAB, w);
   return hipGetLastError();
 }
 
@@ -437,11 +487,12 @@ __global__ __launch_bounds__(256) void k_ao_hess(int64_t npts, const double* __r
   }
 }
 
-// rho, grad rho and sigma at each point from the AO planes and Z = Phi P
-// (one wavefront per point, lanes over the functions).
+// rho, grad rho and sigma at each point from the AO planes and Z = Phi P, and Gd[g][m] = grad rho_g . grad
+// phi_m(g) while the point's row is in the cache (one wavefront per point, lanes over the functions).
 __global__ __launch_bounds__(64) void k_xcg_rho(int64_t npts, int64_t nao, const double* __restrict__ ao,
                                                 const double* __restrict__ Z, double* __restrict__ rho,
-                                                double* __restrict__ grad, double* __restrict__ sigma) {
+                                                double* __restrict__ grad, double* __restrict__ sigma,
+                                                double* __restrict__ Gd) {
   const int64_t g = blockIdx.x;
   if (g >= npts) return;
   const int64_t plane = npts * nao;
@@ -454,62 +505,115 @@ __global__ __launch_bounds__(64) void k_xcg_rho(int64_t npts, int64_t nao, const
 #pragma unroll
   for (int k = 0; k < 4; ++k)
     for (int off = 32; off > 0; off >>= 1) a[k] += __shfl_xor(a[k], off, 64);
+  const double gx = 2.0 * a[1], gy = 2.0 * a[2], gz = 2.0 * a[3];
   if (threadIdx.x == 0) {
     rho[g] = a[0];
-    const double gx = 2.0 * a[1], gy = 2.0 * a[2], gz = 2.0 * a[3];
     grad[3 * g] = gx; grad[3 * g + 1] = gy; grad[3 * g + 2] = gz;
     sigma[g] = gx * gx + gy * gy + gz * gz;
   }
-}
-
-// Gd[g][m] = grad rho_g . grad phi_m(g)
-__global__ __launch_bounds__(256) void k_xcg_gdot(int64_t npts, int64_t nao, const double* __restrict__ ao,
-                                                   const double* __restrict__ grad, double* __restrict__ Gd) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= npts * nao) return;
-  const int64_t g = i / nao, plane = npts * nao;
-  Gd[i] = grad[3 * g] * ao[plane + i] + grad[3 * g + 1] * ao[2 * plane + i] + grad[3 * g + 2] * ao[3 * plane + i];
-}
-
-// q_{g m j} (above) into q[3][npts][nao]; the point part 2 w_g sum_m q to the
-// point's owner atom. xc[3 g ..] = {f, v_rho, v_sigma}; points with
-// rho <= thresh contribute nothing (the energy's density mask).
-__global__ __launch_bounds__(64) void k_xcg_q(int64_t npts, int64_t nao, const double* __restrict__ ao,
-                                              const double* __restrict__ Z, const double* __restrict__ X,
-                                              const double* __restrict__ rho, const double* __restrict__ grad,
-                                              const double* __restrict__ xc, const double* __restrict__ w,
-                                              const int32_t* __restrict__ owner, double thresh, double* __restrict__ q,
-                                              double* __restrict__ gout, double* __restrict__ fm) {
-  const int64_t g = blockIdx.x;
-  if (g >= npts) return;
-  const int64_t plane = npts * nao;
-  const bool on = rho[g] > thresh;
-  if (threadIdx.x == 0) fm[g] = on ? xc[3 * g] : 0.0;   // energy density f of the masked functional
-  const double vr = on ? xc[3 * g + 1] : 0.0, vs = on ? xc[3 * g + 2] : 0.0;
-  const double gr[3] = {grad[3 * g], grad[3 * g + 1], grad[3 * g + 2]};
-  double acc[3] = {0, 0, 0};
   for (int64_t m = threadIdx.x; m < nao; m += 64) {
     const int64_t i = g * nao + m;
-    const double z = Z[i], x = X[i];
-    const double d[3] = {ao[plane + i], ao[2 * plane + i], ao[3 * plane + i]};
-    const double hxx = ao[4 * plane + i], hxy = ao[5 * plane + i], hxz = ao[6 * plane + i];
-    const double hyy = ao[7 * plane + i], hyz = ao[8 * plane + i], hzz = ao[9 * plane + i];
-    const double hg[3] = {hxx * gr[0] + hxy * gr[1] + hxz * gr[2], hxy * gr[0] + hyy * gr[1] + hyz * gr[2],
-                          hxz * gr[0] + hyz * gr[1] + hzz * gr[2]};
+    Gd[i] = gx * ao[plane + i] + gy * ao[2 * plane + i] + gz * ao[3 * plane + i];
+  }
+}
+
+// The sums of q_{g m j} (above) over points and over functions, without storing q: a wavefront walks a
+// contiguous range of points with its 64 KT columns' sums in registers. Column sums go to
+// part[block][3][nao] (k_xcg_cols adds the blocks in order); row sums are held while the owner stays the
+// same (the points of an atom are contiguous) and then reduced once. xc[3 g ..] = {f, v_rho, v_sigma};
+// points with rho <= thresh contribute nothing (the energy's density mask). Bound by reading 9 planes, Z
+// and X once. A tree of 6 heavy atoms, def2-SVP: 1.4 ms, against 5.3 ms with q stored and 26 ms of
+// matrix-vector products that read it back for its column sums.
+constexpr int kXcgWaves = 4;
+template <int KT>
+__global__ __launch_bounds__(64 * kXcgWaves) void k_xcg_sum(
+    int64_t npts, int64_t per, int64_t nao, const double* __restrict__ ao, const double* __restrict__ Z,
+    const double* __restrict__ X, const double* __restrict__ rho, const double* __restrict__ grad,
+    const double* __restrict__ xc, const double* __restrict__ w, const int32_t* __restrict__ owner, double thresh,
+    double* __restrict__ part, double* __restrict__ gout, double* __restrict__ fm) {
+  __shared__ double s_c[kXcgWaves][KT * 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t c0 = (int64_t)blockIdx.y * (64 * KT), plane = npts * nao;
+  int64_t col[KT];
+  bool in[KT];
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const double v = vr * d[j] * z + 2.0 * vs * (hg[j] * z + d[j] * x);
-      q[j * plane + i] = v;
-      acc[j] += v;
+  for (int k = 0; k < KT; ++k) {
+    in[k] = c0 + 64 * k + lane < nao;
+    col[k] = in[k] ? c0 + 64 * k + lane : 0;
+  }
+  double cs[KT][3] = {}, rs[3] = {0.0, 0.0, 0.0};
+  const int64_t g0 = ((int64_t)blockIdx.x * kXcgWaves + wave) * per, g1 = min(npts, g0 + per);
+  int own = g0 < g1 ? owner[g0] : 0;
+  for (int64_t g = g0; g <= g1; ++g) {
+    const bool last = g >= g1;
+    if (last || owner[g] != own) {
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        double v = rs[j];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+        if (lane == 0 && g0 < g1) atomicAdd(&gout[3 * own + j], 2.0 * v);
+        rs[j] = 0.0;
+      }
+      if (last) break;
+      own = owner[g];
+    }
+    const bool on = rho[g] > thresh;
+    if (blockIdx.y == 0 && lane == 0) fm[g] = on ? xc[3 * g] : 0.0;   // energy density f of the masked functional
+    if (!on) continue;
+    const double wg = w[g], vr = wg * xc[3 * g + 1], vs = 2.0 * wg * xc[3 * g + 2];
+    const double gx = grad[3 * g], gy = grad[3 * g + 1], gz = grad[3 * g + 2];
+    const double *row = ao + g * nao, *zr = Z + g * nao, *xr = X + g * nao;
+#pragma unroll
+    for (int k = 0; k < KT; ++k) {
+      const double* r = row + col[k];
+      double z = zr[col[k]], x = xr[col[k]];
+      const double dx = r[plane], dy = r[2 * plane], dz = r[3 * plane];
+      const double hxx = r[4 * plane], hxy = r[5 * plane], hxz = r[6 * plane];
+      const double hyy = r[7 * plane], hyz = r[8 * plane], hzz = r[9 * plane];
+      z = in[k] ? z : 0.0;
+      x = in[k] ? x : 0.0;
+      const double a = vr * z + vs * x, b = vs * z;
+      const double q0 = a * dx + b * (hxx * gx + hxy * gy + hxz * gz);
+      const double q1 = a * dy + b * (hxy * gx + hyy * gy + hyz * gz);
+      const double q2 = a * dz + b * (hxz * gx + hyz * gy + hzz * gz);
+      cs[k][0] += q0;
+      cs[k][1] += q1;
+      cs[k][2] += q2;
+      rs[0] += q0;
+      rs[1] += q1;
+      rs[2] += q2;
     }
   }
 #pragma unroll
-  for (int j = 0; j < 3; ++j)
-    for (int off = 32; off > 0; off >>= 1) acc[j] += __shfl_xor(acc[j], off, 64);
-  if (threadIdx.x == 0 && on) {
-    const int a = owner[g];
+  for (int j = 0; j < 3; ++j) {
+    __syncthreads();
 #pragma unroll
-    for (int j = 0; j < 3; ++j) atomicAdd(&gout[3 * a + j], 2.0 * w[g] * acc[j]);
+    for (int k = 0; k < KT; ++k) s_c[wave][64 * k + lane] = cs[k][j];
+    __syncthreads();
+    for (int i = threadIdx.x; i < 64 * KT; i += 64 * kXcgWaves) {
+      double v = 0.0;
+#pragma unroll
+      for (int u = 0; u < kXcgWaves; ++u) v += s_c[u][i];
+      if (c0 + i < nao) part[((int64_t)blockIdx.x * 3 + j) * nao + c0 + i] = v;
+    }
+  }
+}
+
+// sum[i] += sum_b part[b][i], i < n, 16 columns a workgroup
+__global__ __launch_bounds__(256) void k_xcg_cols(int nb, int64_t n, const double* __restrict__ part,
+                                                  double* __restrict__ sum) {
+  __shared__ double s_p[16][17];
+  const int c = threadIdx.x & 15, s = threadIdx.x >> 4;
+  const int64_t i = (int64_t)blockIdx.x * 16 + c;
+  double v = 0.0;
+  if (i < n)
+    for (int b = s; b < nb; b += 16) v += part[(int64_t)b * n + i];
+  s_p[s][c] = v;
+  __syncthreads();
+  if (s == 0 && i < n) {
+    for (int k = 1; k < 16; ++k) v += s_p[k][c];
+    sum[i] += v;
   }
 }
 
@@ -520,16 +624,121 @@ __global__ __launch_bounds__(64) void k_xcg_q(int64_t npts, int64_t nao, const d
 //   dmu_AB/dR_A = -u_A / R_AB - mu_AB (R_A - R_B) / R_AB^2,
 //   dmu_AB/dR_B =  u_B / R_AB + mu_AB (R_A - R_B) / R_AB^2,
 //   dmu_AB/dr   = (u_A - u_B) / R_AB  (to the owner), u_X = (r - R_X)/|r - R_X|.
-// One thread per point; per-atom sums in LDS, added to gout once per workgroup.
-__device__ __forceinline__ void becke_s(double nu, double& s, double& ds) {
+// s(nu), s(-nu) and ds/dnu
+__device__ __forceinline__ void becke_s(double nu, double& s, double& sb, double& ds) {
   const double f1 = 1.5 * nu - 0.5 * nu * nu * nu;
   const double f2 = 1.5 * f1 - 0.5 * f1 * f1 * f1;
   const double f3 = 1.5 * f2 - 0.5 * f2 * f2 * f2;
   s = 0.5 * (1.0 - f3);
+  sb = 0.5 * (1.0 + f3);
   ds = -0.5 * (1.5 - 1.5 * f2 * f2) * (1.5 - 1.5 * f1 * f1) * (1.5 - 1.5 * nu * nu);
 }
 
+//
+// A wavefront takes 16 points, 4 lanes each: the lanes of a point share its distances in LDS and take
+// every fourth atom A. With both orders of a pair met, C_AB = s' (1 - 2 a mu) (K_A / s_AB - K_B / s_BA) is
+// antisymmetric (nu_BA = -nu_AB, s_BA = 1 - s_AB), so atom A's share is sum_B C_AB dmu_AB/dR_A alone, the
+// owner's is minus the sum of all, and a value leaves a lane once per atom instead of once per pair. Bound
+// by the FP64 chain of a pair, which has no distance, square root or LDS atomic in it. A tree of 6 heavy atoms:
+// 0.34 ms, 13.4 ms with a thread a point and nine LDS atomics a pair (k_becke_grad_far).
+// lds: nw waves x natm x 16 x (r, P) + 3 natm sums.
 __global__ __launch_bounds__(256) void k_becke_grad(int64_t n, const double* __restrict__ pts,
+                                                    const double* __restrict__ raw, const int32_t* __restrict__ owner,
+                                                    const double* __restrict__ f, int natm,
+                                                    const double* __restrict__ atm /*[3 natm]*/,
+                                                    const double* __restrict__ invR, const double* __restrict__ aAB,
+                                                    double* __restrict__ gout) {
+  extern __shared__ double s_bk[];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6, pt = lane & 15, sub = lane >> 4;
+  double* s_g = s_bk;
+  double* s_r = s_bk + 3 * natm + (size_t)wave * 32 * natm + pt;   // [natm][16]
+  double* s_K = s_r + 16 * natm;
+  for (int i = threadIdx.x; i < 3 * natm; i += blockDim.x) s_g[i] = 0.0;
+  const int64_t step = (int64_t)gridDim.x * 16 * nw;
+  for (int64_t t0 = (int64_t)blockIdx.x * 16 * nw; t0 < n; t0 += step) {
+    const int64_t g = t0 + 16 * wave + pt;
+    const bool live = g < n && f[min(g, n - 1)] != 0.0;
+    const int64_t gc = min(g, n - 1);
+    const double px = pts[3 * gc], py = pts[3 * gc + 1], pz = pts[3 * gc + 2];
+    const int own = owner[gc];
+    __syncthreads();
+    for (int a = sub; a < natm; a += 4) {
+      const double dx = px - atm[3 * a], dy = py - atm[3 * a + 1], dz = pz - atm[3 * a + 2];
+      s_r[16 * a] = sqrt(dx * dx + dy * dy + dz * dz + 1e-30);
+    }
+    __syncthreads();
+    double Zs = 0.0;
+    for (int a = sub; a < natm; a += 4) {
+      const double ra = s_r[16 * a];
+      const double *iRa = invR + (int64_t)a * natm, *aa = aAB + (int64_t)a * natm;
+      double prod = 1.0;
+#pragma unroll 4
+      for (int b = 0; b < natm; ++b) {
+        const double mu = (ra - s_r[16 * b]) * iRa[b];
+        double s, sb, ds;
+        becke_s(mu + aa[b] * (1.0 - mu * mu), s, sb, ds);
+        prod *= b == a ? 1.0 : s;
+      }
+      s_K[16 * a] = prod;
+      Zs += prod;
+    }
+    Zs += __shfl_xor(Zs, 16);
+    Zs += __shfl_xor(Zs, 32);
+    __syncthreads();
+    const bool on = live && Zs > 0.0;
+    const double iZ = on ? 1.0 / Zs : 0.0;
+    const double fw = on ? f[gc] * raw[gc] * s_K[16 * own] * iZ : 0.0;
+    __syncthreads();
+    for (int a = sub; a < natm; a += 4) s_K[16 * a] = fw * ((a == own ? 1.0 : 0.0) - s_K[16 * a] * iZ);
+    __syncthreads();
+    double go[3] = {0.0, 0.0, 0.0};
+    for (int a0 = 0; a0 < natm; a0 += 4) {
+      const int a = min(a0 + sub, natm - 1);
+      const double ra = s_r[16 * a], Ka = s_K[16 * a];
+      const double ax = atm[3 * a], ay = atm[3 * a + 1], az = atm[3 * a + 2];
+      const double *iRa = invR + (int64_t)a * natm, *aa = aAB + (int64_t)a * natm;
+      double c1 = 0.0, gx = 0.0, gy = 0.0, gz = 0.0;
+#pragma unroll 2
+      for (int b = 0; b < natm; ++b) {
+        const double iR = iRa[b], ab = aa[b], mu = (ra - s_r[16 * b]) * iR;
+        double s, sb, ds;
+        becke_s(mu + ab * (1.0 - mu * mu), s, sb, ds);
+        const bool oka = s >= 1e-300, okb = sb >= 1e-300;   // a factor of 0 has no logarithmic derivative
+        const double r = 1.0 / (oka && okb ? s * sb : 1.0);
+        double C = (oka ? Ka * (okb ? sb : 1.0) : 0.0) - (okb ? s_K[16 * b] * (oka ? s : 1.0) : 0.0);
+        C = b == a ? 0.0 : C * r * ds * (1.0 - 2.0 * ab * mu) * iR;
+        c1 += C;
+        C *= mu * iR;
+        gx += C * (ax - atm[3 * b]);
+        gy += C * (ay - atm[3 * b + 1]);
+        gz += C * (az - atm[3 * b + 2]);
+      }
+      c1 /= ra;
+      const bool mine = on && a0 + sub < natm;
+      double v[3] = {-(px - ax) * c1 - gx, -(py - ay) * c1 - gy, -(pz - az) * c1 - gz};
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        v[j] = mine ? v[j] : 0.0;
+        go[j] -= v[j];
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) v[j] += __shfl_xor(v[j], o, 16);
+        if (pt == 0 && a0 + sub < natm) atomicAdd(&s_g[3 * a + j], v[j]);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      go[j] += __shfl_xor(go[j], 16);
+      go[j] += __shfl_xor(go[j], 32);
+      if (sub == 0 && on) atomicAdd(&s_g[3 * own + j], go[j]);
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < 3 * natm; i += blockDim.x)
+    if (s_g[i] != 0.0) atomicAdd(&gout[i], s_g[i]);
+}
+
+// The same with one thread per point and nothing kept but the sums, for molecules whose distances do not fit.
+__global__ __launch_bounds__(256) void k_becke_grad_far(int64_t n, const double* __restrict__ pts,
                                                      const double* __restrict__ raw, const int32_t* __restrict__ owner,
                                                      const double* __restrict__ f, int natm,
                                                      const double* __restrict__ atm /*[3 natm]*/,
@@ -557,8 +766,8 @@ __global__ __launch_bounds__(256) void k_becke_grad(int64_t n, const double* __r
         if (b == a) continue;
         const double rb = dist(b, u);
         const double mu = (ra - rb) * invR[a * natm + b];
-        double s, ds;
-        becke_s(mu + aAB[a * natm + b] * (1.0 - mu * mu), s, ds);
+        double s, sb, ds;
+        becke_s(mu + aAB[a * natm + b] * (1.0 - mu * mu), s, sb, ds);
         prod *= s;
       }
       Zs += prod;
@@ -577,8 +786,8 @@ __global__ __launch_bounds__(256) void k_becke_grad(int64_t n, const double* __r
           double ub[3];
           const double rb = dist(b, ub);
           const double mu = (ra - rb) * invR[a * natm + b];
-          double s, ds;
-          becke_s(mu + aAB[a * natm + b] * (1.0 - mu * mu), s, ds);
+          double s, sb, ds;
+          becke_s(mu + aAB[a * natm + b] * (1.0 - mu * mu), s, sb, ds);
           prod *= s;
         }
         const double Ka = fw * ((a == own ? 1.0 : 0.0) - prod / Zs);
@@ -590,8 +799,8 @@ __global__ __launch_bounds__(256) void k_becke_grad(int64_t n, const double* __r
           const double iR = invR[a * natm + b];
           const double mu = (ra - rb) * iR;
           const double ab = aAB[a * natm + b];
-          double s, ds;
-          becke_s(mu + ab * (1.0 - mu * mu), s, ds);
+          double s, sb, ds;
+          becke_s(mu + ab * (1.0 - mu * mu), s, sb, ds);
           if (s < 1e-300) continue;
           const double c = Ka * ds / s * (1.0 - 2.0 * ab * mu);
           for (int x = 0; x < 3; ++x) {
@@ -621,35 +830,55 @@ hipError_t launch_ao_hess(int64_t npts, const double* pts, const ShellSet& S, in
 }
 
 hipError_t launch_xcg_rho(int64_t npts, int64_t nao, const double* ao, const double* Z, double* rho, double* grad,
-                          double* sigma, hipStream_t st) {
+                          double* sigma, double* Gd, hipStream_t st) {
   if (npts == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_xcg_rho, dim3((unsigned)npts), dim3(64), 0, st, npts, nao, ao, Z, rho, grad, sigma);
+  hipLaunchKernelGGL(k_xcg_rho, dim3((unsigned)npts), dim3(64), 0, st, npts, nao, ao, Z, rho, grad, sigma, Gd);
   return hipGetLastError();
 }
 
-hipError_t launch_xcg_gdot(int64_t npts, int64_t nao, const double* ao, const double* grad, double* Gd,
-                           hipStream_t st) {
-  const int64_t total = npts * nao;
-  if (total == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_xcg_gdot, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, npts, nao, ao, grad, Gd);
-  return hipGetLastError();
+// Workgroups of k_xcg_sum: 4 a CU, of at least 4 points a wavefront; part holds xcg_blocks(npts) * 3 nao words
+int xcg_blocks(int64_t npts) {
+  return (int)std::min<int64_t>(1024, (npts + 4 * kXcgWaves - 1) / (4 * kXcgWaves));
 }
-
-hipError_t launch_xcg_q(int64_t npts, int64_t nao, const double* ao, const double* Z, const double* X,
-                        const double* rho, const double* grad, const double* xc, const double* w,
-                        const int32_t* owner, double thresh, double* q, double* gout, double* fm, hipStream_t st) {
+// colsum[3][nao] += sum_g w_g q_{g m j}; gout of each owner += 2 sum_g w_g sum_m q
+hipError_t launch_xcg_sum(int64_t npts, int64_t nao, const double* ao, const double* Z, const double* X,
+                          const double* rho, const double* grad, const double* xc, const double* w,
+                          const int32_t* owner, double thresh, double* part, double* colsum, double* gout, double* fm,
+                          hipStream_t st) {
   if (npts == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_xcg_q, dim3((unsigned)npts), dim3(64), 0, st, npts, nao, ao, Z, X, rho, grad, xc, w, owner,
-                     thresh, q, gout, fm);
+  const int nb = xcg_blocks(npts);
+  const int64_t per = (npts + (int64_t)nb * kXcgWaves - 1) / ((int64_t)nb * kXcgWaves);
+  const int kt = (int)std::min<int64_t>(4, (nao + 63) / 64);   // 24 sums a lane at the most; wider spans by tiles
+  const dim3 grid((unsigned)nb, (unsigned)((nao + 64 * kt - 1) / (64 * kt))), block(64 * kXcgWaves);
+#define DFKS_XCG(K) \
+  if (kt == K) hipLaunchKernelGGL(k_xcg_sum<K>, grid, block, 0, st, npts, per, nao, ao, Z, X, rho, grad, xc, w, owner, \
+                                  thresh, part, gout, fm);
+  DFKS_XCG(1)
+  DFKS_XCG(2)
+  DFKS_XCG(3)
+  DFKS_XCG(4)
+#undef DFKS_XCG
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_xcg_cols, dim3((unsigned)((3 * nao + 15) / 16)), dim3(256), 0, st, nb, 3 * nao, part, colsum);
   return hipGetLastError();
 }
 
+// 64 KB of LDS hold the distances of 62 atoms for 4 wavefronts, of 234 for one
 hipError_t launch_becke_grad(int64_t n, const double* pts, const double* raw, const int32_t* owner, const double* f,
                              int natm, const double* atm, const double* invR, const double* aAB, double* gout,
                              hipStream_t st) {
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_becke_grad, dim3((unsigned)((n + 255) / 256)), dim3(256), 3 * natm * sizeof(double), st, n,
-                     pts, raw, owner, f, natm, atm, invR, aAB, gout);
+  const auto lds = [&](int nw) { return (size_t)natm * (3 + 32 * nw) * sizeof(double); };
+  const int nw = lds(4) <= 65536 ? 4 : 1;
+  if (lds(nw) <= 65536) {
+    const int64_t nb = std::min<int64_t>(1024 * 4 / nw, (n + 16 * nw - 1) / (16 * nw));
+    hipLaunchKernelGGL(k_becke_grad, dim3((unsigned)nb), dim3(64 * nw), lds(nw), st, n, pts, raw, owner, f, natm, atm,
+                       invR, aAB, gout);
+  } else {
+    hipLaunchKernelGGL(k_becke_grad_far, dim3((unsigned)((n + 255) / 256)), dim3(256), 3 * natm * sizeof(double), st, n,
+                       pts, raw, owner, f, natm, atm, invR, aAB, gout);
+  }
   return hipGetLastError();
 }
 

@@ -1,5 +1,6 @@
-"""One-electron integrals by shell pair, and the gradient's kernels where the shipped force vectors do
-not reach: nuclei and auxiliary shells around groups of 16, contractions, g spans, cartesian spans."""
+"""One-electron integrals by shell pair, Becke weights, and the gradient's kernels where the shipped force
+vectors do not reach: nuclei, points and auxiliary shells around groups of 16, contractions, g spans,
+cartesian spans, and molecules on both sides of what the LDS of the Becke kernels holds."""
 from types import SimpleNamespace
 
 import numpy as np
@@ -80,3 +81,51 @@ def test_gradient_terms(name, atoms):
         print(f"  {part:13s} max |d| {err:.2e} of {np.abs(want[k]).max():.2e}", flush=True)
         assert err < TOL_FORCE, part
     assert np.abs(sum(parts.values()).sum(0)).max() < 1e-8
+
+
+@pytest.mark.parametrize("natom,npts", [(1, 1), (2, 15), (5, 17), (128, 65), (129, 63), (513, 33)])
+def test_becke_weights_edges(natom, npts):
+    from dftax_amd import _native as N
+    from oracle import ref
+    rng = np.random.default_rng(natom)
+    side = int(np.ceil(natom ** (1 / 3)))
+    xyz = 2.5 * np.indices((side,) * 3).reshape(3, -1).T[:natom] + rng.uniform(-0.5, 0.5, (natom, 3))
+    bragg = rng.choice([0.66140414, 1.32280829, 1.13383567], natom)
+    own = rng.integers(0, natom, npts).astype(np.int32)
+    pts = xyz[own] + rng.normal(0.0, 1.0, (npts, 3))
+    raw = rng.uniform(0.1, 2.0, npts)
+    P = ref.becke_partition(pts, xyz, bragg)
+    want = raw * P[np.arange(npts), own] / P.sum(1)
+    got = N.becke_weights(pts, raw, own, xyz, bragg)
+    # about 10 natom roundings in each product of cell functions
+    assert np.abs(got - want).max() < 20 * max(natom, 8) * 2.3e-16 * raw.max()
+
+
+@pytest.mark.parametrize("far", [44, 46, 218])
+def test_xc_gradient_with_far_atoms(far):
+    """H2 molecules hundreds of Bohr away change nothing near a cluster: 62 and 64 atoms (four wavefronts and one
+    in the Becke gradient's LDS) and 236 (distances not kept) against the cluster's 18 alone."""
+    import torch
+    from dftax_amd import KS, becke, df, hip
+    from dftax_amd.forces import gradient_parts
+    from dftax_amd.system import Molecule
+    grid = becke(12, 26)
+    near = _molecule("h18")
+    rng = np.random.default_rng(3)
+    Z0 = np.linalg.qr(rng.normal(size=(18, 9)))[0]
+
+    def xc_grad(mol, extra):
+        ks = KS(mol, "PBE0", grid=grid, coulomb=df(chunk=None, engine=hip()))
+        Z = np.zeros((18 + extra, 9 + extra // 2))
+        Z[:18, :9] = Z0
+        for k in range(extra // 2):
+            Z[18 + 2 * k:20 + 2 * k, 9 + k] = 0.55
+        return gradient_parts(ks, SimpleNamespace(mo_coeff=torch.tensor(Z, device="cuda")), grid)["xc"]
+
+    base = xc_grad(near, 0)
+    k = np.arange(far)
+    xyz = np.stack([300.0 + 60.0 * (k // 2) + 1.4 * (k % 2), 0 * k, 0 * k], 1)
+    both = Molecule(["H"] * (18 + far), np.concatenate([near.coords, xyz]), "sto-3g", spherical=True)
+    err = np.abs(xc_grad(both, far)[:18] - base).max()
+    print(f"  {far} far atoms: max |d| {err:.2e} of {np.abs(base).max():.2e}", flush=True)
+    assert err < TOL_FORCE

@@ -165,6 +165,14 @@ hipError_t launch_gemm_partials(int prec, const GemmArgs& g, int nsplit, int sym
 hipError_t launch_gemm_reduce(int prec, const GemmArgs& g, double* C, double alpha, double beta, int nsplit, int sym,
                               const void* ws, hipStream_t st);
 hipError_t launch_gersh(int n, const double* F, double* lohi, double* st, hipStream_t s);
+hipError_t launch_lanczos(int n, const double* F, double* lz, hipStream_t s);
+int metric_ld(int n);
+size_t metric_chol_words(int n);
+hipError_t launch_metric_chol(int n, const double* V, double cutoff, double top, double* work, double* Lt, int* flag,
+                              hipStream_t st);
+size_t fit_words(int naux, int nfit);
+hipError_t launch_fit(int nao, int naux, int nfit, const double* I3, const double* Lt, int tri, double* W, double* B,
+                      hipStream_t st);
 hipError_t launch_sp2_lanczos(int n, const double* F, double* lz, double* st, hipStream_t s);
 hipError_t launch_sp2_init(int n, const double* F, const double* st, double* X, hipStream_t s);
 hipError_t launch_sp2_weyl(int n, const double* F, double* Fp, const double* pb, double* st, hipStream_t s);
@@ -1109,6 +1117,31 @@ void plan_xc_blocks(dfks_ctx* h, hipStream_t st) {
   h->xcb = true;
 }
 
+// Largest eigenvalue of the symmetric tridiagonal matrix of m Lanczos steps, ab = {alpha_k, beta_k} (it ends
+// where a beta is 0), by bisection on the number of eigenvalues below
+double tridiagonal_top(int m, const double* ab) {
+  double lo = ab[0], hi = ab[0];
+  int k = 0;
+  for (; k < m; ++k) {
+    const double r = (k > 0 ? std::abs(ab[2 * k - 1]) : 0.0) + (k + 1 < m ? std::abs(ab[2 * k + 1]) : 0.0);
+    lo = std::max(lo, ab[2 * k]);
+    hi = std::max(hi, ab[2 * k] + r);
+    if (ab[2 * k + 1] == 0.0) { ++k; break; }
+  }
+  for (int it = 0; it < 100 && hi > lo; ++it) {
+    const double x = 0.5 * (lo + hi);
+    int below = 0;
+    double d = 1.0;
+    for (int i = 0; i < k; ++i) {
+      const double b = i > 0 ? ab[2 * i - 1] : 0.0;
+      d = ab[2 * i] - x - b * b / (d != 0.0 ? d : 1e-300);
+      if (d < 0.0) ++below;
+    }
+    (below == k ? hi : lo) = x;
+  }
+  return hi;
+}
+
 void build_all(dfks_ctx* h, hipStream_t st) {
   h->rb = rb_acquire();
   RBCHK(rocblas_set_stream(h->rb, st));
@@ -1185,14 +1218,17 @@ void build_all(dfks_ctx* h, hipStream_t st) {
   sync(st);
   h->build_ms[1] = now_ms() - t0;
   t0 = now_ms();
-  // The metric's eigendecomposition (rocSOLVER, a long chain of small kernels
-  // on an n = naux matrix) needs only (P|Q): it runs on a side stream with its
-  // own rocBLAS handle while the three-centre build and the AO grid plan run on
-  // st, and is collected before the metric factor. d_U, d_w, d_e, the side
-  // stream and handle stay with this build until then.
+  // The metric's factor: the inverse Cholesky factor where no eigenvalue falls under the cutoff
+  // (metric.hip), else its eigendecomposition (rocSOLVER, a long chain of small kernels on an
+  // n = naux matrix). Either needs only (P|Q): it runs on a side stream with its own rocBLAS handle
+  // while the three-centre build and the AO grid plan run on st, and is collected before the fitted
+  // tensor. d_U, d_w, d_e, the Cholesky work, the side stream and handle stay with this build until then.
   double* d_U = dalloc<double>((size_t)naux * naux);
   double* d_w = dalloc<double>(naux);
   double* d_e = dalloc<double>(naux);
+  double* d_chol = dalloc<double>(metric_chol_words(naux));
+  double* d_Lc = dalloc<double>((size_t)naux * naux);
+  double* d_lzm = dalloc<double>(3 * (size_t)naux + kLzParts + 2 * kLzSteps);
   hipStream_t s_eig = nullptr;
   HIPCHK(hipStreamCreateWithFlags(&s_eig, hipStreamNonBlocking));
   rocblas_handle rb_eig = rb_acquire();
@@ -1209,19 +1245,38 @@ void build_all(dfks_ctx* h, hipStream_t st) {
     }
   } side{s_eig, rb_eig};
   RBCHK(rocblas_set_stream(rb_eig, s_eig));
+  // true: V's inverse Cholesky factor is in d_Lc (every eigenvalue above the cutoff)
+  const auto chol_launch = [&](const double* V, hipStream_t s) {
+    // A handle with 32-bit products keeps the eigenvectors: their fitted functions are sorted by scale, which
+    // 32 bits need (water dimer with recomputed slabs: E off by 5.5e-3 Ha with C^-T, under 1e-3 with U w^-1/2;
+    // (H2O)_8 def2-TZVP with B kept: J off by 4.8e-4 against 2.2e-4). And the Lanczos kernel's partial
+    // sums end at 4 kLzParts.
+    if (h->opt.precision == 1 || naux > 4 * kLzParts) return false;
+    HIPCHK(launch_lanczos(naux, V, d_lzm, s));
+    double ab[2 * kLzSteps];
+    HIPCHK(hipMemcpyAsync(ab, d_lzm + 3 * (size_t)naux + kLzParts, sizeof(ab), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    const double top = tridiagonal_top(kLzSteps, ab);
+    if (!(top > 0.0) || !(h->opt.metric_cutoff >= 0.0) || !std::isfinite(top)) return false;
+    // a little above the Ritz value; that no eigenvalue lies higher is one of the three factorisations
+    HIPCHK(launch_metric_chol(naux, V, h->opt.metric_cutoff, top * (1.0 + 1e-3), d_chol, d_Lc, h->d_info, s));
+    int flag = 0;
+    HIPCHK(hipMemcpyAsync(&flag, h->d_info, sizeof(int), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    return flag == 0;
+  };
   const auto eig_launch = [&](const double* V, rocblas_handle rb, hipStream_t s) {
     HIPCHK(hipMemcpyAsync(d_U, V, sizeof(double) * naux * naux, hipMemcpyDeviceToDevice, s));
     RBCHK(rocsolver_dsyevd(rb, rocblas_evect_original, rocblas_fill_upper, naux, d_U, naux, d_w, d_e, h->d_info));
   };
-  // metric pseudo-inverse factor L = U_keep w_keep^{-1/2} (nkeep columns kept by the relative cutoff) from
-  // the eigenpairs in d_U, d_w once stream s has finished them
-  // the side stream's eigensolve runs on its own host thread: rocSOLVER's divide and conquer
-  // holds its calling thread for much of its run, which would otherwise delay the three-centre
-  // launches queued behind it
+  // the side stream's factor runs on its own host thread: rocSOLVER's divide and conquer holds its
+  // calling thread for much of its run, which would otherwise delay the three-centre launches queued
+  // behind it
   struct EigThread {
     std::thread t;
     int code = 0;
     std::string msg;
+    bool chol = false;   // d_Lc holds the factor
     void finish() {
       if (t.joinable()) t.join();
       if (code) fail(code, msg);
@@ -1230,8 +1285,9 @@ void build_all(dfks_ctx* h, hipStream_t st) {
       if (t.joinable()) t.join();
     }
   } eig;
+  // metric pseudo-inverse factor L = U_keep w_keep^{-1/2} (nkeep columns kept by the relative cutoff) from
+  // the eigenpairs in d_U, d_w once stream s has finished them
   const auto eig_factor = [&](int& nkeep, hipStream_t s) {
-    if (s == s_eig) eig.finish();
     std::vector<double> w(naux);
     HIPCHK(hipMemcpyAsync(w.data(), d_w, sizeof(double) * naux, hipMemcpyDeviceToHost, s));
     int info = 0;
@@ -1259,11 +1315,12 @@ void build_all(dfks_ctx* h, hipStream_t st) {
   {
     int dev = 0;
     HIPCHK(hipGetDevice(&dev));
-    eig.t = std::thread([&eig, &eig_launch, h, dev, rb_eig, s_eig] {
+    eig.t = std::thread([&eig, &eig_launch, &chol_launch, h, dev, rb_eig, s_eig] {
       try {
         HIPCHK(hipSetDevice(dev));
         StreamScope ss(s_eig);
-        eig_launch(h->d_int2c, rb_eig, s_eig);
+        eig.chol = chol_launch(h->d_int2c, s_eig);
+        if (!eig.chol) eig_launch(h->d_int2c, rb_eig, s_eig);
         HIPCHK(hipStreamSynchronize(s_eig));
       } catch (const Fail& f) {
         eig.code = f.code;
@@ -1317,15 +1374,26 @@ void build_all(dfks_ctx* h, hipStream_t st) {
   h->build_ms[4] = now_ms() - t0;
   t0 = now_ms();
 
-  // the metric factor from the side stream's eigenpairs, then B
-  double* d_Lt = eig_factor(h->nfit, s_eig);
-  if (!h->recompute) {
-    // B_cm (nfit x nao^2) = Lt (nfit x naux) * int3c_cm (naux x nao^2)
-    h->d_B = dalloc<double>((size_t)nao * nao * h->nfit);
-    const double one = 1.0, zero = 0.0;
-    RBCHK(rocblas_dgemm_64(h->rb, rocblas_operation_none, rocblas_operation_none, h->nfit, (int64_t)nao * nao, naux,
-                           &one, d_Lt, h->nfit, d3, naux, &zero, h->d_B, h->nfit));
+  // the metric factor from the side stream, then B
+  eig.finish();
+  double* d_Lt = nullptr;
+  if (eig.chol) {
+    d_Lt = d_Lc;
+    d_Lc = nullptr;
+    h->nfit = naux;
+  } else {
+    d_Lt = eig_factor(h->nfit, s_eig);
+  }
+  const auto fit = [&](const double* I3, const double* Lt, int nfit, bool tri, double* B) {
+    double* W = dalloc<double>(fit_words(naux, nfit));
+    const hipError_t e = launch_fit(nao, naux, nfit, I3, Lt, tri, W, B, st);
+    dfree(W);
+    HIPCHK(e);
     sync(st);
+  };
+  if (!h->recompute) {
+    h->d_B = dalloc<double>((size_t)nao * nao * h->nfit);
+    fit(d3, d_Lt, h->nfit, eig.chol, h->d_B);
     h->d_Lt = d_Lt;   // kept: the nuclear gradient maps fitted quantities back to (P|Q) (nfit naux words)
     if (h->opt.keep_int3c) h->d_int3c = d3;
     else dfree(d3);
@@ -1359,10 +1427,7 @@ void build_all(dfks_ctx* h, hipStream_t st) {
     eig_launch(d2lr, h->rb, st);
     double* d_Ltlr = eig_factor(h->nfit_lr, st);
     h->d_Blr = dalloc<double>((size_t)nao * nao * h->nfit_lr);
-    const double one = 1.0, zero = 0.0;
-    RBCHK(rocblas_dgemm_64(h->rb, rocblas_operation_none, rocblas_operation_none, h->nfit_lr, (int64_t)nao * nao,
-                           naux, &one, d_Ltlr, h->nfit_lr, d3lr, naux, &zero, h->d_Blr, h->nfit_lr));
-    sync(st);
+    fit(d3lr, d_Ltlr, h->nfit_lr, false, h->d_Blr);
     dfree(d3lr);
     dfree(d2lr);
     dfree(d_Ltlr);
@@ -1373,7 +1438,7 @@ void build_all(dfks_ctx* h, hipStream_t st) {
   sync(st);
   h->build_ms[3] = now_ms() - t0;
   t0 = now_ms();
-  dfree(d_U); dfree(d_w); dfree(d_e);
+  dfree(d_U); dfree(d_w); dfree(d_e); dfree(d_chol); dfree(d_Lc); dfree(d_lzm);
 
   // Fock-build scratch: exchange intermediate for up to nf_chunk factor columns
   h->d_Tx = dalloc<double>((size_t)nao * std::max(h->nfit, h->nfit_lr) * h->nf_chunk);

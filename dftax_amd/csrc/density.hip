@@ -999,9 +999,9 @@ __global__ __launch_bounds__(64) void k_lz_bounds(int n, const double* __restric
   st[kSpEmax] = fmin(st[kSpEmax], emax);
 }
 
-// The Lanczos bounds after launch_gersh: kLzSteps steps, kernels through launch_k
-// (so that they can be recorded as a graph). lz: 3 n + kLzParts + 2 kLzSteps doubles.
-hipError_t launch_sp2_lanczos(int n, const double* F, double* lz, double* st, hipStream_t s) {
+// kLzSteps Lanczos steps of the symmetric F, kernels through launch_k (so that they can be
+// recorded as a graph). lz: 3 n + kLzParts + 2 kLzSteps doubles, the coefficients last.
+hipError_t launch_lanczos(int n, const double* F, double* lz, hipStream_t s) {
   const int nparts = (n + 3) / 4;
   if (nparts > kLzParts) return hipErrorInvalidValue;
   hipError_t e = launch_k(k_lz_start, dim3(1), dim3(1024), s, n, lz);
@@ -1009,6 +1009,12 @@ hipError_t launch_sp2_lanczos(int n, const double* F, double* lz, double* st, hi
     e = launch_k(k_lz_matvec, dim3((unsigned)nparts), dim3(256), s, n, F, lz);
     if (e == hipSuccess) e = launch_k(k_lz_update, dim3(1), dim3(1024), s, n, nparts, k, lz);
   }
+  return e;
+}
+
+// The Lanczos bounds after launch_gersh
+hipError_t launch_sp2_lanczos(int n, const double* F, double* lz, double* st, hipStream_t s) {
+  hipError_t e = launch_lanczos(n, F, lz, s);
   if (e == hipSuccess) e = launch_k(k_lz_bounds, dim3(1), dim3(64), s, n, (const double*)lz, st);
   return e;
 }

@@ -217,15 +217,16 @@ __global__ __launch_bounds__(256) void k_copy_pad(int nr, int nc, int64_t ldi, c
 }
 
 // B[(m, n)][q] = sum_P I3[(m, n)][P] W[q][P] over the pairs m >= n, to both orders of the pair. 128 pairs x 128
-// q a workgroup, 64 x 64 a wavefront: every fragment of a wavefront's 16 k is one 32-byte run of a row, loaded
-// from global memory while the 16 k before it multiply (a CU's four wavefronts ask for 16 bytes a clock, a
-// quarter of what L1 gives, so LDS would only add a copy). tri: W is lower triangular (q, P), and a tile
-// stops at its last q. Workgroup x runs on XCD x % 8: an XCD takes whole strips of pairs, their q tiles
-// longest first, so a strip's integrals are read from HBM once. W: rows of ldw = 16 ceil(naux / 16), zero past naux
-// and past nfit up to a whole tile.
-// Bound by the matrix cores (54 TF/s): 21.5 ms for 480 functions and 2255 fitting functions, eigenvectors, where
-// the product over both orders of a pair takes 33.3 ms at 70 TF/s; (H2O)_24 def2-TZVP, tri, 82 ms against 228.
-__global__ __launch_bounds__(256, 1) void k_fit(int nao, int naux, int nfit, int64_t npair,
+// q a workgroup, 64 x 64 a wavefront: both operands have k along their rows, so a wavefront's fragments of 8 k
+// are 64-byte runs of its rows, loaded from global memory into registers while the 8 k before them multiply.
+// L1 and L2 hold what the wavefronts share; LDS would add a copy and a barrier. Two wavefronts a SIMD: with one
+// and three groups in flight the compiler moves the sums between both register files every turn (54 TF/s).
+// tri: W is lower triangular (q, P), and a tile stops at its last q. Workgroup x runs on XCD x % 8: an XCD
+// takes whole strips of pairs, their q tiles longest first, so a strip's integrals are read from HBM once. W:
+// rows of ldw = 16 ceil(naux / 16), zero past naux and past nfit up to a whole tile.
+// Bound by the matrix cores (63 TF/s): 18.4 ms for 480 functions and 2255 fitting functions, eigenvectors, where
+// the product over both orders of a pair takes 33.3 ms at 70 TF/s; (H2O)_24 def2-TZVP, tri, 68 ms against 228.
+__global__ __launch_bounds__(256, 2) void k_fit(int nao, int naux, int nfit, int64_t npair,
                                                 const double* __restrict__ I3, const double* __restrict__ W, int ldw,
                                                 int tri, double* __restrict__ B) {
   constexpr int MI = 4, TR = 32 * MI;   // tiles of 16 pairs a wavefront, pairs a workgroup
@@ -234,7 +235,8 @@ __global__ __launch_bounds__(256, 1) void k_fit(int nao, int naux, int nfit, int
   const int64_t ip = blockIdx.x / 8, strip = ip / nqt * 8 + blockIdx.x % 8, r0 = TR * strip;
   if (r0 >= npair) return;
   const int q0 = 128 * (nqt - 1 - (int)(ip % nqt));
-  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // uniform: no divergent loop around the sums
   const int wm = 16 * MI * (wave >> 1), wn = 64 * (wave & 1);
   if (tid < TR) {
     const int64_t r = min(r0 + tid, npair - 1);
@@ -247,56 +249,61 @@ __global__ __launch_bounds__(256, 1) void k_fit(int nao, int naux, int nfit, int
   }
   __syncthreads();
   const double* xa[MI];
-  const double* wb[4];
 #pragma unroll
-  for (int i = 0; i < MI; ++i) xa[i] = I3 + s_mn[wm + 16 * i + li] * naux + 4 * lk;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    wb[i] = W + (int64_t)(q0 + wn + 16 * i + li) * ldw + 4 * lk;
-  }
+  for (int i = 0; i < MI; ++i) xa[i] = I3 + s_mn[wm + 16 * i + li] * naux + 2 * lk;
+  // W's rows by a uniform base and one 32-bit offset a lane: with the sums and two groups in flight the
+  // registers are full
+  const double* wrow = W + (int64_t)(q0 + wn) * ldw;
+  const uint32_t woff = (uint32_t)(li * ldw + 2 * lk);
   const int kend = tri ? min(naux, q0 + wn + 64) : naux;
-  const int nfull = kend / 16, tail = kend % 16;   // tail: the last row's integrals end there
+  const int ng = kend / 8, tail = kend % 8;   // tail: the last row's integrals end there
   f64x4 acc[MI][4] = {};
-  const auto mul = [&](const f64x4 (&x)[MI], const f64x4 (&y)[4]) {
+  f64x2u x[2][MI], y[2][4];
+  const auto mul = [&](const f64x2u (&x)[MI], const f64x2u (&y)[4]) {
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
+    for (int s = 0; s < 2; ++s)
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i][s], y[j][s], acc[i][j], 0, 0, 0);
   };
-  const auto load = [&](int q, f64x4 (&x)[MI], f64x4 (&y)[4]) {
+  const auto load = [&](int q, f64x2u (&x)[MI], f64x2u (&y)[4]) {   // group q from xa, wrow
 #pragma unroll
-    for (int i = 0; i < MI; ++i) {
-      const f64x2u lo = *reinterpret_cast<const f64x2u*>(xa[i] + 16 * q);
-      const f64x2u hi = *reinterpret_cast<const f64x2u*>(xa[i] + 16 * q + 2);
-      x[i] = f64x4{lo[0], lo[1], hi[0], hi[1]};
-    }
+    for (int i = 0; i < MI; ++i) x[i] = *reinterpret_cast<const f64x2u*>(xa[i] + 8 * q);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) y[i] = *reinterpret_cast<const f64x4*>(wb[i] + 16 * q);
+    for (int i = 0; i < 4; ++i) y[i] = *reinterpret_cast<const f64x2u*>(wrow + 16 * i * (int64_t)ldw + 8 * q + woff);
   };
-  f64x4 x[MI], y[4], xn[MI], yn[4];
-  if (nfull > 0) load(0, x, y);
-  for (int q = 0; q < nfull; q += 2) {
-    load(min(q + 1, nfull - 1), xn, yn);
-    mul(x, y);
-    if (q + 1 >= nfull) break;
-    load(min(q + 2, nfull - 1), x, y);
-    mul(xn, yn);
+  const auto step = [&](int n) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i) xa[i] += 8 * n;
+    wrow += 8 * n;
+  };
+  if (ng > 0) load(0, x[0], y[0]);
+  int left = ng;
+  for (; left >= 3; left -= 2) {
+    load(1, x[1], y[1]);
+    mul(x[0], y[0]);
+    load(2, x[0], y[0]);
+    mul(x[1], y[1]);
+    step(2);
   }
+  if (left > 1) load(1, x[1], y[1]);
+  if (left > 0) mul(x[0], y[0]);
+  if (left > 1) mul(x[1], y[1]);
   if (tail > 0) {
+    step(left);
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const int k = 4 * lk + s;
-        const double v = xa[i][16 * nfull + (k < tail ? s : -4 * lk)];   // clamped to the group's first
-        x[i][s] = k < tail ? v : 0.0;
+      for (int s = 0; s < 2; ++s) {
+        const bool in = 2 * lk + s < tail;
+        const double v = xa[i][in ? s : -2 * lk];   // clamped to the group's first
+        x[0][i][s] = in ? v : 0.0;
       }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) y[i] = *reinterpret_cast<const f64x4*>(wb[i] + 16 * nfull);
-    mul(x, y);
+    for (int i = 0; i < 4; ++i) y[0][i] = *reinterpret_cast<const f64x2u*>(wrow + 16 * i * (int64_t)ldw + woff);
+    mul(x[0], y[0]);
   }
 #pragma unroll
   for (int i = 0; i < MI; ++i)

@@ -1508,6 +1508,19 @@ int split_for(int64_t tiles, int64_t K) {
   if (s * tiles > 256 && s * tiles < 1024) s = s * tiles / 256 * 256 / tiles;
   return (int)std::max<int64_t>(1, s);
 }
+// Splits for k_gemm_nt, whose splits go to the 8 XCDs in turn: an XCD holds 256 wavefronts of it at a time, and
+// as many splits a XCD (of at least 128 k, 64 in all) as fill whole rounds best are taken. 465 functions, 36
+// tiles of a wavefront: 7 a XCD fill 252 of 256, 1.00 ms; 8 start a second round, 1.21 ms.
+int nt_split(int64_t tiles, int64_t K) {
+  const int64_t most = std::min<int64_t>(8, std::max<int64_t>(1, K / (8 * 128)));
+  int64_t best = 1;
+  double fill = 0.0;
+  for (int64_t r = 1; r <= most; ++r) {
+    const double f = (double)(r * tiles) / (double)((r * tiles + 255) / 256 * 256);
+    if (f > fill * 1.02) { fill = f; best = r; }
+  }
+  return (int)std::min<int64_t>(8 * best, std::max<int64_t>(1, K / 128));
+}
 
 // (mn|P) for the functions of slab s into d_slab, layout [m][n][p] with
 // p = P - p0 (kept bra pairs only; the others stay zero).
@@ -1591,7 +1604,7 @@ void coulomb_recompute(dfks_ctx* h, hipStream_t st) {
 // that shape. Both compute the same T to rounding.
 // Per-shape choice among the variants of a product. Tags and variants:
 //   0  FP64 exchange T = B^T C:      0 rocBLAS, 1 k_gemm, 2 k_gemm_w8, 3 k_gemm_t
-//   3  FP64 exchange K partials:     0 k_gemm, 1 k_gemm_w8, 2 k_gemm_w8 split by XCD (base 1)
+//   3  FP64 exchange K partials:     0 k_gemm, 1 k_gemm_w8, 2 k_gemm_nt (base 1)
 //   4  split-BF16 exchange T:        0 k_gemm, 1 k_gemm_b3w8 (base 1)
 //   5  SP2 product partials X X:     0 k_gemm, 1 k_gemm_w8   (base 1)
 //   6  split-BF16 exchange K:        0 k_gemm, 1 k_gemm split by XCD (base 1)
@@ -1685,11 +1698,12 @@ void k_product_f64(dfks_ctx* h, int64_t kd, double* Kout, double sg, double beta
   const int nao = h->nao;
   const int ntn = (nao + 127) / 128;
   const int nsplit = split_for((int64_t)ntn * (ntn + 1) / 2, kd);
-  const int nsx = 16;   // the split by XCD: each XCD's tiles on the same k-window of T
+  // k_gemm_nt: whole splits on an XCD
+  const int nsx = nt_split((int64_t)((nao + 63) / 64) * ((nao + 63) / 64 + 1) / 2, kd);
   if (h->opt.gemm != 1) {
     const GemmArgs g{nao, nao, kd, h->d_Tx, kd, true, h->d_Tx, kd, true};
     const int v = tuned_product(h, 3, nao, kd, nsplit, 3, 1, [&](int c) {
-      HIPCHK(launch_gemm_partials(kF64, g, c == 2 ? nsx : nsplit, c == 2 ? 3 : 1, h->d_gws, c == 2 ? 1 : c, st));
+      HIPCHK(launch_gemm_partials(kF64, g, c == 2 ? nsx : nsplit, 1, h->d_gws, c, st));
     }, st);
     HIPCHK(launch_gemm_reduce(kF64, g, Kout, sg, beta, v == 2 ? nsx : nsplit, 1, h->d_gws, st));
   } else {

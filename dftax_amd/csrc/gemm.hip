@@ -339,19 +339,14 @@ template <bool AK, int NJ>
 __global__ __launch_bounds__(512, 1) void k_gemm_w8(int64_t M, int N, int64_t K, const double* __restrict__ A,
                                                    int64_t lda, const double* __restrict__ B, int64_t ldb,
                                                    double* __restrict__ C, int64_t ldc, int64_t split_stride,
-                                                   int64_t kchunk, int sym, int ntiles, int vec_a, int vec_b,
-                                                   RowDot rd) {
+                                                   int64_t kchunk, int sym, int vec_a, int vec_b, RowDot rd) {
   constexpr int BN = 32 * NJ;
   __shared__ double sA[2][kW8BM][kW8BK + 1];
   __shared__ double sB[2][BN][kW8BK + 1];
-  // split-by-XCD mode (sym bit 1) as in k_gemm
-  const bool xs = (sym & 2) != 0;
-  const int tile = xs ? (int)(blockIdx.x >> 3) : (int)blockIdx.x;
-  const int split = xs ? (int)((blockIdx.x & 7) + 8 * blockIdx.z) : (int)blockIdx.z;
-  if (tile >= ntiles) return;
+  const int tile = (int)blockIdx.x, split = (int)blockIdx.z;
   const int ntn = (N + BN - 1) / BN;
   int tm, tn;
-  tile_of(tile, ntn, (sym & 1) != 0, tm, tn);
+  tile_of(tile, ntn, sym != 0, tm, tn);
   const int64_t m0 = (int64_t)tm * kW8BM;
   const int n0 = tn * BN;
   const int64_t k_begin = (int64_t)split * kchunk;
@@ -847,32 +842,138 @@ static hipError_t launch_gemm_t(const GemmArgs& g, Out* C, int64_t ldc, int nspl
   return run(k_gemm<PREC, false, false, Out, NJ>);
 }
 
+// 16 bytes of a row: rows start on any 8 bytes
+typedef double dbl2u __attribute__((ext_vector_type(2), aligned(8)));
+
+// Split-K partial tiles of A B^T for K-contiguous operands (the exchange K = T T^T). 128 x 128 a workgroup,
+// 64 x 64 a wavefront, no LDS: a wavefront's fragments of 8 k are 64-byte runs of its rows, loaded from global
+// memory into registers while the 8 k before them multiply; what the wavefronts share comes from L1 and L2.
+// Two wavefronts a SIMD, and groups of 8 k rather than 16, so that sums and groups fit the registers without
+// copies. Workgroup x runs on XCD x % 8: an XCD takes whole splits, all tiles of a split before the next, so
+// their windows of A and B are read from HBM once. Bound by the matrix cores. 144 functions: 0.055 ms (8-wavefront
+// tiles 0.083, k_gemm 0.129); 465: 1.01 (1.42, 2.42); 602: 1.00 (1.03, 1.23); 1032: 8.07 (8.50, 9.25). Where a
+// round is left half empty the 8-wavefront tiles stay ahead (344 functions, 36,800 k: 0.151 against 0.192).
+__global__ __launch_bounds__(256, 2) void k_gemm_nt(int M, int N, int64_t K, const double* __restrict__ A, int64_t lda,
+                                                    const double* __restrict__ B, int64_t ldb, double* __restrict__ C,
+                                                    int64_t split_stride, int64_t kchunk, int nsplit, int ntiles,
+                                                    int sym) {
+  const int per = (ntiles + 3) / 4, ip = (int)(blockIdx.x >> 3), split = ip / per * 8 + (int)(blockIdx.x & 7);
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);   // uniform: no divergent loop around the sums
+  const int tile = 4 * (ip % per) + wave;
+  if (split >= nsplit || tile >= ntiles) return;
+  int tm, tn;
+  tile_of(tile, (N + 63) / 64, sym != 0, tm, tn);
+  const int m0 = 64 * tm, n0 = 64 * tn;
+  const int64_t k_begin = min(K, split * kchunk), k_end = min(K, k_begin + kchunk);
+  const double *pa[4], *pb[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {   // a row past the end repeats the last one and is not stored
+    pa[i] = A + (int64_t)min(m0 + 16 * i + li, M - 1) * lda + k_begin + 2 * lk;
+    pb[i] = B + (int64_t)min(n0 + 16 * i + li, N - 1) * ldb + k_begin + 2 * lk;
+  }
+  dbl4 acc[4][4] = {};
+  dbl2u x[2][4], y[2][4];
+  const auto mul = [&](const dbl2u (&x)[4], const dbl2u (&y)[4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i][s], y[j][s], acc[i][j], 0, 0, 0);
+  };
+  const auto load = [&](int q, dbl2u (&x)[4], dbl2u (&y)[4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      x[i] = *reinterpret_cast<const dbl2u*>(pa[i] + 8 * q);
+      y[i] = *reinterpret_cast<const dbl2u*>(pb[i] + 8 * q);
+    }
+  };
+  const auto step = [&](int n) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      pa[i] += 8 * n;
+      pb[i] += 8 * n;
+    }
+  };
+  const int len = (int)(k_end - k_begin), tail = len & 7;
+  int left = len >> 3;
+  if (left > 0) load(0, x[0], y[0]);
+  for (; left >= 3; left -= 2) {
+    load(1, x[1], y[1]);
+    mul(x[0], y[0]);
+    load(2, x[0], y[0]);
+    mul(x[1], y[1]);
+    step(2);
+  }
+  if (left > 1) load(1, x[1], y[1]);
+  if (left > 0) mul(x[0], y[0]);
+  if (left > 1) mul(x[1], y[1]);
+  if (tail > 0) {
+    step(left);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const bool in = 2 * lk + s < tail;
+        const double u = pa[i][in ? s : -2 * lk], v = pb[i][in ? s : -2 * lk];   // clamped to the group's first
+        x[0][i][s] = in ? u : 0.0;
+        y[0][i][s] = in ? v : 0.0;
+      }
+    mul(x[0], y[0]);
+  }
+  double* __restrict__ Cz = C + (int64_t)split * split_stride;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int gm = m0 + 16 * i + lk + 4 * r;
+      if (gm >= M) continue;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int gn = n0 + 16 * j + li;
+        if (gn < N) Cz[(int64_t)gm * N + gn] = acc[i][j][r];
+      }
+    }
+}
+
+static hipError_t launch_nt_partials(const GemmArgs& g, double* ws, int nsplit, int sym, hipStream_t st) {
+  if (!g.a_kcontig || !g.b_kcontig) return hipErrorInvalidValue;
+  const int64_t ntm = ((int64_t)g.M + 63) / 64, ntn = ((int64_t)g.N + 63) / 64;
+  const int64_t ntl = (sym & 1) ? ntn * (ntn + 1) / 2 : ntm * ntn;
+  const int64_t kchunk = ((g.K + nsplit - 1) / nsplit + 7) / 8 * 8;
+  const int64_t nb = (int64_t)(nsplit + 7) / 8 * 8 * ((ntl + 3) / 4);
+  if (nb > 0x7fffffff || kchunk > 0x7fffffff) return hipErrorInvalidValue;
+  return launch_k(k_gemm_nt, dim3((unsigned)nb), dim3(256), st, (int)g.M, (int)g.N, (int64_t)g.K,
+                  static_cast<const double*>(g.A), g.lda, static_cast<const double*>(g.B), g.ldb, ws,
+                  (int64_t)g.M * g.N, kchunk, nsplit, (int)ntl, sym & 1);
+}
+
 // k_gemm_w8 launch: ldc, split and symmetric mode as launch_gemm_t (NJ = 5
 // only without the symmetric mode); B must be K-contiguous.
 template <int NJ>
 static hipError_t launch_w8_t(const GemmArgs& g, double* C, int64_t ldc, int nsplit, int sym, hipStream_t st,
                               const RowDot& rd = RowDot()) {
   constexpr int BN = 32 * NJ;
-  if (!g.b_kcontig || ((sym & 1) && NJ != 4)) return hipErrorInvalidValue;
+  if (!g.b_kcontig || (sym && NJ != 4)) return hipErrorInvalidValue;
   if (rd.out && (g.N > BN || nsplit != 1 || sym || rd.nq < kW8BM)) return hipErrorInvalidValue;
-  const bool xs = (sym & 2) != 0;
-  if (xs && nsplit % 8 != 0) return hipErrorInvalidValue;
   const int64_t ntm = ((int64_t)g.M + kW8BM - 1) / kW8BM, ntn = (g.N + BN - 1) / BN;
-  const int64_t ntl = (sym & 1) ? ntn * (ntn + 1) / 2 : ntm * ntn;
-  if (8 * ntl > 0x7fffffff || nsplit > 65535) return hipErrorInvalidValue;
+  const int64_t ntl = sym ? ntn * (ntn + 1) / 2 : ntm * ntn;
+  if (ntl > 0x7fffffff || nsplit > 65535) return hipErrorInvalidValue;
   int64_t kchunk = (g.K + nsplit - 1) / nsplit;
   kchunk = (kchunk + kW8BK - 1) / kW8BK * kW8BK;
   const double* A = static_cast<const double*>(g.A);
   const double* B = static_cast<const double*>(g.B);
   const int vec_a = ((uintptr_t)A % 16 == 0) && (g.lda % 2 == 0);
   const int vec_b = ((uintptr_t)B % 16 == 0) && (g.ldb % 2 == 0);
-  const dim3 grid = xs ? dim3((unsigned)(8 * ntl), 1, (unsigned)(nsplit / 8)) : dim3((unsigned)ntl, 1, (unsigned)nsplit);
+  const dim3 grid((unsigned)ntl, 1, (unsigned)nsplit);
   const int64_t split_stride = (int64_t)g.M * ldc;
   if (g.a_kcontig)
     return launch_k(k_gemm_w8<true, NJ>, grid, dim3(512), st, (int64_t)g.M, g.N, g.K, A, g.lda, B, g.ldb, C, ldc,
-                    split_stride, kchunk, sym, (int)ntl, vec_a, vec_b, rd);
+                    split_stride, kchunk, sym, vec_a, vec_b, rd);
   return launch_k(k_gemm_w8<false, NJ>, grid, dim3(512), st, (int64_t)g.M, g.N, g.K, A, g.lda, B, g.ldb, C, ldc,
-                  split_stride, kchunk, sym, (int)ntl, vec_a, vec_b, rd);
+                  split_stride, kchunk, sym, vec_a, vec_b, rd);
 }
 
 // C = A B^T in FP64 by k_gemm_w8, no split (ldc = N): 128- or 160-wide N
@@ -901,8 +1002,6 @@ template <int NJ>
 struct TTile {
   static constexpr int MI = NJ <= 4 ? 4 : 2, ROWS = 64 * MI;   // 16-row blocks per wavefront, rows per workgroup
 };
-// 16 bytes of A: rows are 8-byte aligned only when M is odd
-typedef double dbl2u __attribute__((ext_vector_type(2), aligned(8)));
 
 template <int NJ>
 __global__ __launch_bounds__(256, NJ <= 1 ? 4 : 2) void k_gemm_t(int64_t M, int N, int K, const double* __restrict__ A,
@@ -1048,12 +1147,13 @@ hipError_t launch_gemm_t64(const GemmArgs& g, double* C, const RowDot& rd, hipSt
 
 // Split-K partial tiles of A B^T into ws (nsplit x M x N, FP64 for kF64 and
 // FP32 for kBF16x3; upper tiles only in the symmetric mode). variant 1 takes
-// the 8-wavefront FP64 tile where it applies (B K-contiguous), 0 k_gemm.
+// the 8-wavefront FP64 tile where it applies (B K-contiguous), 2 k_gemm_nt (both operands K-contiguous), 0 k_gemm.
 hipError_t launch_gemm_partials(int prec, const GemmArgs& g, int nsplit, int sym, void* ws, int variant,
                                 hipStream_t st) {
   if (g.M <= 0 || g.N <= 0) return hipSuccess;
   if (!ws || nsplit < 1) return hipErrorInvalidValue;
   if (prec == kF64) {
+    if (variant == 2) return launch_nt_partials(g, static_cast<double*>(ws), nsplit, sym, st);
     if (variant == 1 && g.b_kcontig) return launch_w8_t<4>(g, static_cast<double*>(ws), g.N, nsplit, sym, st);
     return launch_gemm_t<kF64, double>(g, static_cast<double*>(ws), g.N, nsplit, sym, st);
   }

@@ -43,7 +43,8 @@ class HipSpec:
     ``"mfma"``, with the 8-wavefront 128 x 160 tile for T) or ``"mfma8d"`` (as
     ``"mfma8"``, with each product's further variant where it has one: the
     split-BF16 T with two k-steps of operands in flight, the FP64 T by the
-    kernel whose tile is as wide as the factor, the FP64 K split by XCD). Mixed steps use the library's
+    kernel whose tile is as wide as the factor, the FP64 K by wavefront tiles without
+    LDS). Mixed steps use the library's
     split-BF16 kernels for the exchange products and FP32 rocBLAS products on
     the compact XC grid. ``metric_cutoff`` is the relative eigenvalue cutoff of the
     metric pseudo-inverse (terms.py:190-192). ``density`` is how each SCF step

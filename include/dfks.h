@@ -89,7 +89,7 @@ typedef struct {
                               for all; 2 library kernels for all; 3 as 2 with the 8-wavefront tile for
                               T; 4 as 3 with each product's further library variant where it has one
                               (split-BF16 T with two k-steps of operands in flight, FP64 T by the tile
-                              as wide as the factor, FP64 K split by XCD). Mixed steps always use the library's split-BF16 kernels. */
+                              as wide as the factor, FP64 K by wavefront tiles without LDS). Mixed steps always use split-BF16 kernels. */
   int32_t density;         /* SCF density from the orthonormal-basis Fock matrix: 0 spectral projection
                               (SP2 purification + pivoted Cholesky factor; the eigensolver runs only
                               when purification does not converge, and once for dfks_scf_result's

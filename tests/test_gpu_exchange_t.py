@@ -33,3 +33,29 @@ def test_factor_widths(pairs, name, nf):
         got.append(k.coulomb.energy_fock_factored(Cf))
     for a, b in zip(*got):
         assert float((a - b).abs().max()) < TOL * max(1.0, float(b.abs().max()))
+
+
+@pytest.mark.parametrize("nao,naux,nf", [(1, 3, 1), (63, 5, 3), (64, 16, 8), (65, 17, 1), (128, 7, 1), (129, 40, 33),
+                                         (200, 130, 9)])
+def test_exchange_k_tiles(nao, naux, nf):
+    """K = T T^T on tiles of 64 functions and groups of 8 k: sizes on either side of both, rows that start on odd
+    words, fewer k than splits."""
+    import numpy as np
+    import torch
+    from dftax_amd.ks import HipDFKS, HipSpec
+    from dftax_amd.system import Molecule
+    from dftax_amd.xc import PBE0
+    from test_gpu_eri_pair import _basis
+    rng = np.random.default_rng(nao)
+    mol = Molecule(["O"] * 2, np.array([[0.0, 0.0, 0.0], [0.0, 0.1, 2.1]]), "sto-3g")
+    site = 1.6 * np.indices((6, 6, 6)).reshape(3, -1).T + rng.uniform(-0.1, 0.1, (216, 3))
+    orb = _basis([(0, 0, x, [1.1]) for x in site[:nao]], True)
+    aux = _basis([(0, 0, x, [0.9]) for x in site[:naux]], True)
+    got = []
+    for gemm in ("mfma8d", "rocblas"):
+        c = HipDFKS(orb, aux, mol, np.zeros((1, 3)) + 5.0, np.ones(1), PBE0(), 2, HipSpec(gemm=gemm), chunk=None)
+        g = torch.Generator(device=c.device).manual_seed(nf)
+        Cf = torch.randn((c.nao, nf), dtype=torch.float64, device=c.device, generator=g) * (0.5 / nf ** 0.5)
+        got.append(c.energy_fock_factored(Cf))
+    for a, b in zip(*got):
+        assert float((a - b).abs().max()) < TOL * max(1.0, float(b.abs().max()))

@@ -165,6 +165,16 @@ hipError_t launch_gemm_partials(int prec, const GemmArgs& g, int nsplit, int sym
 hipError_t launch_gemm_reduce(int prec, const GemmArgs& g, double* C, double alpha, double beta, int nsplit, int sym,
                               const void* ws, hipStream_t st);
 hipError_t launch_gersh(int n, const double* F, double* lohi, double* st, hipStream_t s);
+size_t plan_sort_words(int64_t ng);
+hipError_t launch_plan_sort(int64_t ng, const double* X, uint32_t* work, const int32_t** idx, hipStream_t st);
+hipError_t launch_plan_scan(int64_t ng, const double* X, const int32_t* idx, const ShellSet& S, const double* rcut,
+                            int32_t* loc, int32_t* nfn, int32_t* nshell, int32_t* nblk_of, hipStream_t st);
+hipError_t launch_plan_fill(int64_t ng, const double* X, const double* gw, const int32_t* idx, const ShellSet& S,
+                            const int32_t* loc, const int32_t* order, const int32_t* w, const int64_t* col0,
+                            const int64_t* shoff, double* pts, double* wts, int32_t* cols, int2* shl, hipStream_t st);
+hipError_t launch_plan_rows(int64_t nblk, const ShellSet& S, const int32_t* loc, const int32_t* order, const int32_t* w,
+                            const int64_t* col0, const int64_t* q0, const int64_t* vrow, int64_t* vprow, int64_t* vpcol,
+                            int32_t* vlen, hipStream_t st);
 hipError_t launch_lanczos(int n, const double* F, double* lz, hipStream_t s);
 int metric_ld(int n);
 size_t metric_chol_words(int n);
@@ -841,7 +851,6 @@ void setup_slabs(dfks_ctx* h, hipStream_t st) {
 // ---------------------------------------------------------------------------
 // Compact XC grid
 // ---------------------------------------------------------------------------
-constexpr int kXcG = 128;          // points per block
 constexpr double kXcTau = 1e-14;   // AO value / gradient bound below which a shell is dropped in a block
 
 // max over r >= d of r^p exp(-a r^2)
@@ -879,104 +888,64 @@ double shell_radius(const Basis& B, int s) {
   return hi;
 }
 
-uint32_t spread3(uint32_t v) {  // 10 bits -> every third bit
-  v &= 0x3ff;
-  v = (v | (v << 16)) & 0x030000ff;
-  v = (v | (v << 8)) & 0x0300f00f;
-  v = (v | (v << 4)) & 0x030c30c3;
-  v = (v | (v << 2)) & 0x09249249;
-  return v;
-}
-
-// Blocks of kXcG grid points in Morton order; per block the shells whose bound
-// reaches kXcTau anywhere in the block's bounding sphere; blocks binned by the
-// padded count of their functions (multiples of 32). Uploads the binned points,
-// weights, column maps, shell lists and the row lists of the Vxc assembly, and
-// evaluates the compact AO values and gradients (resident).
 // Whether a bin's blocks go through the one-launch FP64 kernels (the others, and every bin with
 // gemm = rocblas, take rocBLAS batched products bin by bin)
 bool xc_one_launch(const dfks_ctx* h, const dfks_ctx::XcBin& bn) {
   return h->opt.gemm != 1 && bn.n <= kXfMaxN && (int64_t)h->nao * h->nao <= 0x7fffffff;
 }
 
+// Blocks of kXcG grid points in Morton order; per block the shells whose bound
+// reaches kXcTau anywhere in the block's bounding sphere; blocks binned by the
+// padded count of their functions (multiples of 32). The lists are formed
+// on the device (xc_plan.hip); the host sees the blocks' counts alone, which
+// order the blocks and size the buffers. Ends with the compact AO values and gradients (resident).
 void plan_xc_blocks(dfks_ctx* h, hipStream_t st) {
   const double tp0 = now_ms();
   const int64_t ng = h->ng;
   const int nao = h->nao;
   const Basis& O = h->orb;
   const int nsh = O.n();
-  const double* X = h->gxyz_host.data();
-  double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-  for (int64_t g = 0; g < ng; ++g)
-    for (int d = 0; d < 3; ++d) { lo[d] = std::min(lo[d], X[3 * g + d]); hi[d] = std::max(hi[d], X[3 * g + d]); }
-  // points in Morton order of their 30-bit keys: a stable LSD radix sort (three
-  // 10-bit passes), so equal keys keep the input order
-  std::vector<std::pair<uint32_t, int64_t>> key((size_t)ng), tmp((size_t)ng);
-  for (int64_t g = 0; g < ng; ++g) {
-    uint32_t c = 0;
-    for (int d = 0; d < 3; ++d) {
-      const double t = (X[3 * g + d] - lo[d]) / (hi[d] - lo[d] + 1e-12);
-      c |= spread3((uint32_t)std::min(1023.0, std::max(0.0, t * 1023.0))) << d;
-    }
-    key[g] = {c, g};
-  }
-  for (int pass = 0; pass < 3; ++pass) {
-    const int sh = 10 * pass;
-    std::vector<int64_t> cnt(1025, 0);
-    for (int64_t g = 0; g < ng; ++g) ++cnt[((key[g].first >> sh) & 1023u) + 1];
-    for (int b = 0; b < 1024; ++b) cnt[b + 1] += cnt[b];
-    for (int64_t g = 0; g < ng; ++g) tmp[cnt[(key[g].first >> sh) & 1023u]++] = key[g];
-    key.swap(tmp);
-  }
-  std::vector<std::pair<uint32_t, int64_t>>().swap(tmp);
-  const double tp1 = now_ms();
+  const ShellSet S = O.view();
+  if (ng > 0x7fffffff) fail(1, "compact XC grid: too many points");
   const int64_t nblk = (ng + kXcG - 1) / kXcG;
+  // buffers of the plan itself
+  std::vector<void*> tmp;
+  struct Free {
+    std::vector<void*>& p;
+    ~Free() { for (void* q : p) dfree(q); }
+  } fr{tmp};
+  const auto keep = [&](auto* p) { tmp.push_back(p); return p; };
+  const auto up = [&](const auto& v) {
+    using T = typename std::decay_t<decltype(v)>::value_type;
+    T* p = dalloc<T>(v.size());
+    HIPCHK(hipMemcpyAsync(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, st));
+    return p;
+  };
+  const double* d_X = keep(up(h->gxyz_host));
+  const double* d_gw = keep(up(h->gw_host));
+  // points in Morton order, then the shells of each block (xc_plan.hip)
+  double* sortw = keep(dalloc<double>((plan_sort_words(ng) + 1) / 2));
+  const int32_t* d_idx = nullptr;
+  HIPCHK(launch_plan_sort(ng, d_X, reinterpret_cast<uint32_t*>(sortw), &d_idx, st));
+  sync(st);
+  const double tp1 = now_ms();
   std::vector<double> rcut(nsh);
   for (int s = 0; s < nsh; ++s) rcut[s] = shell_radius(O, s);
-  std::vector<std::vector<int>> bsh((size_t)nblk);
+  const double* d_rcut = keep(up(rcut));
+  int32_t* d_loc = keep(dalloc<int32_t>(nblk * nsh));
+  int32_t* d_cnt = keep(dalloc<int32_t>(2 * nblk + nsh));   // functions and shells of a block, blocks of a shell
+  HIPCHK(hipMemsetAsync(d_cnt + 2 * nblk, 0, sizeof(int32_t) * nsh, st));
+  HIPCHK(launch_plan_scan(ng, d_X, d_idx, S, d_rcut, d_loc, d_cnt, d_cnt + nblk, d_cnt + 2 * nblk, st));
+  std::vector<int32_t> cnt((size_t)(2 * nblk + nsh));
+  HIPCHK(hipMemcpyAsync(cnt.data(), d_cnt, cnt.size() * sizeof(int32_t), hipMemcpyDeviceToHost, st));
+  sync(st);
   std::vector<int> npad((size_t)nblk);
-  // blocks are independent: host threads take interleaved blocks
-  auto scan_block = [&](int64_t b) {
-    const int64_t p0 = b * kXcG, p1 = std::min(ng, p0 + kXcG);
-    double c[3] = {0, 0, 0};
-    for (int64_t p = p0; p < p1; ++p)
-      for (int d = 0; d < 3; ++d) c[d] += X[3 * key[p].second + d];
-    for (int d = 0; d < 3; ++d) c[d] /= (double)(p1 - p0);
-    double rad = 0.0;
-    for (int64_t p = p0; p < p1; ++p) {
-      const double* x = X + 3 * key[p].second;
-      rad = std::max(rad, std::sqrt((x[0] - c[0]) * (x[0] - c[0]) + (x[1] - c[1]) * (x[1] - c[1]) +
-                                    (x[2] - c[2]) * (x[2] - c[2])));
-    }
-    int nb = 0;
-    for (int s = 0; s < nsh; ++s) {
-      if (rcut[s] < 0.0) continue;
-      const double* A = &O.centre[3 * s];
-      const double dist = std::sqrt((A[0] - c[0]) * (A[0] - c[0]) + (A[1] - c[1]) * (A[1] - c[1]) +
-                                    (A[2] - c[2]) * (A[2] - c[2]));
-      if (dist - rad <= rcut[s]) {
-        bsh[b].push_back(s);
-        nb += nfun(O.l[s], O.spherical);
-      }
-    }
-    npad[b] = std::max(32, (nb + 31) / 32 * 32);
-  };
-  {
-    // a few threads only: the process may run many builds at once (the serving loop) and
-    // share a CPU quota with the host runtime's own worker threads
-    const int nth = (int)std::max<int64_t>(1, std::min<int64_t>({(int64_t)std::thread::hardware_concurrency(), 4,
-                                                                   (nblk + 63) / 64}));
-    std::vector<std::thread> pool;
-    for (int t = 1; t < nth; ++t)
-      pool.emplace_back([&, t] { for (int64_t b = t; b < nblk; b += nth) scan_block(b); });
-    for (int64_t b = 0; b < nblk; b += nth) scan_block(b);
-    for (auto& th : pool) th.join();
-  }
+  for (int64_t b = 0; b < nblk; ++b) npad[b] = std::max(32, (cnt[b] + 31) / 32 * 32);
   const double tp2 = now_ms();
   // bins of equal padded width, blocks ordered by (width, position)
-  std::vector<int64_t> order((size_t)nblk);
-  for (int64_t b = 0; b < nblk; ++b) order[b] = b;
-  std::stable_sort(order.begin(), order.end(), [&](int64_t a, int64_t b) { return npad[a] < npad[b]; });
+  std::vector<int32_t> order((size_t)nblk);
+  for (int64_t b = 0; b < nblk; ++b) order[b] = (int32_t)b;
+  std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return npad[a] < npad[b]; });
   h->xbins.clear();
   int64_t ao_tot = 0, q_tot = 0, col_tot = 0, zw_max = 0;
   for (int64_t i = 0; i < nblk;) {
@@ -1012,75 +981,39 @@ void plan_xc_blocks(dfks_ctx* h, hipStream_t st) {
   h->xk_nblk = (int)xk.size();
   h->xk_nwg = (int)xw.size();
   const int64_t npts = nblk * kXcG;
-  std::vector<double> pts((size_t)(3 * npts)), w((size_t)npts, 0.0);
-  std::vector<int32_t> cols((size_t)col_tot, -1);
-  std::vector<int64_t> shoff((size_t)nblk + 1, 0);
-  std::vector<int2> shl;
-  for (const auto& bn : h->xbins) {
-    for (int64_t k = 0; k < bn.nblk; ++k) {
-      const int64_t ob = bn.blk0 + k;             // block in bin order
-      const int64_t b = order[ob];                // Morton block
-      const int64_t p0 = b * kXcG, p1 = std::min(ng, p0 + kXcG);
-      for (int64_t p = 0; p < kXcG; ++p) {
-        const int64_t src = key[std::min(p0 + p, p1 - 1)].second;
-        for (int d = 0; d < 3; ++d) pts[3 * (ob * kXcG + p) + d] = X[3 * src + d];
-        w[ob * kXcG + p] = p0 + p < p1 ? h->gw_host[src] : 0.0;
-      }
-      int col = 0;
-      int32_t* cb = cols.data() + bn.col_off + k * bn.n;
-      for (int s : bsh[b]) {
-        shl.push_back(make_int2(s, col));
-        const int nf = nfun(O.l[s], O.spherical);
-        for (int f = 0; f < nf; ++f) cb[col + f] = O.ao0[s] + f;
-        col += nf;
-      }
-      shoff[ob + 1] = (int64_t)shl.size();
-    }
-  }
-  // row lists of the Vxc assembly (CSR by AO row m): one entry per (block, local
-  // column i) with cols = m, in bin and block order -- a counting pass, then the fill
-  std::vector<int64_t> vrow((size_t)nao + 1, 0);
+  // per block of the plan: width, columns and products; shells before it; and the first entry of each AO row m
+  // in the lists of the Vxc assembly, one entry per (block, local column i) with cols = m, in plan order
+  std::vector<int32_t> width((size_t)nblk);
+  std::vector<int64_t> col0((size_t)nblk), q0((size_t)nblk), shoff((size_t)nblk + 1, 0);
   for (const auto& bn : h->xbins)
-    for (int64_t e = 0; e < bn.nblk * bn.n; ++e) {
-      const int32_t m = cols[bn.col_off + e];
-      if (m >= 0) ++vrow[m + 1];
+    for (int64_t k = 0; k < bn.nblk; ++k) {
+      const int64_t ob = bn.blk0 + k;
+      width[ob] = bn.n;
+      col0[ob] = bn.col_off + k * bn.n;
+      q0[ob] = bn.q_off + k * (int64_t)bn.n * bn.n;
+      shoff[ob + 1] = shoff[ob] + cnt[nblk + order[ob]];
     }
+  std::vector<int64_t> vrow((size_t)nao + 1, 0);
+  for (int s = 0; s < nsh; ++s)
+    for (int f = 0; f < nfun(O.l[s], O.spherical); ++f) vrow[O.ao0[s] + f + 1] = cnt[2 * nblk + s];
   for (int m = 0; m < nao; ++m) vrow[m + 1] += vrow[m];
-  const int64_t nent = vrow[nao];
-  std::vector<int64_t> vprow((size_t)std::max<int64_t>(nent, 1), 0), vpcol((size_t)std::max<int64_t>(nent, 1), 0);
-  std::vector<int32_t> vlen((size_t)std::max<int64_t>(nent, 1), 0);
-  {
-    std::vector<int64_t> fill(vrow.begin(), vrow.end() - 1);
-    for (const auto& bn : h->xbins)
-      for (int64_t k = 0; k < bn.nblk; ++k) {
-        const int64_t qb = bn.q_off + k * (int64_t)bn.n * bn.n, cbo = bn.col_off + k * bn.n;
-        for (int i = 0; i < bn.n; ++i) {
-          const int32_t m = cols[cbo + i];
-          if (m < 0) continue;
-          const int64_t e = fill[m]++;
-          vprow[e] = qb + (int64_t)i * bn.n;
-          vpcol[e] = cbo;
-          vlen[e] = bn.n;
-        }
-      }
-  }
+  const int64_t nent = std::max<int64_t>(vrow[nao], 1);
   const double tp3 = now_ms();
-  auto up = [&](auto& v) {
-    using T = typename std::decay_t<decltype(v)>::value_type;
-    T* p = dalloc<T>(v.size());
-    HIPCHK(hipMemcpyAsync(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, st));
-    return p;
-  };
-  h->d_xc_pts = up(pts);
-  h->d_xc_w = up(w);
-  h->d_xc_cols = up(cols);
+  const int32_t *d_order = keep(up(order)), *d_width = keep(up(width));
+  const int64_t *d_col0 = keep(up(col0)), *d_q0 = keep(up(q0));
+  h->d_xc_pts = dalloc<double>(3 * npts);
+  h->d_xc_w = dalloc<double>(npts);
+  h->d_xc_cols = dalloc<int32_t>(col_tot);
   h->d_xc_shoff = up(shoff);
-  if (shl.empty()) shl.push_back(make_int2(0, 0));
-  h->d_xc_shl = up(shl);
+  h->d_xc_shl = dalloc<int2>(std::max<int64_t>(shoff[nblk], 1));
   h->d_xc_vrow = up(vrow);
-  h->d_xc_vprow = up(vprow);
-  h->d_xc_vpcol = up(vpcol);
-  h->d_xc_vlen = up(vlen);
+  h->d_xc_vprow = dalloc<int64_t>(nent);
+  h->d_xc_vpcol = dalloc<int64_t>(nent);
+  h->d_xc_vlen = dalloc<int32_t>(nent);
+  HIPCHK(launch_plan_fill(ng, d_X, d_gw, d_idx, S, d_loc, d_order, d_width, d_col0, h->d_xc_shoff, h->d_xc_pts,
+                          h->d_xc_w, h->d_xc_cols, h->d_xc_shl, st));
+  HIPCHK(launch_plan_rows(nblk, S, d_loc, d_order, d_width, d_col0, d_q0, h->d_xc_vrow, h->d_xc_vprow, h->d_xc_vpcol,
+                          h->d_xc_vlen, st));
   h->xc_npts = npts;
   h->xc_nblk = nblk;
   h->xc_zw = zw_max;
@@ -1097,7 +1030,6 @@ void plan_xc_blocks(dfks_ctx* h, hipStream_t st) {
   h->d_xc_ao = dalloc<double>(ao_tot);
   const double tp4 = now_ms();
   HIPCHK(hipMemsetAsync(h->d_xc_ao, 0, sizeof(double) * ao_tot, st));
-  const ShellSet S = O.view();
   for (const auto& bn : h->xbins)
     HIPCHK(launch_ao_cmp((int)bn.nblk, kXcG, bn.n, h->d_xc_pts + 3 * bn.pt0, h->d_xc_shl, h->d_xc_shoff + bn.blk0, S,
                          h->d_xc_ao + bn.ao_off, st));

@@ -58,6 +58,7 @@ struct XcBlock {
   int32_t n, pad;
 };
 constexpr int kPanel = 32;            // pivoted Cholesky panel width
+constexpr int kXcG = 128;             // points per block of the compact XC grid
 constexpr int kLzSteps = 24;          // Lanczos steps for the SP2 spectral bounds
 constexpr int kLzParts = 4096;        // partial dot products of its matrix-vector kernel (n <= 4 kLzParts)
 

@@ -997,10 +997,11 @@ hipError_t launch_gemm_w8(const GemmArgs& g, double* C, const RowDot& rd, hipStr
 // of k_gemm_w8 pad: below about 64 columns the product is bound by reading A
 // once. K = 344, 40 columns ((H2O)_8 def2-TZVP): 0.26 ms = 3.4 TB/s, against
 // 0.53 (k_gemm), 0.60 (rocBLAS) and 0.65 ms; K = 1032, 48 columns: 5.2 against
-// 10.7 ms. At 120 columns rocBLAS is ahead (12.6 against 14.2 ms).
+// 10.7 ms. Up to 80 columns a wavefront takes 64 rows, beyond them 32, which is where the registers end (K =
+// 602, 70 columns: 1.73 ms with 64 rows, 1.88 with 32). At 120 columns rocBLAS is ahead (12.7 against 14.2 ms).
 template <int NJ>
 struct TTile {
-  static constexpr int MI = NJ <= 4 ? 4 : 2, ROWS = 64 * MI;   // 16-row blocks per wavefront, rows per workgroup
+  static constexpr int MI = NJ <= 5 ? 4 : 2, ROWS = 64 * MI;   // 16-row blocks per wavefront, rows per workgroup
 };
 
 template <int NJ>
@@ -1118,7 +1119,7 @@ __global__ __launch_bounds__(256, NJ <= 1 ? 4 : 2) void k_gemm_t(int64_t M, int 
 
 // C = A B^T (ldc = N) by k_gemm_t in equal column tiles of at most 160; A M-contiguous, B K-contiguous. rd.out
 // (optional): the row terms of gamma, for one column tile and rd.nq at least gemm_t_rows(N).
-int gemm_t_rows(int N) { return (N + 15) / 16 <= 4 ? TTile<4>::ROWS : TTile<5>::ROWS; }
+int gemm_t_rows(int N) { return (N + 15) / 16 <= 5 ? TTile<5>::ROWS : TTile<6>::ROWS; }
 
 hipError_t launch_gemm_t64(const GemmArgs& g, double* C, const RowDot& rd, hipStream_t st) {
   if (g.M <= 0 || g.N <= 0) return hipSuccess;

@@ -226,9 +226,10 @@ __global__ __launch_bounds__(64) void k_plan_scan(int64_t ng, const double* __re
 
 // Block ob of the plan (Morton block order[ob], width w[ob], columns from col0[ob]): points and weights (a short
 // block repeats its last point with weight 0), columns (-1 past the block's functions) and shell list
-__global__ __launch_bounds__(64) void k_plan_fill(int64_t ng, const double* __restrict__ X, const double* __restrict__ gw,
-                                                  const int32_t* __restrict__ idx, ShellSet S,
-                                                  const int32_t* __restrict__ loc, const int32_t* __restrict__ order,
+__global__ __launch_bounds__(64) void k_plan_fill(int64_t ng, const double* __restrict__ X,
+                                                  const double* __restrict__ gw, const int32_t* __restrict__ idx,
+                                                  ShellSet S, const int32_t* __restrict__ loc,
+                                                  const int32_t* __restrict__ order,
                                                   const int32_t* __restrict__ w, const int64_t* __restrict__ col0,
                                                   const int64_t* __restrict__ shoff, double* __restrict__ pts,
                                                   double* __restrict__ wts, int32_t* __restrict__ cols,

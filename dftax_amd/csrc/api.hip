@@ -175,6 +175,7 @@ hipError_t launch_plan_fill(int64_t ng, const double* X, const double* gw, const
 hipError_t launch_plan_rows(int64_t nblk, const ShellSet& S, const int32_t* loc, const int32_t* order, const int32_t* w,
                             const int64_t* col0, const int64_t* q0, const int64_t* vrow, int64_t* vprow, int64_t* vpcol,
                             int32_t* vlen, hipStream_t st);
+hipError_t launch_dots(const DotList& d, double* part, double* E, hipStream_t st);
 hipError_t launch_lanczos(int n, const double* F, double* lz, hipStream_t s);
 int metric_ld(int n);
 size_t metric_chol_words(int n);
@@ -1092,7 +1093,7 @@ void build_all(dfks_ctx* h, hipStream_t st) {
     HIPCHK(hipMemcpyAsync(h->d_gxyz, h->gxyz_host.data(), 3 * h->ng * sizeof(double), hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(h->d_gw, h->gw_host.data(), h->ng * sizeof(double), hipMemcpyHostToDevice, st));
   }
-  h->d_part = dalloc<double>(1024);
+  h->d_part = dalloc<double>(kDotList * 512);
   h->d_Edev = dalloc<double>(8);
   h->d_info = dalloc<int32_t>(1);
   const int nao = h->nao, naux = h->naux;
@@ -2052,22 +2053,21 @@ void energy_fock_factored(dfks_ctx* h, const double* P, const double* Cf, const 
   if (h->mixed_now && h->opt.precision != 1) fail(1, "mixed precision needs options.precision = 1 at create");
   h->mark(0, st);
   HIPCHK(hipMemsetAsync(E, 0, 8 * sizeof(double), st));
-  // one-electron energy
-  HIPCHK(launch_dot(nn, P, h->d_H, h->d_part, 1.0, E + DFKS_E_ONE, 0, st));
   jk_factored(h, Cf, sgn, nf, st);
   if (h->hf_lr != 0.0) k_lr_factored(h, Cf, sgn, nf, st);
-  // E_J = 1/2 |gamma|^2
-  HIPCHK(launch_dot(nfit, h->d_gamma, h->d_gamma, h->d_part, 0.5, E + DFKS_E_J, 0, st));
-  // E_K = -1/4 sum P o (a_x K + a_lr K_lr) (E was cleared above)
-  if (h->hf != 0.0) HIPCHK(launch_dot(nn, P, h->d_K, h->d_part, -0.25 * h->hf, E + DFKS_E_K, 1, st));
-  if (h->hf_lr != 0.0) HIPCHK(launch_dot(nn, P, h->d_Klr, h->d_part, -0.25 * h->hf_lr, E + DFKS_E_K, 1, st));
   xc_potential(h, P, E, st);
   HIPCHK(launch_fock(nao, h->d_H, h->d_J, h->hf != 0.0 ? h->d_K : nullptr, -0.5 * h->hf,
                      ng > 0 ? h->d_Vxc : nullptr, F, st));
   if (h->hf_lr != 0.0) HIPCHK(launch_axpy(nn, -0.5 * h->hf_lr, h->d_Klr, F, 1, st));
-  // totals: E_tot = e1 + eJ + eK + exc + enn
+  // one-electron energy, E_J = 1/2 |gamma|^2, E_K = -1/4 sum P o (a_x K + a_lr K_lr) (E was cleared above), and
+  // E_tot = e1 + eJ + eK + exc + enn
   HIPCHK(hipMemcpyAsync(E + DFKS_E_NN, &h->e_nn, sizeof(double), hipMemcpyHostToDevice, st));
-  HIPCHK(launch_dot(5, E + 1, nullptr, h->d_part, 1.0, E + DFKS_E_TOT, 0, st));
+  DotList d;
+  d.push(nn, P, h->d_H, 1.0, E + DFKS_E_ONE, 0);
+  d.push(nfit, h->d_gamma, h->d_gamma, 0.5, E + DFKS_E_J, 0);
+  if (h->hf != 0.0) d.push(nn, P, h->d_K, -0.25 * h->hf, E + DFKS_E_K, 1);
+  if (h->hf_lr != 0.0) d.push(nn, P, h->d_Klr, -0.25 * h->hf_lr, E + DFKS_E_K, 1);
+  HIPCHK(launch_dots(d, h->d_part, E, st));
   h->mark(kStFock + 1, st);
 }
 
@@ -2986,8 +2986,11 @@ void scf_step(dfks_ctx* h, double* out3, hipStream_t st) {
     gemm(h, false, false, nmo, nmo, nao, 1.0, h->d_W2, nmo, h->d_X, nao, 0.0, err, nmo);
   }
   // DIIS history
-  for (int i = 0; i < count; ++i)
-    HIPCHK(launch_dot(mm, err, h->d_Es + i * mm, h->d_part, 1.0, h->d_dots + i, 0, st));
+  for (int i = 0; i < count; i += kDotList) {
+    DotList d;
+    for (int k = i; k < std::min(count, i + kDotList); ++k) d.push(mm, err, h->d_Es + k * mm, 1.0, h->d_dots + k, 0);
+    HIPCHK(launch_dots(d, h->d_part, nullptr, st));
+  }
   HIPCHK(launch_gram_update(m, slot, count, h->d_dots, h->d_gram, st));
   HIPCHK(launch_diis_solve(m, count, h->d_gram, h->d_coef, st));
   HIPCHK(launch_diis_extrap(m, mm, h->d_coef, h->d_Fs, h->d_Ws, st));

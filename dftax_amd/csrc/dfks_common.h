@@ -58,6 +58,20 @@ struct XcBlock {
   int32_t n, pad;
 };
 constexpr int kPanel = 32;            // pivoted Cholesky panel width
+// out[k] = scale[k] sum x[k] y[k] (+= with add), k < count
+constexpr int kDotList = 8;
+struct DotList {
+  int count = 0;
+  int64_t n[kDotList];
+  const double *x[kDotList], *y[kDotList];
+  double scale[kDotList];
+  double* out[kDotList];
+  int add[kDotList];
+  void push(int64_t n_, const double* x_, const double* y_, double scale_, double* out_, int add_) {
+    n[count] = n_, x[count] = x_, y[count] = y_, scale[count] = scale_, out[count] = out_, add[count] = add_;
+    ++count;
+  }
+};
 constexpr int kXcG = 128;             // points per block of the compact XC grid
 constexpr int kLzSteps = 24;          // Lanczos steps for the SP2 spectral bounds
 constexpr int kLzParts = 4096;        // partial dot products of its matrix-vector kernel (n <= 4 kLzParts)

@@ -8,6 +8,7 @@
 //  * deterministic two-pass reductions for the energy terms
 //  * DIIS: Gram row, bordered solve (one lane, FP64, partial pivoting),
 //    extrapolation (dftax/ks/scf.py:252-276)
+#include <algorithm>
 #include <cstdint>
 
 #include "dfks_common.h"
@@ -15,6 +16,10 @@
 namespace dfks {
 
 constexpr int kRedBlocks = 512;
+__host__ __device__ inline int64_t dot_blocks(int64_t n) {
+  const int64_t nb = (n + 255) / 256;
+  return nb > kRedBlocks ? kRedBlocks : nb < 1 ? 1 : nb;
+}
 
 // partial[b] = sum over a grid-stride slice of x[i]*y[i] (y may be null -> x only)
 __global__ __launch_bounds__(256) void k_dot_partial(int64_t n, const double* __restrict__ x,
@@ -49,11 +54,58 @@ __global__ __launch_bounds__(256) void k_sum_final(int np, const double* __restr
 
 hipError_t launch_dot(int64_t n, const double* x, const double* y, double* part, double scale, double* out,
                       int accumulate, hipStream_t st) {
-  int nb = (int)((n + 255) / 256);
-  if (nb > kRedBlocks) nb = kRedBlocks;
-  if (nb < 1) nb = 1;
+  const int nb = (int)dot_blocks(n);
   hipLaunchKernelGGL(k_dot_partial, dim3(nb), dim3(256), 0, st, n, x, y, part);
   hipLaunchKernelGGL(k_sum_final, dim3(1), dim3(256), 0, st, nb, part, scale, out, accumulate);
+  return hipGetLastError();
+}
+
+// Several dots in two launches, each summed as launch_dot sums it: an SCF step takes about a dozen, and a
+// launch costs more than the sum it makes (344 functions: 3.5 us each).
+__global__ __launch_bounds__(256) void k_dots_partial(DotList d, double* __restrict__ part) {
+  __shared__ double s[256];
+  const int k = blockIdx.y;
+  const double *x = d.x[k], *y = d.y[k];
+  double acc = 0.0;
+  const int64_t n = d.n[k], nb = dot_blocks(n);
+  if (blockIdx.x >= nb) return;
+  for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < n; i += nb * 256) acc += x[i] * y[i];
+  s[threadIdx.x] = acc;
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if (threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) part[k * kRedBlocks + blockIdx.x] = s[0];
+}
+
+__global__ __launch_bounds__(256) void k_dots_final(DotList d, const double* __restrict__ part, double* __restrict__ E) {
+  __shared__ double s[256];
+  for (int k = 0; k < d.count; ++k) {
+    const int np = (int)dot_blocks(d.n[k]);
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < np; i += 256) acc += part[k * kRedBlocks + i];
+    __syncthreads();
+    s[threadIdx.x] = acc;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+      if (threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) d.out[k][0] = d.add[k] ? d.out[k][0] + d.scale[k] * s[0] : d.scale[k] * s[0];
+  }
+  // the five terms of an energy, in the order of launch_dot's tree
+  if (E && threadIdx.x == 0) E[0] = ((E[1] + E[5]) + E[3]) + (E[2] + E[4]);
+}
+
+// The list's dots (part: kDotList * 512 words); E (optional): then E[0] = E[1] + .. + E[5]
+hipError_t launch_dots(const DotList& d, double* part, double* E, hipStream_t st) {
+  if (d.count == 0 && !E) return hipSuccess;
+  int64_t nb = 1;
+  for (int k = 0; k < d.count; ++k) nb = std::max(nb, dot_blocks(d.n[k]));
+  if (d.count > 0)
+    hipLaunchKernelGGL(k_dots_partial, dim3((unsigned)nb, (unsigned)d.count), dim3(256), 0, st, d, part);
+  hipLaunchKernelGGL(k_dots_final, dim3(1), dim3(256), 0, st, d, part, E);
   return hipGetLastError();
 }
 

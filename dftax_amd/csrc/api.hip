@@ -664,6 +664,7 @@ struct dfks_ctx {
   // recompute mode (options.aux_chunk > 0): screened bra pairs per (la, lb)
   // class, auxiliary slabs with per-lc shell lists, slab and exchange buffers
   bool recompute = false;
+  bool lt_tri = false;   // d_Lt[P][Q] = 0 for P > Q (inverse Cholesky factor)
   bool slab_zero = false;   // screened pairs leave holes: clear a slab before filling it
   int2* d_pairs3 = nullptr;
   std::vector<size_t> pair3_off;
@@ -1310,6 +1311,7 @@ void build_all(dfks_ctx* h, hipStream_t st) {
   // the metric factor from the side stream, then B
   eig.finish();
   double* d_Lt = nullptr;
+  h->lt_tri = eig.chol;
   if (eig.chol) {
     d_Lt = d_Lc;
     d_Lc = nullptr;
@@ -1511,9 +1513,17 @@ void exchange_recompute(dfks_ctx* h, const double* Cf, const float* Cf32, int nc
     HIPCHK(hipMemcpy2DAsync(h->d_Ttil + (size_t)h->slab_p0[s] * nc, sizeof(double) * naux * nc, h->d_Tslab,
                             sizeof(double) * np * nc, sizeof(double) * np * nc, nao, hipMemcpyDeviceToDevice, st));
   }
-  RBCHK(rocblas_dgemm_strided_batched(h->rb, rocblas_operation_none, rocblas_operation_transpose, nc, nfit, naux, &one,
-                                      h->d_Ttil, nc, (rocblas_stride)naux * nc, h->d_Lt, nfit, 0, &zero, h->d_Tx, nc,
-                                      (rocblas_stride)nfit * nc, nao));
+  // T_m[Q][i] = sum_P L[P,Q] T~_m[P][i]; an inverse Cholesky factor has nothing past P = Q: four strips of Q, each
+  // with the P up to its last Q ((H2O)_12 def2-TZVP: 27.9 ms a build of F, 29.6 in one piece)
+  const int parts = h->lt_tri ? 4 : 1;
+  for (int k = 0; k < parts; ++k) {
+    const int q0 = (int)((int64_t)nfit * k / parts), q1 = (int)((int64_t)nfit * (k + 1) / parts);
+    if (q1 == q0) continue;
+    RBCHK(rocblas_dgemm_strided_batched(h->rb, rocblas_operation_none, rocblas_operation_transpose, nc, q1 - q0,
+                                        h->lt_tri ? q1 : naux, &one, h->d_Ttil, nc, (rocblas_stride)naux * nc,
+                                        h->d_Lt + q0, nfit, 0, &zero, h->d_Tx + (size_t)q0 * nc, nc,
+                                        (rocblas_stride)nfit * nc, nao));
+  }
 }
 
 // J = sum_P (mn|P) d_P with d = L gamma, slab by slab.

@@ -11,7 +11,7 @@
 // the blocks of every width spread over the XCDs. Blocks come widest first.
 //
 // (H2O)_24 def2-TZVP on the MI355X: rho 5.3 ms, the pointwise pass 0.2 ms, Vh
-// 3.9 ms, against 14 ms for the per-bin gathers, batched products and
+// 3.85 ms, against 14 ms for the per-bin gathers, batched products and
 // wavefront-per-point kernels they replace. Vh is near what its AO rows read
 // and products written take at the copy rate (3 ms); rho is between its reads
 // (1.7 ms) and its matrix work (2.8 ms). An MFMA sums over any order of k as
@@ -216,7 +216,7 @@ __device__ __forceinline__ void v_strip(const XcBlock& b, int c0, const double* 
   }
 }
 
-__global__ __launch_bounds__(256) void k_xcb_v(const XcBlock* __restrict__ blks, const int32_t* __restrict__ wgs,
+__global__ __launch_bounds__(256, 2) void k_xcb_v(const XcBlock* __restrict__ blks, const int32_t* __restrict__ wgs,
                                                const double* __restrict__ ao, const double* __restrict__ coef,
                                                double* __restrict__ q) {
   __shared__ __attribute__((aligned(16))) double s_w[kG * 64];

@@ -176,6 +176,8 @@ hipError_t launch_plan_rows(int64_t nblk, const ShellSet& S, const int32_t* loc,
                             const int64_t* col0, const int64_t* q0, const int64_t* vrow, int64_t* vprow, int64_t* vpcol,
                             int32_t* vlen, hipStream_t st);
 hipError_t launch_dots(const DotList& d, double* part, double* E, hipStream_t st);
+hipError_t launch_gemm_small(bool ta, bool tb, int M, int N, int K, double alpha, const double* A, int64_t lda,
+                             const double* B, int64_t ldb, double beta, double* C, int64_t ldc, hipStream_t st);
 hipError_t launch_lanczos(int n, const double* F, double* lz, hipStream_t s);
 int metric_ld(int n);
 size_t metric_chol_words(int n);
@@ -2202,6 +2204,16 @@ void energy_fock_general(dfks_ctx* h, const double* P, double* E, double* F, hip
 // ---------------------------------------------------------------------------
 void gemm(dfks_ctx* h, bool ta, bool tb, int64_t m, int64_t n, int64_t k, double alpha, const double* A, int64_t lda,
           const double* B, int64_t ldb, double beta, double* C, int64_t ldc) {
+  // Up to 600 tiles of 32 x 32 the library's tiles leave compute units idle (us, k_gemm_s against rocBLAS): 344 cubed
+  // 7 against 13 to 23, 602 cubed 12 to 15 against 23 to 31, 1032 x 120 x 1032 15 against 24; beyond, rocBLAS is
+  // ahead (1032 cubed, 1089 tiles: 65 against 54)
+  if (h->opt.gemm != 1 && !(ta && tb) && m > 0 && n > 0 && k > 0 && k <= 2048 &&
+      (m + 31) / 32 * ((n + 31) / 32) <= 600) {
+    hipStream_t st = nullptr;
+    RBCHK(rocblas_get_stream(h->rb, &st));
+    HIPCHK(launch_gemm_small(ta, tb, (int)m, (int)n, (int)k, alpha, A, lda, B, ldb, beta, C, ldc, st));
+    return;
+  }
   RBCHK(rocblas_dgemm_64(h->rb, ta ? rocblas_operation_transpose : rocblas_operation_none,
                          tb ? rocblas_operation_transpose : rocblas_operation_none, m, n, k, &alpha, A, lda, B, ldb,
                          &beta, C, ldc));

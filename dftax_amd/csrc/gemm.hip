@@ -950,6 +950,143 @@ static hipError_t launch_nt_partials(const GemmArgs& g, double* ws, int nsplit, 
                   (int64_t)g.M * g.N, kchunk, nsplit, (int)ntl, sym & 1);
 }
 
+// C = alpha op(A) op(B) + beta C (column-major) for the SCF step's products of a few hundred to about a thousand
+// functions. 32 x 32 a workgroup, its four wavefronts a quarter of k each, summed in LDS in their order: at 344
+// functions that is 121 workgroups, where 128-wide tiles leave most of the chip idle. Fragments of 8 k come straight
+// from global memory, two words a load: of two rows where the operand's rows are contiguous (tile e has the rows
+// 2 li + e), of two k where its k are (k = 2 lk + s in step s). Bound by the chain of loads and products of a
+// quarter of k. 602 cubed 12 us (rocBLAS 23 to 31); where it stops being ahead is at its caller.
+template <bool KC>
+struct SmallOperand {
+  const double* p[2];   // row (pair) pointers at k = 0
+  int64_t ld;
+  int last;             // rows past the end repeat the last
+  bool full;
+  // rows r0 .. r0 + 31 of a matrix of n rows
+  __device__ __forceinline__ void init(const double* A, int64_t ld_, int r0, int n) {
+    const int li = threadIdx.x & 15;
+    ld = ld_;
+    if constexpr (KC) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) p[e] = A + (int64_t)min(r0 + 16 * e + li, n - 1) * ld;
+    } else {
+      full = r0 + 32 <= n;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) p[e] = A + min(r0 + 2 * li + e, n - 1);
+    }
+  }
+  // x[e][s]: tile e, k = k0 + 2 lk + s (k past K: any element)
+  __device__ __forceinline__ void load(int k0, int K, double (&x)[2][2]) const {
+    const int k = k0 + 2 * ((threadIdx.x & 63) >> 4);
+    if constexpr (KC) {
+      if (k0 + 8 <= K) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const dbl2u v = *reinterpret_cast<const dbl2u*>(p[e] + k);
+          x[e][0] = v[0];
+          x[e][1] = v[1];
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+          for (int s = 0; s < 2; ++s) x[e][s] = p[e][min(k + s, K - 1)];
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int64_t o = (int64_t)min(k + s, K - 1) * ld;
+        if (full) {
+          const dbl2u v = *reinterpret_cast<const dbl2u*>(p[0] + o);
+          x[0][s] = v[0];
+          x[1][s] = v[1];
+        } else {
+          x[0][s] = p[0][o];
+          x[1][s] = p[1][o];
+        }
+      }
+    }
+  }
+  // the operand's row of tile e, row r
+  static __device__ __forceinline__ int row(int e, int r) { return KC ? 16 * e + r : 2 * r + e; }
+};
+
+template <bool TA, bool TB>
+__global__ __launch_bounds__(256, 2) void k_gemm_s(int M, int N, int K, double alpha, const double* __restrict__ A,
+                                                int64_t lda, const double* __restrict__ B, int64_t ldb, double beta,
+                                                double* __restrict__ C, int64_t ldc) {
+  __shared__ double s_acc[4][4][4][64];   // wavefront, tile, register, lane
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int li = lane & 15, lk = lane >> 4;
+  const int m0 = 32 * (int)blockIdx.x, n0 = 32 * (int)blockIdx.y;
+  SmallOperand<TA> a;
+  SmallOperand<!TB> b;
+  a.init(A, lda, m0, M);
+  b.init(B, ldb, n0, N);
+  const int groups = (K + 7) / 8, g0 = groups * wave / 4, g1 = groups * (wave + 1) / 4;
+  dbl4 acc[2][2] = {};
+  double x[2][2][2], y[2][2][2];
+  const auto mul = [&](int k0, double (&u)[2][2], double (&v)[2][2]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const bool in = k0 + 2 * lk + s < K;
+      const double u0 = in ? u[0][s] : 0.0, u1 = in ? u[1][s] : 0.0;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        acc[0][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(u0, v[j][s], acc[0][j], 0, 0, 0);
+        acc[1][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(u1, v[j][s], acc[1][j], 0, 0, 0);
+      }
+    }
+  };
+  if (g0 < g1) {
+    a.load(8 * g0, K, x[0]);
+    b.load(8 * g0, K, y[0]);
+    int g = g0;
+    for (; g + 2 <= g1; g += 2) {
+      a.load(8 * (g + 1), K, x[1]);
+      b.load(8 * (g + 1), K, y[1]);
+      mul(8 * g, x[0], y[0]);
+      const int gn = min(g + 2, g1 - 1);
+      a.load(8 * gn, K, x[0]);
+      b.load(8 * gn, K, y[0]);
+      mul(8 * (g + 1), x[1], y[1]);
+    }
+    if (g < g1) mul(8 * g, x[0], y[0]);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s_acc[wave][2 * i + j][r][lane] = acc[i][j][r];
+  __syncthreads();
+  // wavefront t sums and stores tile t: register r is row lk + 4 r of the A tile, column li of the B tile
+  const int ti = wave >> 1, tj = wave & 1;
+  const int gn = n0 + SmallOperand<!TB>::row(tj, li);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int gm = m0 + SmallOperand<TA>::row(ti, lk + 4 * r);
+    if (gm >= M || gn >= N) continue;
+    const double v = ((s_acc[0][wave][r][lane] + s_acc[1][wave][r][lane]) + s_acc[2][wave][r][lane]) +
+                     s_acc[3][wave][r][lane];
+    double* c = C + gm + (int64_t)gn * ldc;
+    *c = beta != 0.0 ? alpha * v + beta * *c : alpha * v;
+  }
+}
+
+// C = alpha op(A) op(B) + beta C by k_gemm_s (column-major), at most one operand transposed
+hipError_t launch_gemm_small(bool ta, bool tb, int M, int N, int K, double alpha, const double* A, int64_t lda,
+                             const double* B, int64_t ldb, double beta, double* C, int64_t ldc, hipStream_t st) {
+  if (M <= 0 || N <= 0) return hipSuccess;
+  if (K <= 0 || (ta && tb)) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)((M + 31) / 32), (unsigned)((N + 31) / 32));
+  const auto run = [&](auto kern) {
+    return launch_k(kern, grid, dim3(256), st, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
+  };
+  if (ta) return run(k_gemm_s<true, false>);
+  return tb ? run(k_gemm_s<false, true>) : run(k_gemm_s<false, false>);
+}
+
 // k_gemm_w8 launch: ldc, split and symmetric mode as launch_gemm_t (NJ = 5
 // only without the symmetric mode); B must be K-contiguous.
 template <int NJ>

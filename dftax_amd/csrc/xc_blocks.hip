@@ -10,7 +10,7 @@
 // block are 8 ids apart, so they share that XCD's L2 for the block's AO rows and
 // the blocks of every width spread over the XCDs. Blocks come widest first.
 //
-// (H2O)_24 def2-TZVP on the MI355X: rho 5.3 ms, the pointwise pass 0.2 ms, Vh
+// (H2O)_24 def2-TZVP on the MI355X: rho 4.0 ms, the pointwise pass 0.2 ms, Vh
 // 3.85 ms, against 14 ms for the per-bin gathers, batched products and
 // wavefront-per-point kernels they replace. Vh is near what its AO rows read
 // and products written take at the copy rate (3 ms); rho is between its reads

@@ -91,7 +91,7 @@ hipError_t launch_axpy(int64_t n, double a, const double* x, double* y, int acc,
 hipError_t launch_antisym(int n, const double* A, double* E, hipStream_t st);
 hipError_t launch_eye_dev(int n, const double* G, double* out, hipStream_t st);
 hipError_t launch_store2(double* dst, double a, double b, hipStream_t st);
-hipError_t launch_diis_solve(int m, int count, const double* gram, double* coef, hipStream_t st);
+hipError_t launch_diis_solve(int m, int count, int newest, const double* gram, double* coef, hipStream_t st);
 hipError_t launch_diis_extrap(int m, int64_t n, const double* coef, const double* Fs, double* out, hipStream_t st);
 hipError_t launch_gram_update(int m, int slot, int count, const double* dots, double* gram, hipStream_t st);
 hipError_t launch_scaled_cols(int n, int k0, const double* U, const double* w, double* X, hipStream_t st);
@@ -3014,7 +3014,8 @@ void scf_step(dfks_ctx* h, double* out3, hipStream_t st) {
     HIPCHK(launch_dots(d, h->d_part, nullptr, st));
   }
   HIPCHK(launch_gram_update(m, slot, count, h->d_dots, h->d_gram, st));
-  HIPCHK(launch_diis_solve(m, count, h->d_gram, h->d_coef, st));
+  // the FP64 steps after a mixed phase scale the ridge; an FP64 handle's steps are the reference's, fixed ridge and all
+  HIPCHK(launch_diis_solve(m, count, h->opt.precision == 1 && !h->mixed_now ? slot : -1, h->d_gram, h->d_coef, st));
   HIPCHK(launch_diis_extrap(m, mm, h->d_coef, h->d_Fs, h->d_Ws, st));
   if (h->level_shift != 0.0) {
     // F' += b X^T (S - 1/2 S P S) X (the AO term in d_Fx)

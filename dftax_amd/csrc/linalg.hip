@@ -79,7 +79,8 @@ __global__ __launch_bounds__(256) void k_dots_partial(DotList d, double* __restr
   if (threadIdx.x == 0) part[k * kRedBlocks + blockIdx.x] = s[0];
 }
 
-__global__ __launch_bounds__(256) void k_dots_final(DotList d, const double* __restrict__ part, double* __restrict__ E) {
+__global__ __launch_bounds__(256) void k_dots_final(DotList d, const double* __restrict__ part,
+                                                    double* __restrict__ E) {
   __shared__ double s[256];
   for (int k = 0; k < d.count; ++k) {
     const int np = (int)dot_blocks(d.n[k]);
@@ -459,14 +460,19 @@ hipError_t launch_antisym(int n, const double* A, double* E, hipStream_t st) {
 // Builds A, solves A c = (0,..,0,-1) by Gaussian elimination with partial pivoting
 // on one lane and writes c[0..m). Mirrors dftax/ks/scf.py:252-276 (identity on
 // empty slots, 1e-10 ridge on filled ones).
-// DIIS coefficients from the bordered system [[G + 1e-10 I, -1], [-1^T, 0]] c = [0, -1]
+// DIIS coefficients from the bordered system [[G + r I, -1], [-1^T, 0]] c = [0, -1], r = 1e-10
 // (unused slots become identity rows with c = 0), by Gaussian elimination with
 // partial pivoting. One wavefront: lane i holds row i (m + 1 <= 17 rows, 18
 // columns with the right-hand side) in registers; pivot search, row swap and the
 // pivot row go through shuffles. The pivot (first largest |a_ik|), the updates
 // and the back substitution run in the same order as a serial elimination.
-__global__ __launch_bounds__(64) void k_diis_solve(int m, int count, const double* __restrict__ gram,
+// newest >= 0 (the FP64 steps after a mixed phase): r is at most 1e-6 of the newest error's square, and at least
+// 1e-22. Once errors are under 1e-5 a fixed 1e-10 outweighs G and the coefficients turn into a plain average of the
+// history: (H2O)_14 took 33 to 42 steps to 1e-8, about 20 of them under 1e-6, and takes 18 or 19. The split-BF16 steps
+// keep 1e-10, which stands at the square of their noise.
+__global__ __launch_bounds__(64) void k_diis_solve(int m, int count, int newest, const double* __restrict__ gram,
                                                    double* __restrict__ coef) {
+  const double ridge = newest >= 0 ? fmax(fmin(1e-10, 1e-6 * gram[newest * m + newest]), 1e-22) : 1e-10;
   constexpr int kR = 17, kC = 18;
   const int lane = threadIdx.x;
   const int n = m + 1;
@@ -478,7 +484,7 @@ __global__ __launch_bounds__(64) void k_diis_solve(int m, int count, const doubl
       if (j < m) {
         const bool vi = lane < count, vj = j < count;
         v = (vi && vj) ? gram[lane * m + j] : (lane == j ? 1.0 : 0.0);
-        if (lane == j && vi) v += 1e-10;
+        if (lane == j && vi) v += ridge;
       } else if (j == m) {
         v = lane < count ? -1.0 : 0.0;
       }
@@ -554,8 +560,8 @@ __global__ __launch_bounds__(64) void k_diis_solve(int m, int count, const doubl
   }
 }
 
-hipError_t launch_diis_solve(int m, int count, const double* gram, double* coef, hipStream_t st) {
-  hipLaunchKernelGGL(k_diis_solve, dim3(1), dim3(64), 0, st, m, count, gram, coef);
+hipError_t launch_diis_solve(int m, int count, int newest, const double* gram, double* coef, hipStream_t st) {
+  hipLaunchKernelGGL(k_diis_solve, dim3(1), dim3(64), 0, st, m, count, newest, gram, coef);
   return hipGetLastError();
 }
 

@@ -79,8 +79,9 @@ __global__ __launch_bounds__(256) void k_dots_partial(DotList d, double* __restr
   if (threadIdx.x == 0) part[k * kRedBlocks + blockIdx.x] = s[0];
 }
 
+// E holds some of the list's results, so it may not be restrict: its terms are read after they are stored.
 __global__ __launch_bounds__(256) void k_dots_final(DotList d, const double* __restrict__ part,
-                                                    double* __restrict__ E) {
+                                                    double* E) {
   __shared__ double s[256];
   for (int k = 0; k < d.count; ++k) {
     const int np = (int)dot_blocks(d.n[k]);

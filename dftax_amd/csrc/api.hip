@@ -3014,8 +3014,10 @@ void scf_step(dfks_ctx* h, double* out3, hipStream_t st) {
     HIPCHK(launch_dots(d, h->d_part, nullptr, st));
   }
   HIPCHK(launch_gram_update(m, slot, count, h->d_dots, h->d_gram, st));
-  // the FP64 steps after a mixed phase scale the ridge; an FP64 handle's steps are the reference's, fixed ridge and all
-  HIPCHK(launch_diis_solve(m, count, h->opt.precision == 1 && !h->mixed_now ? slot : -1, h->d_gram, h->d_coef, st));
+  // the ridge is scaled where the history holds the FP64 steps after a mixed phase alone (diis_base > 0); every other
+  // step is the reference's, fixed ridge and all, also an FP64 step of a handle with 32-bit products
+  const bool after_mixed = h->diis_base > 0 && !h->restart_diis && !h->mixed_now;
+  HIPCHK(launch_diis_solve(m, count, after_mixed ? slot : -1, h->d_gram, h->d_coef, st));
   HIPCHK(launch_diis_extrap(m, mm, h->d_coef, h->d_Fs, h->d_Ws, st));
   if (h->level_shift != 0.0) {
     // F' += b X^T (S - 1/2 S P S) X (the AO term in d_Fx)

@@ -467,10 +467,11 @@ hipError_t launch_antisym(int n, const double* A, double* E, hipStream_t st) {
 // columns with the right-hand side) in registers; pivot search, row swap and the
 // pivot row go through shuffles. The pivot (first largest |a_ik|), the updates
 // and the back substitution run in the same order as a serial elimination.
-// newest >= 0 (the FP64 steps after a mixed phase): r is at most 1e-6 of the newest error's square, and at least
-// 1e-22. Once errors are under 1e-5 a fixed 1e-10 outweighs G and the coefficients turn into a plain average of the
-// history: (H2O)_14 took 33 to 42 steps to 1e-8, about 20 of them under 1e-6, and takes 18 or 19. The split-BF16 steps
-// keep 1e-10, which stands at the square of their noise.
+// newest >= 0 (the history holds FP64 steps that follow a mixed phase, and no others): r is at most 1e-6 of the newest
+// error's square, and at least 1e-22. Once errors are under 1e-5 a fixed 1e-10 outweighs G and the coefficients turn
+// into a plain average of the history: (H2O)_14 took 33 to 42 steps to 1e-8, about 20 of them under 1e-6, and takes 18
+// or 19. The split-BF16 steps, and the one that still extrapolates over them, keep 1e-10, which stands at the square of
+// their noise.
 __global__ __launch_bounds__(64) void k_diis_solve(int m, int count, int newest, const double* __restrict__ gram,
                                                    double* __restrict__ coef) {
   const double ridge = newest >= 0 ? fmax(fmin(1e-10, 1e-6 * gram[newest * m + newest]), 1e-22) : 1e-10;

@@ -17,3 +17,18 @@ def test_tight_convergence(name):
     assert got[1].n_iter <= 40
     assert abs(got[0].e_tot - got[1].e_tot) < 1e-10
     assert float((got[0].P - got[1].P).abs().max()) < 1e-8
+
+
+@pytest.mark.parametrize("name", ["water_svp", "water2_tzvp"])
+def test_no_mixed_phase(name):
+    """FP64 steps alone on a handle with 32-bit products follow an FP64 handle's: the two differ by the rounding of the
+    metric's factor (1e-10 of F), which the errors down to 1e-6 carry as 1e-4 of themselves at the most."""
+    from dftax_amd import KS, Molecule, WATER, becke, df, hip, scf, water_cluster
+    mol = (Molecule.from_xyz(WATER, "def2-svp", spherical=True) if name == "water_svp" else
+           water_cluster((2, 1, 1), seed=1, basis="def2-tzvp"))
+    a, b = (scf(KS(mol, "PBE0", grid=becke(30, 110), coulomb=df(engine=hip(precision=p))), precision="fp64",
+                e_tol=1e-9, d_tol=1e-6).history for p in ("fp64", "mixed"))
+    errors = [(x[2], y[2]) for x, y in zip(a, b) if x[2] > 1e-6]
+    assert errors[-1][0] < 1e-5
+    for x, y in errors:
+        assert abs(y - x) < 1e-3 * x

@@ -87,6 +87,8 @@ hipError_t launch_symfill(int n, double* A, hipStream_t st);
 hipError_t launch_metric_factor(int nq, int k0, const double* U, const double* w, double* Lt, hipStream_t st);
 hipError_t launch_factor_cols(int n, int nf, const double* V, const double* lam, const int32_t* sel, double* Cf,
                               double* sgn, hipStream_t st);
+hipError_t launch_gather_fun(int64_t nrow, int n, int rows_too, const int32_t* fun, const double* in, double* out,
+                             hipStream_t st);
 hipError_t launch_axpy(int64_t n, double a, const double* x, double* y, int acc, hipStream_t st);
 hipError_t launch_antisym(int n, const double* A, double* E, hipStream_t st);
 hipError_t launch_eye_dev(int n, const double* G, double* out, hipStream_t st);
@@ -483,6 +485,37 @@ struct Basis {
     }
     if (expect != nfunc) fail(1, "nfunc does not match the shells");
   }
+  // Shells by falling l, tight ones first within an l (ties in the caller's order), the order in which the Cholesky
+  // factor of the fitting metric loses least to rounding (metric.hip). Returns the new place of each of the caller's
+  // functions, nothing where the order stands already.
+  std::vector<int32_t> sort_shells() {
+    const int ns = n();
+    std::vector<double> least(ns);
+    std::vector<int32_t> order(ns), at(ns), fun;
+    for (int i = 0; i < ns; ++i) {
+      least[i] = *std::min_element(exps.begin() + prim0[i], exps.begin() + prim0[i] + nprim[i]);
+      order[i] = i;
+    }
+    std::stable_sort(order.begin(), order.end(),
+                     [&](int32_t a, int32_t b) { return l[a] != l[b] ? l[a] > l[b] : least[a] > least[b]; });
+    if (std::is_sorted(order.begin(), order.end())) return fun;
+    const std::vector<int32_t> l0 = l, np0 = nprim, pr0 = prim0;
+    const std::vector<double> c0 = centre;
+    int32_t ao = 0;
+    for (int k = 0; k < ns; ++k) {
+      const int32_t i = order[k];
+      l[k] = l0[i];
+      nprim[k] = np0[i];
+      prim0[k] = pr0[i];
+      for (int x = 0; x < 3; ++x) centre[3 * k + x] = c0[3 * i + x];
+      ao0[k] = at[i] = ao;
+      ao += nfun(l[k], spherical);
+    }
+    fun.reserve(nfunc);
+    for (int i = 0; i < ns; ++i)
+      for (int f = 0; f < nfun(l0[i], spherical); ++f) fun.push_back(at[i] + f);
+    return fun;
+  }
   // device copies on g_st; the host vectors stay alive with the Basis
   void upload() {
     auto up = [](auto& v) {
@@ -552,6 +585,9 @@ struct dfks_ctx {
   double hf = 0.0, e_nn = 0.0;
   dfks_options opt{};
   Basis orb, aux;
+  // the fitting functions are held in the order of sort_shells: the place of each of the caller's (empty: as given)
+  std::vector<int32_t> aux_fun;
+  int32_t* d_aux_fun = nullptr;
   std::vector<double> atm_host;  // x, y, z, Z
   std::vector<double> boys_host, gxyz_host, gw_host;
   hipStream_t st = nullptr;      // stream of the last call (the destructor frees on it)
@@ -697,7 +733,7 @@ struct dfks_ctx {
                     d_fitd, d_aob, d_zwb, d_fxc, d_rho0, d_Rf, d_xc_pts, d_xc_w, d_xc_exc, d_xc_ao,
                     d_xc_zw, d_xc_q, d_xc_ao32, d_xc_cols, d_xc_vlen, d_xc_shl, d_xc_shoff, d_xc_vrow,
                     d_xc_vprow, d_xc_vpcol, d_xc_zw2, d_xc_q2, d_Vxc2, d_uP, d_uJ, d_uK, d_ug, d_xcf_tab,
-                    d_xcf_ws, d_Blr, d_Klr, d_xk_blk, d_xk_wg, d_xk_part[0], d_xk_part[1], d_xk_coef[0],
+                    d_xcf_ws, d_Blr, d_Klr, d_aux_fun, d_xk_blk, d_xk_wg, d_xk_part[0], d_xk_part[1], d_xk_coef[0],
                     d_xk_coef[1]};
     for (void* p : ptrs) dfree(p);
     void* ptrs32[] = {d_gws, d_gpart, d_B32, d_ao32, d_zw32, t32_alias ? nullptr : d_T32, d_Cf32, d_P32, d_ws32,
@@ -1085,6 +1121,11 @@ void build_all(dfks_ctx* h, hipStream_t st) {
   // inputs to the device
   h->orb.upload();
   h->aux.upload();
+  if (!h->aux_fun.empty()) {
+    h->d_aux_fun = dalloc<int32_t>(h->aux_fun.size());
+    HIPCHK(hipMemcpyAsync(h->d_aux_fun, h->aux_fun.data(), h->aux_fun.size() * sizeof(int32_t), hipMemcpyHostToDevice,
+                          st));
+  }
   h->d_atm = dalloc<double>(h->atm_host.size());
   HIPCHK(hipMemcpyAsync(h->d_atm, h->atm_host.data(), h->atm_host.size() * sizeof(double), hipMemcpyHostToDevice, st));
   h->d_boys = dalloc<double>(h->boys_host.size());
@@ -3200,6 +3241,7 @@ int dfks_create(const dfks_system_desc* sys, const dfks_options* opt, dfks_handl
       }
       h->orb.load(sys->orbital);
       h->aux.load(sys->aux);
+      h->aux_fun = h->aux.sort_shells();
       if (sys->ngrid < 0) fail(1, "negative grid size");
       if (h->orb.maxl() > 3) fail(1, "orbital shells above f (l > 3) are not supported");
       if (h->aux.maxl() > 4) fail(1, "auxiliary shells above g (l > 4) are not supported");
@@ -3355,6 +3397,11 @@ int dfks_get_matrix(dfks_handle h, int32_t which, double* dev_out, dfks_stream s
       default: fail(1, "unknown matrix selector");
     }
     if (!src) fail(1, "this matrix is not held by the handle (recomputed slabs or a streamed AO grid)");
+    if (h->d_aux_fun && (which == DFKS_INT2C || which == DFKS_INT3C)) {
+      HIPCHK(launch_gather_fun((int64_t)(n / h->naux), h->naux, which == DFKS_INT2C, h->d_aux_fun, src, dev_out,
+                               S_(stream)));
+      return;
+    }
     HIPCHK(hipMemcpyAsync(dev_out, src, n * sizeof(double), hipMemcpyDeviceToDevice, S_(stream)));
   });
 }

@@ -79,6 +79,23 @@ __global__ __launch_bounds__(256) void k_dots_partial(DotList d, double* __restr
   if (threadIdx.x == 0) part[k * kRedBlocks + blockIdx.x] = s[0];
 }
 
+// out[r][c] = in[r or fun[r]][fun[c]]: a matrix over the fitting functions in the caller's order
+__global__ __launch_bounds__(256) void k_gather_fun(int64_t nrow, int n, int rows_too, const int32_t* __restrict__ fun,
+                                                    const double* __restrict__ in, double* __restrict__ out) {
+  for (int64_t r = blockIdx.x; r < nrow; r += gridDim.x) {
+    const double* src = in + (rows_too ? (int64_t)fun[r] : r) * n;
+    for (int c = threadIdx.x; c < n; c += 256) out[r * n + c] = src[fun[c]];
+  }
+}
+
+hipError_t launch_gather_fun(int64_t nrow, int n, int rows_too, const int32_t* fun, const double* in, double* out,
+                             hipStream_t st) {
+  if (nrow == 0 || n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_gather_fun, dim3((unsigned)std::min<int64_t>(nrow, 1 << 20)), dim3(256), 0, st, nrow, n, rows_too,
+                     fun, in, out);
+  return hipGetLastError();
+}
+
 // E holds some of the list's results, so it may not be restrict: its terms are read after they are stored.
 __global__ __launch_bounds__(256) void k_dots_final(DotList d, const double* __restrict__ part,
                                                     double* E) {

@@ -44,3 +44,39 @@ def test_fitted_tensor_edges(naux, norb, close, spec):
     b3 = B.reshape(norb, norb, -1)
     assert np.array_equal(b3, b3.transpose(1, 0, 2))
     c.close()
+
+
+def _cholesky80(V):
+    L = V.astype(np.longdouble)
+    for j in range(len(L)):
+        L[j, j] = np.sqrt(L[j, j])
+        L[j + 1:, j] /= L[j, j]
+        L[j + 1:, j + 1:] -= np.outer(L[j + 1:, j], L[j + 1:, j])
+    return np.tril(L)
+
+
+@pytest.mark.parametrize("heavy,seed", [(3, 0), (5, 0), (5, 1), (5, 2), (6, 0)])
+def test_rounding_on_molecules(heavy, seed):
+    """B B^T at a molecule's conditioning (3e6 to 7e6) against 80 bits, over 200 pairs: eigenvectors of the metric are
+    1.3 to 4.2e-15 off (norm against norm) on trees of 2 to 10 heavy atoms, a Cholesky factor taken atom by atom 2.0 to
+    7.1e-15; a blocked factor by falling l and exponent, replayed with the integrals of the oracle, at most 1.4e-15."""
+    from dftax_amd import Molecule, _native as N, tree_molecule
+    from dftax_amd.basis import build_basis
+    mol = tree_molecule(heavy, np.random.default_rng(heavy), basis="def2-svp")
+    xyz = mol.coords + 0.05 * np.random.default_rng(seed).standard_normal(mol.coords.shape)
+    mol = Molecule(mol.symbols, xyz, "def2-svp", spherical=True)
+    orb, aux = (build_basis(mol.symbols, xyz, b, spherical=True) for b in ("def2-svp", "even-tempered-jk"))
+    c = _handle(orb, aux, mol)
+    assert c.nfit == c.naux
+    V = c.matrix(N.DFKS_INT2C, (c.naux, c.naux)).cpu().numpy().astype(np.longdouble)
+    rows = np.random.default_rng(0).choice(c.nao ** 2, 200, replace=False)
+    I = c.matrix(N.DFKS_INT3C, (c.nao ** 2, c.naux)).cpu().numpy()[rows].T.astype(np.longdouble)
+    B = c.matrix(N.DFKS_BFIT, (c.nao ** 2, c.nfit)).cpu().numpy()[rows].T.astype(np.longdouble)
+    c.close()
+    L = _cholesky80(0.5 * (V + V.T))
+    Y = I.copy()
+    for i in range(len(L)):
+        Y[i] = (Y[i] - L[i, :i] @ Y[:i]) / L[i, i]
+    want = Y.T @ Y
+    off = np.linalg.norm((B.T @ B - want).astype(float)) / np.linalg.norm(want.astype(float))
+    assert off < 2.5e-15

@@ -1199,13 +1199,18 @@ void build_all(dfks_ctx* h, hipStream_t st) {
   // (metric.hip), else its eigendecomposition (rocSOLVER, a long chain of small kernels on an
   // n = naux matrix). Either needs only (P|Q): it runs on a side stream with its own rocBLAS handle
   // while the three-centre build and the AO grid plan run on st, and is collected before the fitted
-  // tensor. d_U, d_w, d_e, the Cholesky work, the side stream and handle stay with this build until then.
-  double* d_U = dalloc<double>((size_t)naux * naux);
-  double* d_w = dalloc<double>(naux);
-  double* d_e = dalloc<double>(naux);
-  double* d_chol = dalloc<double>(metric_chol_words(naux));
-  double* d_Lc = dalloc<double>((size_t)naux * naux);
-  double* d_lzm = dalloc<double>(3 * (size_t)naux + kLzParts + 2 * kLzSteps);
+  // tensor. Each takes its buffers where it runs: the Cholesky work (4 naux^2 words, given back as soon as the factor
+  // stands) on FP64 handles alone, the eigenvectors where they are needed.
+  struct MetricWork {
+    double *U = nullptr, *w = nullptr, *e = nullptr, *Lc = nullptr;
+    void release() {
+      for (double** p : {&U, &w, &e, &Lc}) {
+        dfree(*p);
+        *p = nullptr;
+      }
+    }
+    ~MetricWork() { release(); }
+  } mw;
   hipStream_t s_eig = nullptr;
   HIPCHK(hipStreamCreateWithFlags(&s_eig, hipStreamNonBlocking));
   rocblas_handle rb_eig = rb_acquire();
@@ -1222,29 +1227,44 @@ void build_all(dfks_ctx* h, hipStream_t st) {
     }
   } side{s_eig, rb_eig};
   RBCHK(rocblas_set_stream(rb_eig, s_eig));
-  // true: V's inverse Cholesky factor is in d_Lc (every eigenvalue above the cutoff)
+  // true: V's inverse Cholesky factor is in mw.Lc (every eigenvalue above the cutoff)
   const auto chol_launch = [&](const double* V, hipStream_t s) {
     // A handle with 32-bit products keeps the eigenvectors: their fitted functions are sorted by scale, which
     // 32 bits need (water dimer with recomputed slabs: E off by 5.5e-3 Ha with C^-T, under 1e-3 with U w^-1/2;
     // (H2O)_8 def2-TZVP with B kept: J off by 4.8e-4 against 2.2e-4). And the Lanczos kernel's partial
     // sums end at 4 kLzParts.
-    if (h->opt.precision == 1 || naux > 4 * kLzParts) return false;
-    HIPCHK(launch_lanczos(naux, V, d_lzm, s));
+    if (h->opt.precision == 1 || naux > 4 * kLzParts || !(h->opt.metric_cutoff >= 0.0)) return false;
+    struct Work {
+      double* p = nullptr;
+      ~Work() { dfree(p); }
+    } lz, chol;
+    try {
+      lz.p = dalloc<double>(3 * (size_t)naux + kLzParts + 2 * kLzSteps);
+      chol.p = dalloc<double>(metric_chol_words(naux));
+      mw.Lc = dalloc<double>((size_t)naux * naux);
+    } catch (const Fail&) {
+      (void)hipGetLastError();
+      return false;   // no room beside the integrals: the eigenvectors need less
+    }
+    HIPCHK(launch_lanczos(naux, V, lz.p, s));
     double ab[2 * kLzSteps];
-    HIPCHK(hipMemcpyAsync(ab, d_lzm + 3 * (size_t)naux + kLzParts, sizeof(ab), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipMemcpyAsync(ab, lz.p + 3 * (size_t)naux + kLzParts, sizeof(ab), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
     const double top = tridiagonal_top(kLzSteps, ab);
-    if (!(top > 0.0) || !(h->opt.metric_cutoff >= 0.0) || !std::isfinite(top)) return false;
+    if (!(top > 0.0) || !std::isfinite(top)) return false;
     // a little above the Ritz value; that no eigenvalue lies higher is one of the three factorisations
-    HIPCHK(launch_metric_chol(naux, V, h->opt.metric_cutoff, top * (1.0 + 1e-3), d_chol, d_Lc, h->d_info, s));
+    HIPCHK(launch_metric_chol(naux, V, h->opt.metric_cutoff, top * (1.0 + 1e-3), chol.p, mw.Lc, h->d_info, s));
     int flag = 0;
     HIPCHK(hipMemcpyAsync(&flag, h->d_info, sizeof(int), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
     return flag == 0;
   };
   const auto eig_launch = [&](const double* V, rocblas_handle rb, hipStream_t s) {
-    HIPCHK(hipMemcpyAsync(d_U, V, sizeof(double) * naux * naux, hipMemcpyDeviceToDevice, s));
-    RBCHK(rocsolver_dsyevd(rb, rocblas_evect_original, rocblas_fill_upper, naux, d_U, naux, d_w, d_e, h->d_info));
+    if (!mw.U) mw.U = dalloc<double>((size_t)naux * naux);
+    if (!mw.w) mw.w = dalloc<double>(naux);
+    if (!mw.e) mw.e = dalloc<double>(naux);
+    HIPCHK(hipMemcpyAsync(mw.U, V, sizeof(double) * naux * naux, hipMemcpyDeviceToDevice, s));
+    RBCHK(rocsolver_dsyevd(rb, rocblas_evect_original, rocblas_fill_upper, naux, mw.U, naux, mw.w, mw.e, h->d_info));
   };
   // the side stream's factor runs on its own host thread: rocSOLVER's divide and conquer holds its
   // calling thread for much of its run, which would otherwise delay the three-centre launches queued
@@ -1253,7 +1273,7 @@ void build_all(dfks_ctx* h, hipStream_t st) {
     std::thread t;
     int code = 0;
     std::string msg;
-    bool chol = false;   // d_Lc holds the factor
+    bool chol = false;   // mw.Lc holds the factor
     void finish() {
       if (t.joinable()) t.join();
       if (code) fail(code, msg);
@@ -1263,10 +1283,10 @@ void build_all(dfks_ctx* h, hipStream_t st) {
     }
   } eig;
   // metric pseudo-inverse factor L = U_keep w_keep^{-1/2} (nkeep columns kept by the relative cutoff) from
-  // the eigenpairs in d_U, d_w once stream s has finished them
+  // the eigenpairs in mw.U, mw.w once stream s has finished them
   const auto eig_factor = [&](int& nkeep, hipStream_t s) {
     std::vector<double> w(naux);
-    HIPCHK(hipMemcpyAsync(w.data(), d_w, sizeof(double) * naux, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipMemcpyAsync(w.data(), mw.w, sizeof(double) * naux, hipMemcpyDeviceToHost, s));
     int info = 0;
     HIPCHK(hipMemcpyAsync(&info, h->d_info, sizeof(int), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
@@ -1276,12 +1296,11 @@ void build_all(dfks_ctx* h, hipStream_t st) {
     while (k0 < naux && !(w[k0] > h->opt.metric_cutoff * wmax)) ++k0;
     nkeep = naux - k0;
     double* Lt = dalloc<double>((size_t)nkeep * naux);  // column-major nkeep x naux
-    HIPCHK(launch_metric_factor(naux, k0, d_U, d_w, Lt, st));
+    HIPCHK(launch_metric_factor(naux, k0, mw.U, mw.w, Lt, st));
     return Lt;
   };
   {
-    // the side stream starts after st's (P|Q) and the allocations above (stream-ordered on st, and a
-    // reused buffer's wait for its previous user is queued on st)
+    // the side stream starts after st's (P|Q)
     hipEvent_t ready = nullptr;
     HIPCHK(hipEventCreateWithFlags(&ready, hipEventDisableTiming));
     const hipError_t e1 = hipEventRecord(ready, st);
@@ -1292,12 +1311,16 @@ void build_all(dfks_ctx* h, hipStream_t st) {
   {
     int dev = 0;
     HIPCHK(hipGetDevice(&dev));
-    eig.t = std::thread([&eig, &eig_launch, &chol_launch, h, dev, rb_eig, s_eig] {
+    eig.t = std::thread([&eig, &eig_launch, &chol_launch, &mw, h, dev, rb_eig, s_eig] {
       try {
         HIPCHK(hipSetDevice(dev));
         StreamScope ss(s_eig);
         eig.chol = chol_launch(h->d_int2c, s_eig);
-        if (!eig.chol) eig_launch(h->d_int2c, rb_eig, s_eig);
+        if (!eig.chol) {
+          dfree(mw.Lc);
+          mw.Lc = nullptr;
+          eig_launch(h->d_int2c, rb_eig, s_eig);
+        }
         HIPCHK(hipStreamSynchronize(s_eig));
       } catch (const Fail& f) {
         eig.code = f.code;
@@ -1356,11 +1379,12 @@ void build_all(dfks_ctx* h, hipStream_t st) {
   double* d_Lt = nullptr;
   h->lt_tri = eig.chol;
   if (eig.chol) {
-    d_Lt = d_Lc;
-    d_Lc = nullptr;
+    d_Lt = mw.Lc;
+    mw.Lc = nullptr;
     h->nfit = naux;
   } else {
     d_Lt = eig_factor(h->nfit, s_eig);
+    mw.release();
   }
   const auto fit = [&](const double* I3, const double* Lt, int nfit, bool tri, double* B) {
     double* W = dalloc<double>(fit_words(naux, nfit));
@@ -1416,7 +1440,7 @@ void build_all(dfks_ctx* h, hipStream_t st) {
   sync(st);
   h->build_ms[3] = now_ms() - t0;
   t0 = now_ms();
-  dfree(d_U); dfree(d_w); dfree(d_e); dfree(d_chol); dfree(d_Lc); dfree(d_lzm);
+  mw.release();
 
   // Fock-build scratch: exchange intermediate for up to nf_chunk factor columns
   h->d_Tx = dalloc<double>((size_t)nao * std::max(h->nfit, h->nfit_lr) * h->nf_chunk);

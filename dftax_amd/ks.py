@@ -140,16 +140,21 @@ def memory_plan(nao: int, naux: int, ngrid: int, nocc: int, precision: str, chun
     Word counts (FP64, the mixed path adds FP32 copies): B is nao^2 naux and
     the build holds (mn|P) and B together (a range-separated hybrid,
     ``tensors = 2``, keeps its long-range B beside it and is materialised
-    only); the recompute path holds a slab
-    of nao^2 x chunk, the raw and fitted exchange intermediates (2 nao naux
-    nf) and the metric factor; the AO grid is 4 ng nao values plus ng nao for
-    Z/W. ``budget`` is the device bytes the handle may use.
+    only), (P|Q), the metric factor and its padded copy; the recompute path
+    holds a slab of nao^2 x chunk, the raw and fitted exchange intermediates
+    (2 nao naux nf), (P|Q) and the metric factor, and before the fitted
+    intermediate the work of that factor (4 naux^2 for the Cholesky factor of an
+    FP64 handle, naux^2 for eigenvectors); the AO grid is 4 ng nao values plus
+    ng nao for Z/W. ``budget`` is the device bytes the handle may use.
     """
     w = 8
     f32 = 1.5 if precision == "mixed" else 1.0
     nf = max(1, min(nao, 512, max(nocc, 1)))
     exch = nao * naux * nf * w * f32 + 64 * nao * nao * w
-    mat = max((1 + tensors) * nao * nao * naux * w, tensors * nao * nao * naux * w * f32 + exch)
+    metric = naux * naux * w
+    work = metric if precision == "mixed" else 4 * metric
+    mat = max((1 + tensors) * nao * nao * naux * w + metric, nao * nao * naux * w + work,
+              tensors * nao * nao * naux * w * f32 + exch) + 2 * metric
     if chunk is None or tensors > 1:
         aux_chunk = 0
     elif isinstance(chunk, int):
@@ -160,9 +165,10 @@ def memory_plan(nao: int, naux: int, ngrid: int, nocc: int, precision: str, chun
         if aux_chunk == -1:
             # slab of about 1/8 of the budget, 32 .. 2048 functions
             aux_chunk = int(min(2048, max(32, budget // 8 // (nao * nao * w))))
-        df_bytes = nao * nao * aux_chunk * w + 2 * nao * naux * nf * w + naux * naux * w + 64 * nao * nao * w
+        steady = nao * naux * nf * w + 64 * nao * nao * w
         if precision == "mixed":
-            df_bytes += nao * nao * aux_chunk * 4 + naux * naux * 4   # FP32 slab and metric factor
+            steady += nao * nao * aux_chunk * 4 + naux * naux * 4   # FP32 slab and metric factor
+        df_bytes = nao * nao * aux_chunk * w + nao * naux * nf * w + 2 * metric + max(steady, work)
     else:
         df_bytes = mat
     grid = 5 * ngrid * nao * w * f32

@@ -4,7 +4,8 @@ Requests (molecules) arrive over time; each one needs a full DF-KS solve.
 The server keeps a FIFO of arrived requests and admits the head as soon as
 a worker slot is free and its HBM footprint fits the remaining budget. The
 footprint counts B (nao^2 * nfit words, plus its FP32 copy and the unfitted
-tensor during the build), the AO grid and the SCF workspaces. Each admitted
+tensor during the build), the metric and its factor, the AO grid and the SCF
+workspaces. Each admitted
 request runs on its own HIP stream from its own worker thread: its native
 handle is built, the SCF runs (mixed precision with FP64 refinement by
 default) and the handle is freed, returning its budget. Kernels of
@@ -63,8 +64,10 @@ def footprint_bytes(mol, auxbasis: str, grid: Becke, precision: str) -> int:
     nocc = mol.nelectron // 2
     w3 = nao * nao * naux
     f32 = precision == "mixed"
-    build_peak = 2 * 8 * w3                                   # (mn|P) and B together
-    steady = 8 * w3 + (4 * w3 if f32 else 0)                  # B (+ FP32 copy)
+    metric = 8 * naux * naux
+    # (mn|P) and B together, the metric factor's padded copy; before B, the work of the factor
+    build_peak = max(2 * 8 * w3 + metric, 8 * w3 + (metric if f32 else 4 * metric)) + 2 * metric
+    steady = 8 * w3 + (4 * w3 if f32 else 0) + 2 * metric     # B (+ FP32 copy), (P|Q) and the metric factor
     steady += ng * nao * (8 * 5 + (4 * 5 if f32 else 0))      # AO planes + Z/W (+ FP32 copies)
     steady += nao * naux * max(nocc, 1) * (8 + (4 if f32 else 0))
     steady += 8 * nao * nao * (64 + 40)                       # split-K workspace, DIIS, matrices

@@ -60,3 +60,35 @@ def test_kept_buffers_are_reused_and_counted(water_dimer_tzvp):
     dev_released, _ = torch.cuda.mem_get_info(0)
     _say(f"after dfks_release_memory: device free {dev_released / 1e9:.3f} GB")
     assert dev_released >= after - SLACK
+
+
+def test_mixed_build_takes_no_cholesky_work():
+    """A handle with 32-bit products takes the metric's eigenvectors: its build holds (P|Q), the factor and the
+    eigenvectors, whose buffer the factor's padded copy takes over, and none of the 5 naux^2 words of the Cholesky
+    factor and its work. Every buffer that a build
+    took stays with the library afterwards, so what the device counts as used is their sum (rocSOLVER's workspace, which
+    stays with its handle, is in place before)."""
+    import torch
+    from dftax_amd import _native
+    from dftax_amd.ks import HipDFKS, HipSpec
+    from dftax_amd.system import Molecule
+    from dftax_amd.xc import PBE0
+    from test_gpu_eri_pair import _basis
+    naux = 2048
+    site = 1.6 * np.indices((13, 13, 13)).reshape(3, -1).T[:naux] + 0.0
+    aux = _basis([(0, 0, x, [0.9]) for x in site], True)
+    orb = _basis([(0, 0, x, [0.8]) for x in site[:2]], True)
+    mol = Molecule(["O"] * 2, np.array([[0.0, 0.0, 0.0], [0.0, 0.1, 2.1]]), "sto-3g")
+
+    def build():
+        HipDFKS(orb, aux, mol, np.zeros((1, 3)) + 5.0, np.ones(1), PBE0(), 2, HipSpec(precision="mixed"),
+                chunk=None).close()
+        torch.cuda.synchronize()
+
+    build()
+    _native.release_memory(0)
+    before, _ = torch.cuda.mem_get_info(0)
+    build()
+    after, _ = torch.cuda.mem_get_info(0)
+    _say(f"taken by a build of {naux} fitting functions: {(before - after) / (8 * naux * naux):.2f} naux^2 words")
+    assert 2 * 8 * naux * naux < before - after < 6 * 8 * naux * naux

@@ -180,3 +180,16 @@ def test_mixed_phase_switch_rule():
     assert mixed_phase_done([1e-2] * 30) and not mixed_phase_done([1e-2] * 29)
     # stall detection off
     assert not mixed_phase_done(plateau, stall=0)
+
+
+def test_memory_plan_counts_the_metric():
+    """Where the fitting span outgrows the pairs of orbitals, a build's peak is the metric's factor: (P|Q), the factor
+    and 4 naux^2 words of Cholesky work in FP64, as much as the eigenvectors take on a mixed handle."""
+    from dftax_amd.ks import memory_plan
+    nao, naux, gb = 40, 20000, 1 << 30
+    mm = 8 * naux * naux
+    for precision, work in (("fp64", 6 * mm), ("mixed", 3 * mm)):
+        kept = memory_plan(nao, naux, 0, 1, precision, None, 0, 200 * gb)
+        assert work + 8 * nao * nao * naux <= kept.bytes_est <= 1.1 * (work + 24 * nao * nao * naux)
+        slabs = memory_plan(nao, naux, 0, 1, precision, 64, 0, 200 * gb)
+        assert work <= slabs.bytes_est <= 1.1 * work

@@ -975,35 +975,37 @@ struct SmallOperand {
       for (int e = 0; e < 2; ++e) p[e] = A + min(r0 + 2 * li + e, n - 1);
     }
   }
-  // x[e][s]: tile e, k = k0 + 2 lk + s (k past K: any element)
+  // x[e][s]: tile e, k = k0 + 2 lk + s, zero for k past K (in both operands: an infinity of one would meet the
+  // other's zero otherwise)
   __device__ __forceinline__ void load(int k0, int K, double (&x)[2][2]) const {
     const int k = k0 + 2 * ((threadIdx.x & 63) >> 4);
+    const bool whole = k0 + 8 <= K;
     if constexpr (KC) {
-      if (k0 + 8 <= K) {
+      if (whole) {
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
           const dbl2u v = *reinterpret_cast<const dbl2u*>(p[e] + k);
           x[e][0] = v[0];
           x[e][1] = v[1];
         }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 2; ++e)
-#pragma unroll
-          for (int s = 0; s < 2; ++s) x[e][s] = p[e][min(k + s, K - 1)];
+        return;
       }
-    } else {
+    } else if (whole && full) {
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
-        const int64_t o = (int64_t)min(k + s, K - 1) * ld;
-        if (full) {
-          const dbl2u v = *reinterpret_cast<const dbl2u*>(p[0] + o);
-          x[0][s] = v[0];
-          x[1][s] = v[1];
-        } else {
-          x[0][s] = p[0][o];
-          x[1][s] = p[1][o];
-        }
+        const dbl2u v = *reinterpret_cast<const dbl2u*>(p[0] + (int64_t)(k + s) * ld);
+        x[0][s] = v[0];
+        x[1][s] = v[1];
+      }
+      return;
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int64_t kc = min(k + s, K - 1), o = KC ? kc : kc * ld;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const double v = p[e][o];
+        x[e][s] = k + s < K ? v : 0.0;
       }
     }
   }
@@ -1026,17 +1028,14 @@ __global__ __launch_bounds__(256, 2) void k_gemm_s(int M, int N, int K, double a
   const int groups = (K + 7) / 8, g0 = groups * wave / 4, g1 = groups * (wave + 1) / 4;
   dbl4 acc[2][2] = {};
   double x[2][2][2], y[2][2][2];
-  const auto mul = [&](int k0, double (&u)[2][2], double (&v)[2][2]) __attribute__((always_inline)) {
+  const auto mul = [&](double (&u)[2][2], double (&v)[2][2]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const bool in = k0 + 2 * lk + s < K;
-      const double u0 = in ? u[0][s] : 0.0, u1 = in ? u[1][s] : 0.0;
+    for (int s = 0; s < 2; ++s)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        acc[0][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(u0, v[j][s], acc[0][j], 0, 0, 0);
-        acc[1][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(u1, v[j][s], acc[1][j], 0, 0, 0);
-      }
-    }
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(u[i][s], v[j][s], acc[i][j], 0, 0, 0);
   };
   if (g0 < g1) {
     a.load(8 * g0, K, x[0]);
@@ -1045,13 +1044,13 @@ __global__ __launch_bounds__(256, 2) void k_gemm_s(int M, int N, int K, double a
     for (; g + 2 <= g1; g += 2) {
       a.load(8 * (g + 1), K, x[1]);
       b.load(8 * (g + 1), K, y[1]);
-      mul(8 * g, x[0], y[0]);
+      mul(x[0], y[0]);
       const int gn = min(g + 2, g1 - 1);
       a.load(8 * gn, K, x[0]);
       b.load(8 * gn, K, y[0]);
-      mul(8 * (g + 1), x[1], y[1]);
+      mul(x[1], y[1]);
     }
-    if (g < g1) mul(8 * g, x[0], y[0]);
+    if (g < g1) mul(x[0], y[0]);
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i)

@@ -201,6 +201,7 @@ hipError_t launch_sp2_tile(int n, const double* X, double* Xn, int nocc, const d
 hipError_t launch_sp2_settle(int nocc, double* st, hipStream_t s);
 int pfactor_panel(int n);
 int pfactor_max_n();
+int pfactor_columns(const double* st, double tol);
 hipError_t launch_pfactor(int n, int c0, int npanel, double tol, double* R, double* d, double* L, double* st,
                           double* part, hipStream_t s);
 hipError_t launch_diag(int n, const double* R, double* d, hipStream_t s);
@@ -2151,7 +2152,7 @@ void energy_fock_factored(dfks_ctx* h, const double* P, const double* Cf, const 
 // P = L L^T of a positive semidefinite P by pivoted Cholesky (columns to d_Cf), stopped where the residual's
 // diagonal is down to rounding, 1e-14 of P's largest diagonal element, the relative cutoff of the eigenvalues
 // below. Returns the number of columns, -1 when the residual is not down to rounding everywhere, as for an
-// indefinite or unsymmetric P (or past the kernel's size).
+// indefinite or unsymmetric P or one that is not finite (or past the kernel's size).
 int factor_psd(dfks_ctx* h, const double* P, hipStream_t st) {
   const int nao = h->nao, pb = pfactor_panel(nao);
   const double tol = 1e-14;
@@ -2164,7 +2165,7 @@ int factor_psd(dfks_ctx* h, const double* P, hipStream_t st) {
     double s[4];
     HIPCHK(hipMemcpyAsync(s, h->d_part, sizeof(s), hipMemcpyDeviceToHost, st));
     sync(st);
-    if (s[2] != 0.0) return s[3] <= 8.0 * tol * s[0] ? (int)s[1] : -1;
+    if (s[2] != 0.0) return pfactor_columns(s, tol);
   }
   return -1;
 }

@@ -29,6 +29,7 @@
 // panel's pivots (largest residual diagonal) and forms its columns, then a
 // GEMM removes the panel from the trailing residual. (The SCF driver uses it
 // on the first step; later steps project the previous factor.)
+#include <cmath>
 #include <cstdint>
 
 #include "dfks_common.h"
@@ -1137,6 +1138,12 @@ hipError_t launch_sp2_settle(int nocc, double* st, hipStream_t s) {
 
 int pfactor_panel(int n) { return n <= 2 * kPfThreads ? 32 : 16; }   // columns per panel
 int pfactor_max_n() { return 4 * kPfThreads; }
+
+// What a finished factorisation found, st as launch_pfactor leaves it: the columns, or -1 where the residual is not down
+// to rounding everywhere. A largest diagonal that is not finite bounds nothing.
+int pfactor_columns(const double* st, double tol) {
+  return std::isfinite(st[0]) && st[3] <= 8.0 * tol * st[0] ? (int)st[1] : -1;
+}
 
 // npanel panels of the pivoted Cholesky of R (n x n, destroyed; d: n words, L: column-major, room for n
 // columns), from column c0 (a multiple of the panel; 0 starts afresh): st[0..3] = largest diagonal, columns,

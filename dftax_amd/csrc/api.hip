@@ -3384,10 +3384,10 @@ int dfks_stats(dfks_handle h, int64_t* out, int32_t n) {
     if (!h || !out) fail(1, "null argument");
     int64_t width = 0;
     for (const auto& bn : h->xbins) width += bn.nblk * bn.n;
-    const int64_t v[11] = {h->pairs_kept, h->pairs_total, (int64_t)h->slab_np.size(), h->max_np, h->ao_block,
+    const int64_t v[12] = {h->pairs_kept, h->pairs_total, (int64_t)h->slab_np.size(), h->max_np, h->ao_block,
                            h->n_eigh_steps, h->sp2_guess, h->xc_nblk, (int64_t)h->xbins.size(), width,
-                           h->n_pchol_steps};
-    for (int i = 0; i < n; ++i) out[i] = i < 11 ? v[i] : 0;
+                           h->n_pchol_steps, h->lt_tri ? 1 : 0};
+    for (int i = 0; i < n; ++i) out[i] = i < 12 ? v[i] : 0;
   });
 }
 

@@ -70,3 +70,33 @@ def test_general(kind):
         K += B[:, l] @ X[l].T
     _close(F, H + J - 0.125 * K)
     c.close()
+
+
+@pytest.mark.parametrize("kind,size", [("antisymmetric", 1e-16), ("antisymmetric", 1e-13), ("antisymmetric", 1e-6),
+                                       ("negative", 1e-15), ("negative", 1e-13), ("negative", 1e-12)])
+def test_about_the_residual_limit(kind, size):
+    """Parts that the residual limit (8e-14 of the largest diagonal element) lets pass as rounding and parts that it does
+    not: an antisymmetric one, which J of a symmetric tensor and the symmetrised K do not see, and a negative one. What
+    is dropped is at most its size times the largest integral sums, within the bound for a unit density."""
+    import torch
+    from dftax_amd import _native as N
+    c = _handle(2, "def2-tzvp")
+    n = c.nao
+    A, D = _factor(c, 9, 1), _factor(c, 5, 2)
+    S = A @ A.T
+    R = D @ D.T if kind == "negative" else D @ A[:, :5].T - A[:, :5] @ D.T
+    P = (S - size * float(S.diag().max()) * R / float(R.abs().max())).contiguous()
+    E, F = c.energy_fock(P)
+    P = 0.5 * (P + P.T)
+    B = c.matrix(N.DFKS_BFIT, (n, n, c.nfit))
+    H = c.matrix(N.DFKS_HCORE, (n, n))
+    J = B @ torch.einsum("mnq,mn->q", B, P)
+    X = (P @ B.reshape(n, n * c.nfit)).reshape(n, n, c.nfit)
+    K = torch.zeros_like(P)
+    for l in range(n):
+        K += B[:, l] @ X[l].T
+    want = H + J - 0.125 * K
+    c.close()
+    # an antisymmetric part beyond rounding goes to the eigenvectors of one triangle, whose own symmetric part it is
+    slack = 0.0 if kind == "negative" or size < 1e-7 else 1e3 * size
+    assert float((F - want).abs().max()) < (TOL + slack) * max(1.0, float(want.abs().max()))

@@ -80,3 +80,53 @@ def test_rounding_on_molecules(heavy, seed):
     want = Y.T @ Y
     off = np.linalg.norm((B.T @ B - want).astype(float)) / np.linalg.norm(want.astype(float))
     assert off < 2.5e-15
+
+
+def _span(case):
+    """Fitting functions, the metric cutoff as a multiple of the smallest eigenvalue's share (None: the default), and
+    whether every eigenvalue is kept by a factor without eigenvectors."""
+    rng = np.random.default_rng(5)
+    if case == "wide":
+        # 400 functions far apart, eigenvalues 4 pi / exponent = sqrt(i / 400): crowded at the top, where 24 Lanczos
+        # steps end 1.7e-3 short, so that the bound 1.001 times the Ritz value is under the largest
+        site = 1e8 * np.indices((8, 8, 8)).reshape(3, -1).T[:400] + 0.0
+        return _basis([(0, 0, x, [4.0 * np.pi / np.sqrt(k / 400.0)]) for k, x in enumerate(site, 1)], True), None, False
+    site = 1.6 * np.indices((5, 5, 5)).reshape(3, -1).T[:90] + rng.uniform(-0.1, 0.1, (90, 3))
+    aux = _basis([(0, 0, x, [0.9]) for x in site], True)
+    return aux, *{"kept": (None, True), "above": (0.97, True), "below": (1.03, False), "zero": (0.0, True)}[case]
+
+
+@pytest.mark.parametrize("case", ["kept", "above", "below", "zero", "wide"])
+def test_which_factor(case):
+    """The Cholesky factor stands where the smallest eigenvalue is 3 % over the cutoff, and eigenvectors where it is 3 %
+    under it (one function fewer) or where the bound on the largest does not hold; B B^T is that of the eigenvalues
+    above the cutoff in every case."""
+    from dftax_amd import _native as N
+    from dftax_amd.system import Molecule
+    from oracle import ref
+    aux, share, chol = _span(case)
+    orb = _basis([(0, 0, x, [0.8]) for x in np.random.default_rng(6).uniform(0.0, 6.0, (5, 3))], True)
+    V, I = ref.int2c(aux), ref.int3c(orb, aux).reshape(25, -1)
+    w, U = np.linalg.eigh(V)
+    cutoff = 1e-7 if share is None else share * w[0] / w[-1]
+    mol = Molecule(["O"] * 2, np.array([[0.0, 0.0, 0.0], [0.0, 0.1, 2.1]]), "sto-3g")
+    c = _handle(orb, aux, mol, metric_cutoff=cutoff)
+    keep = w > cutoff * w[-1]
+    assert c.nfit == keep.sum() == len(w) - (case == "below")
+    assert c.stats()["metric_cholesky"] == chol
+    B = c.matrix(N.DFKS_BFIT, (25, c.nfit)).cpu().numpy()
+    c.close()
+    if chol:   # C^-T: the first fitted function is the first fitting function alone
+        assert np.abs(B[:, 0] - I[:, 0] / np.sqrt(V[0, 0])).max() < 1e-12 * max(1.0, np.abs(I).max())
+    want = (I @ (U[:, keep] / w[keep])) @ (I @ U[:, keep]).T
+    assert np.abs(B @ B.T - want).max() < 1e-9 * max(1.0, np.abs(want).max())
+
+
+def test_mixed_handle_keeps_eigenvectors():
+    from dftax_amd.system import Molecule
+    aux, _, _ = _span("kept")
+    orb = _basis([(0, 0, np.zeros(3), [0.8])], True)
+    mol = Molecule(["O"] * 2, np.array([[0.0, 0.0, 0.0], [0.0, 0.1, 2.1]]), "sto-3g")
+    c = _handle(orb, aux, mol, precision="mixed")
+    assert c.nfit == c.naux and c.stats()["metric_cholesky"] == 0
+    c.close()

@@ -1177,7 +1177,7 @@ __global__ __launch_bounds__(256, NJ <= 1 ? 4 : 2) void k_gemm_t(int64_t M, int 
   // FULL: all of the workgroup's rows exist
   const auto product = [&](auto FULL) __attribute__((always_inline)) {
     const auto load_a = [&](int s, int k0) __attribute__((always_inline)) {
-      const double* src = A + (int64_t)min(k0 + 4 * s + lk, K - 1) * lda;   // past the end: B is zero there
+      const double* src = A + (int64_t)min(k0 + 4 * s + lk, K - 1) * lda;
 #pragma unroll
       for (int p = 0; p < MP; ++p) {
         const int64_t m = mw + 32 * p + 2 * li;
@@ -1200,6 +1200,13 @@ __global__ __launch_bounds__(256, NJ <= 1 ? 4 : 2) void k_gemm_t(int64_t M, int 
       __syncthreads();     // the other buffer's readers passed the previous barrier
       const int kn = min(k0 + 16, K - 1);      // the last step's reloads are not used
       load_b(kn);
+      if (k0 + 16 > K) {   // past the end both operands are zero
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int p = 0; p < MP; ++p)
+            if (k0 + 4 * s + lk >= K) a[s][p] = dbl2u{0.0, 0.0};
+      }
       double bf[2][NJ];
 #pragma unroll
       for (int j = 0; j < NJ; ++j) bf[0][j] = sb[j * 64 + lane];

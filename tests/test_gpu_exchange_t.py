@@ -59,3 +59,43 @@ def test_exchange_k_tiles(nao, naux, nf):
         got.append(c.energy_fock_factored(Cf))
     for a, b in zip(*got):
         assert float((a - b).abs().max()) < TOL * max(1.0, float(b.abs().max()))
+
+
+@pytest.mark.parametrize("N", [3, 40, 80, 81, 150])
+@pytest.mark.parametrize("K", [1, 15, 16, 18, 37])
+def test_infinities_in_the_last_group_of_t(N, K):
+    """One infinite element at the last k of either operand of T = A B^T reaches its row or column as an infinity, on
+    whole and partial tiles of rows and on both sides of the groups of 16 (k past the end is zero in both operands)."""
+    import ctypes
+    import torch
+    from dftax_amd import _native
+
+    class Gemm(ctypes.Structure):
+        _fields_ = [("M", ctypes.c_int), ("N", ctypes.c_int), ("K", ctypes.c_int64), ("A", ctypes.c_void_p),
+                    ("lda", ctypes.c_int64), ("a_kcontig", ctypes.c_bool), ("B", ctypes.c_void_p),
+                    ("ldb", ctypes.c_int64), ("b_kcontig", ctypes.c_bool)]
+
+    class RowDot(ctypes.Structure):   # no row terms: out = null
+        _fields_ = [("cf", ctypes.c_void_p), ("sg", ctypes.c_void_p), ("nao", ctypes.c_int), ("nq", ctypes.c_int),
+                    ("out", ctypes.c_void_p)]
+
+    f = _native.lib()["_ZN4dfks15launch_gemm_t64ERKNS_8GemmArgsEPdRKNS_6RowDotEP12ihipStream_t"]
+    f.restype = ctypes.c_int
+    f.argtypes = [ctypes.POINTER(Gemm), ctypes.c_void_p, ctypes.POINTER(RowDot), ctypes.c_void_p]
+    M = 261   # one whole tile of rows, of 256 or 128, and a partial one
+    g = torch.Generator().manual_seed(K)
+    for at in ((0, 0), (258, N - 1)):
+        for which in ("a", "b"):
+            A = torch.rand((M, K), dtype=torch.float64, generator=g) + 0.5
+            B = torch.rand((N, K), dtype=torch.float64, generator=g) + 0.5
+            (A[at[0]] if which == "a" else B[at[1]])[K - 1] = float("inf")
+            want = A @ B.T
+            a, b = A.T.contiguous().cuda(), B.cuda()
+            c = torch.empty((M, N), dtype=torch.float64, device="cuda")
+            assert f(Gemm(M, N, K, a.data_ptr(), M, False, b.data_ptr(), K, True), c.data_ptr(),
+                     RowDot(None, None, 0, 1, None),
+                     torch.cuda.current_stream().cuda_stream) == 0
+            got = c.cpu()
+            assert torch.equal(got.isinf(), want.isinf()) and not got.isnan().any()
+            # sums of K terms under 2.25
+            assert (got - want)[want.isfinite()].abs().max() < 1e-14 * K

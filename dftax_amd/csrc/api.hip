@@ -1010,7 +1010,8 @@ void plan_xc_blocks(dfks_ctx* h, hipStream_t st) {
     const int nt = (bn->n + 63) / 64;
     for (int64_t k = 0; k < bn->nblk; ++k) {
       xk.push_back({bn->ao_off + k * kXcG * bn->n, bn->nblk * kXcG * bn->n, bn->col_off + k * bn->n,
-                    bn->q_off + k * (int64_t)bn->n * bn->n, bn->pt0 + k * kXcG, h->xk_nparts, bn->n, 0});
+                    bn->q_off + k * (int64_t)bn->n * bn->n, bn->pt0 + k * kXcG, h->xk_nparts, bn->n,
+                    cnt[order[bn->blk0 + k]]});
       h->xk_nparts += nt;
     }
   }

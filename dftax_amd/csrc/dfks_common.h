@@ -49,13 +49,13 @@ struct XcfBin {
   int64_t ao_off, col_off, q_off, pt0, part_off, coef_off;
   int32_t wz0, wp0, wv0, pad;
 };
-// One block of the compact XC grid for the FP64 kernels (xc_blocks.hip): n functions, the
+// One block of the compact XC grid for the FP64 kernels (xc_blocks.hip): n columns, nf of them functions, the
 // offsets of its AO rows (first plane; planes are plane doubles apart), columns, product,
 // first point and first strip of partial sums. A workgroup id packs block * kXcbStrips + strip.
 constexpr int kXcbStrips = 32;        // strips of 64 columns: n <= kXfMaxN
 struct XcBlock {
   int64_t ao0, plane, col0, q0, pt0, part0;
-  int32_t n, pad;
+  int32_t n, nf;
 };
 constexpr int kPanel = 32;            // pivoted Cholesky panel width
 // out[k] = scale[k] sum x[k] y[k] (+= with add), k < count

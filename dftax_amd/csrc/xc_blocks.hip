@@ -1,7 +1,7 @@
 // FP64 products of the XC term on the compact grid, all blocks in one launch.
 //
 // Block b holds 128 grid points and the n functions cols[0..n) that reach them
-// (n a multiple of 32, -1 pads); its AO planes are ao[k plane + g n + i].
+// (n a multiple of 32, -1 pads past the first nf); its AO planes are ao[k plane + g n + i].
 //   k_xcb_rho  Z = Phi P_b over a strip of at most 64 columns, reduced at once to the
 //              strip's share of rho and grad rho, so Z is never stored
 //   k_xcb_v    Vh_b = Phi^T W over a strip, W = a phi + b . grad phi formed in LDS
@@ -72,10 +72,7 @@ __device__ __forceinline__ void rho_strip(const XcBlock& b, int c0, const double
   dbl2 a[2][2][2];   // k half, point group, pair of k
   const auto load_p = [&](int k0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int e = 0; e < PER; ++e) {
-      // a padded k or column meets zero AO values: any element of P will do there
-      p[e] = pcol[(int64_t)max(cols[k0 + pk + STEP * e], 0) * nao];
-    }
+    for (int e = 0; e < PER; ++e) p[e] = pcol[(int64_t)max(cols[k0 + pk + STEP * e], 0) * nao];
   };
   const auto load_a = [&](int q, int k0) __attribute__((always_inline)) {
 #pragma unroll
@@ -90,6 +87,11 @@ __device__ __forceinline__ void rho_strip(const XcBlock& b, int c0, const double
   load_a(1, 0);
   for (int k0 = 0, buf = 0; k0 < n; k0 += kKC, buf ^= 1) {
     double* sp = s_p + buf * (kKC * 64);
+    if (k0 + kKC > b.nf || c0 + W > b.nf) {   // padded k and columns: zero, whatever P[0][.] and P[.][0] hold
+#pragma unroll
+      for (int e = 0; e < PER; ++e)
+        if (k0 + pk + STEP * e >= b.nf || c0 + pc >= b.nf) p[e] = 0.0;
+    }
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
       const int k = pk + STEP * e;   // its step (k / 16, k % 4) and lane group (k % 16) / 4

@@ -57,3 +57,28 @@ def test_spin_polarised(spin, charge, name):
         got.append(k.coulomb.energy_fock(initial_density(k, None)))
     for a, b in zip(*got):
         assert float((a - b).abs().max()) < TOL * max(1.0, float(b.abs().max()))
+
+
+def test_what_is_not_finite_stays_with_its_blocks():
+    """NaN in P[0][0] masks the points that function 0 reaches and no others: the columns that fill up a block to 32 are
+    zero whatever P holds."""
+    import ctypes
+    import torch
+    from dftax_amd import KS, _native, becke, df, hip, water_cluster
+    from dftax_amd.scf import initial_density
+    mol = water_cluster((3, 1, 1), seed=2, basis="def2-svp")
+    got = []
+    for gemm in ("auto", "rocblas"):
+        k = KS(mol, "PBE", grid=becke(30, 110), coulomb=df(engine=hip(gemm=gemm)))
+        c, P = k.coulomb, initial_density(k, None).contiguous().clone()
+        P[0, 0] = float("nan")
+        cm, signs = torch.zeros((1, c.nao), dtype=torch.float64, device=P.device), (ctypes.c_double * 1)(1.0)
+        F = torch.empty_like(P)
+        _native.check(c.L.dfks_energy_fock_factored(c.handle, ctypes.c_void_p(P.data_ptr()),
+                                                    ctypes.c_void_p(cm.data_ptr()), signs, 1,
+                                                    ctypes.c_void_p(c._E.data_ptr()), ctypes.c_void_p(F.data_ptr()),
+                                                    c._stream()))
+        got.append((float(c._E[4]), F.clone()))
+    (a, Fa), (b, Fb) = got
+    assert b < -1.0 and abs(a - b) < TOL * abs(b)
+    assert float((Fa - Fb).abs().max()) < TOL * max(1.0, float(Fb.abs().max()))

@@ -9,6 +9,7 @@
 //   X, C   column-major       nao x nmo orthonormaliser / MO coefficients
 // Plain GEMM/SYRK/SYR2K shapes go to rocBLAS and the symmetric eigensolves to
 // rocSOLVER; every other step is a kernel of this library.
+#include <dlfcn.h>
 #include <hip/hip_runtime.h>
 #include <rocblas/rocblas.h>
 #include <rocsolver/rocsolver.h>
@@ -1116,6 +1117,14 @@ double tridiagonal_top(int m, const double* ab) {
   return hi;
 }
 
+// Whether a ROCprofiler tool is in the process (tools export rocprofiler_configure and are named in
+// ROCP_TOOL_LIBRARIES). Two builds under one ended in a host access violation inside rocSOLVER's launches on the
+// metric's side thread, cause not shown: with a tool present the factor runs on the calling thread.
+bool profiler_loaded() {
+  const char* tools = std::getenv("ROCP_TOOL_LIBRARIES");
+  return (tools && *tools) || dlsym(RTLD_DEFAULT, "rocprofiler_configure");
+}
+
 void build_all(dfks_ctx* h, hipStream_t st) {
   h->rb = rb_acquire();
   RBCHK(rocblas_set_stream(h->rb, st));
@@ -1313,7 +1322,7 @@ void build_all(dfks_ctx* h, hipStream_t st) {
   {
     int dev = 0;
     HIPCHK(hipGetDevice(&dev));
-    eig.t = std::thread([&eig, &eig_launch, &chol_launch, &mw, h, dev, rb_eig, s_eig] {
+    const auto factor = [&eig, &eig_launch, &chol_launch, &mw, h, dev, rb_eig, s_eig] {
       try {
         HIPCHK(hipSetDevice(dev));
         StreamScope ss(s_eig);
@@ -1331,7 +1340,9 @@ void build_all(dfks_ctx* h, hipStream_t st) {
         eig.code = 9;
         eig.msg = e.what();
       }
-    });
+    };
+    if (profiler_loaded()) factor();
+    else eig.t = std::thread(factor);
   }
   // bra pairs (Schwarz-screened when screen > 0)
   setup_pairs(h, pairs, d_pairs, pair_off, st);

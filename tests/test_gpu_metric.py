@@ -130,3 +130,25 @@ def test_mixed_handle_keeps_eigenvectors():
     c = _handle(orb, aux, mol, precision="mixed")
     assert c.nfit == c.naux and c.stats()["metric_cholesky"] == 0
     c.close()
+
+
+@pytest.mark.parametrize("spec", [{}, {"precision": "mixed"}])
+def test_factor_on_the_calling_thread(spec, monkeypatch):
+    """With a profiler tool named in the environment the metric's factor runs on the calling thread: the same B."""
+    import torch
+    from dftax_amd import _native as N
+    from dftax_amd.system import Molecule
+    torch.cuda.init()   # the tool's name is read when the runtime starts: from here on the build alone sees it
+    torch.zeros(1, device="cuda")
+    aux, _, _ = _span("kept")
+    orb = _basis([(0, 0, np.zeros(3) + x, [0.8]) for x in (0.0, 1.0)], True)
+    mol = Molecule(["O"] * 2, np.array([[0.0, 0.0, 0.0], [0.0, 0.1, 2.1]]), "sto-3g")
+    got = []
+    for tool in (None, "none.so"):
+        if tool:
+            monkeypatch.setenv("ROCP_TOOL_LIBRARIES", tool)
+        c = _handle(orb, aux, mol, **spec)
+        assert c.nfit == c.naux and c.stats()["metric_cholesky"] == (not spec)
+        got.append(c.matrix(N.DFKS_BFIT, (4, c.nfit)).clone())
+        c.close()
+    assert torch.equal(*got)

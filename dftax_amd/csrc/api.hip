@@ -292,6 +292,11 @@ void pool_setup() {
 // on that event before its first use. At most a third of the device's memory
 // (and never more than 96 GB) is kept; any allocation that fails, large or
 // small, returns every kept block of its device to the pool and tries again.
+// A fresh block first gives back what is kept where it would leave less than
+// kHeadroom of the device free: the runtime allocates too (scratch of a queue's
+// kernels), takes nothing back from the library when that fails, and ends the process. Handles within 85 % of the device, 96 GB kept and the
+// pool's reserve would fill it: 512 requests at twice the load of one after another
+// ended so, and at that load itself 39 GB were left at the lowest.
 struct BigBlock {
   size_t bytes;
   int dev;
@@ -299,11 +304,13 @@ struct BigBlock {
 };
 constexpr size_t kCacheMin = size_t(8) << 20;
 constexpr size_t kCacheKeepMax = size_t(96) << 30;
+constexpr size_t kHeadroom = size_t(8) << 30;
 std::mutex g_cache_mu;
 std::map<void*, BigBlock> g_big_live;                // handed out
 std::vector<std::pair<void*, BigBlock>> g_big_free;  // kept for reuse
 std::map<int, size_t> g_big_free_bytes;              // kept bytes per device
 std::map<int, size_t> g_cache_keep;                  // keep limit per device
+std::map<int, size_t> g_big_pending;                 // bytes of fresh blocks on their way, per device
 
 size_t size_class(size_t b) {
   const int k = 63 - __builtin_clzll(b);
@@ -322,20 +329,24 @@ size_t cache_keep(int dev) {
   return keep;
 }
 
-// Returns every kept block of device dev to the pool. The blocks leave the
+// Returns kept blocks of device dev to the pool, largest first, until they hold
+// `need` bytes (all of them without one). The blocks leave the
 // list under the lock; the waits for their last users and the frees happen
 // after it is dropped, so other threads' allocations do not queue behind a
 // long kernel on another stream.
-void cache_release(int dev) {
+void cache_release(int dev, size_t need = SIZE_MAX) {
   std::vector<std::pair<void*, BigBlock>> out;
   {
     std::lock_guard<std::mutex> lk(g_cache_mu);
-    for (size_t i = 0; i < g_big_free.size();) {
+    std::stable_sort(g_big_free.begin(), g_big_free.end(),
+                     [](const auto& a, const auto& b) { return a.second.bytes > b.second.bytes; });
+    size_t got = 0;
+    for (size_t i = 0; i < g_big_free.size() && got < need;) {
       if (g_big_free[i].second.dev != dev) { ++i; continue; }
       out.push_back(g_big_free[i]);
+      got += g_big_free[i].second.bytes;
       g_big_free_bytes[dev] -= g_big_free[i].second.bytes;
-      g_big_free[i] = g_big_free.back();
-      g_big_free.pop_back();
+      g_big_free.erase(g_big_free.begin() + i);
     }
   }
   for (auto& f : out) {
@@ -354,6 +365,34 @@ void release_for_retry(int dev) {
   hipMemPool_t pool;
   if (hipDeviceGetDefaultMemPool(&pool, dev) == hipSuccess) (void)hipMemPoolTrimTo(pool, 0);
 }
+
+// A fresh block of device dev on its way: counted while it is allocated, so that threads that allocate at the same time
+// see each other, after room has been made for all of them
+struct Pending {
+  int dev;
+  size_t bytes;
+  Pending(int d, size_t b) : dev(d), bytes(b) {
+    size_t want = kHeadroom;
+    {
+      std::lock_guard<std::mutex> lk(g_cache_mu);
+      want += g_big_pending[dev] += bytes;
+    }
+    size_t fr = 0, tot = 0;
+    hipMemPool_t pool;
+    if (hipMemGetInfo(&fr, &tot) != hipSuccess || fr >= want ||
+        hipDeviceGetDefaultMemPool(&pool, dev) != hipSuccess)
+      return;
+    (void)hipMemPoolTrimTo(pool, 0);
+    if (hipMemGetInfo(&fr, &tot) != hipSuccess || fr >= want) return;
+    cache_release(dev, want - fr);
+    (void)hipStreamSynchronize(g_st);
+    (void)hipMemPoolTrimTo(pool, 0);
+  }
+  ~Pending() {
+    std::lock_guard<std::mutex> lk(g_cache_mu);
+    g_big_pending[dev] -= bytes;
+  }
+};
 
 void* big_alloc(size_t bytes) {
   const size_t cb = size_class(bytes);
@@ -374,10 +413,14 @@ void* big_alloc(size_t bytes) {
   }
   // the lock is not held across the allocation, which can take a second
   void* p = nullptr;
-  hipError_t e = hipMallocAsync(&p, cb, g_st);
-  if (e != hipSuccess) {
-    release_for_retry(dev);
+  hipError_t e;
+  {
+    const Pending pending(dev, cb);
     e = hipMallocAsync(&p, cb, g_st);
+    if (e != hipSuccess) {
+      release_for_retry(dev);
+      e = hipMallocAsync(&p, cb, g_st);
+    }
   }
   if (e != hipSuccess) fail(4, "hipMallocAsync of " + std::to_string(cb) + " bytes: " + hipGetErrorString(e));
   hipEvent_t ev = nullptr;

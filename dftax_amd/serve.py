@@ -276,6 +276,9 @@ def run_stream(n: int = 64, rates=(1.0, 2.0), *, seed: int = 0, slots: int = 16,
         arr = np.cumsum(gaps) - gaps[0]
         reqs = [Request(rid=k, mol=m, arrival=float(a)) for k, (m, a) in enumerate(zip(mols, arr))]
         srv.run(reqs, progress=progress)
+        for r in reqs:
+            if r.error:
+                say(f"request {r.rid} ({len(r.mol.symbols)} atoms) failed: {r.error}")
         st = latency_stats(reqs, alone)
         st["p99_over_isolated"] = st["p99_s"] / tau if st["p99_s"] else None
         st["p99_over_isolated_p99"] = st["p99_s"] / out["isolated_solve_s_p99"] if st["p99_s"] else None

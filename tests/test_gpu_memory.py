@@ -92,3 +92,41 @@ def test_mixed_build_takes_no_cholesky_work():
     after, _ = torch.cuda.mem_get_info(0)
     _say(f"taken by a build of {naux} fitting functions: {(before - after) / (8 * naux * naux):.2f} naux^2 words")
     assert 2 * 8 * naux * naux < before - after < 6 * 8 * naux * naux
+
+
+def test_fresh_blocks_leave_room_for_the_runtime():
+    """With 10.5 GB of the device free and more than that kept, a build that needs some 3.5 GB of fresh blocks gives kept
+    ones back: 8 GiB stay free for what the runtime itself allocates (a queue's scratch, which ends the process when
+    there is no room for it)."""
+    import torch
+    from dftax_amd import _native, water_cluster
+    from dftax_amd.basis import build_basis
+    from dftax_amd.ks import HipDFKS, HipSpec
+    from dftax_amd.xc import PBE0
+
+    def handle(n):
+        m = water_cluster((n, 1, 1), seed=1, basis="def2-tzvp")
+        return HipDFKS(*(build_basis(m.symbols, m.coords, b, spherical=True) for b in ("def2-tzvp", "even-tempered-jk")),
+                       m, np.zeros((1, 3)) + 1.0, np.zeros(1), PBE0(), m.nelectron, HipSpec(), chunk=None)
+
+    _native.release_memory(0)
+    handle(24).close()
+    torch.cuda.synchronize()
+    free, _ = torch.cuda.mem_get_info(0)
+    kept = _native.device_free(0) - free
+    _say(f"kept {kept / 1e9:.1f} GB, device free {free / 1e9:.1f} GB")
+    assert kept > 20e9
+    fill = torch.empty(free - int(10.5e9), dtype=torch.uint8, device="cuda")
+    try:
+        c = handle(12)
+        C = torch.eye(c.nao, 60, dtype=torch.float64, device="cuda")
+        E, F, _ = c.energy_fock_factored(C)
+        left, _ = torch.cuda.mem_get_info(0)
+        _say(f"device free beside the second handle {left / 1e9:.1f} GB")
+        assert bool(torch.isfinite(F).all())
+        assert left > (8 << 30) - (256 << 20)   # blocks under 8 MiB come on top
+        c.close()
+    finally:
+        del fill
+        torch.cuda.empty_cache()
+        _native.release_memory(0)

@@ -1129,12 +1129,14 @@ hipError_t launch_gemm_w8(const GemmArgs& g, double* C, const RowDot& rd, hipStr
 // the MFMA operand registers directly (two consecutive rows per 16-byte load,
 // 256-byte runs), each step's registers reloaded for the next 16 k as soon as
 // its products are issued; B is staged 16 k at a time in LDS in fragment order.
+// A last partial group stands after the loop: zeroing its A within the loop took 4 % (430 functions, 50 columns).
 // The tile is as wide as the factor (16 NJ), where the 128- and 160-wide tiles
 // of k_gemm_w8 pad: below about 64 columns the product is bound by reading A
 // once. K = 344, 40 columns ((H2O)_8 def2-TZVP): 0.26 ms = 3.4 TB/s, against
 // 0.53 (k_gemm), 0.60 (rocBLAS) and 0.65 ms; K = 1032, 48 columns: 5.2 against
-// 10.7 ms. Up to 80 columns a wavefront takes 64 rows, beyond them 32, which is where the registers end (K =
-// 602, 70 columns: 1.73 ms with 64 rows, 1.88 with 32). At 120 columns rocBLAS is ahead (12.7 against 14.2 ms).
+// 10.7 ms. Up to 80 columns a wavefront takes 64 rows, beyond them 32 (K = 602, 70 columns: 1.73 ms with 64
+// rows, 1.88 with 32), which two wavefronts a SIMD have registers for but at 80 columns (12 words spill), 128 (3), 144
+// (18) and 160 (39). At 120 columns rocBLAS is ahead (12.7 against 14.2 ms).
 template <int NJ>
 struct TTile {
   static constexpr int MI = NJ <= 5 ? 4 : 2, ROWS = 64 * MI;   // 16-row blocks per wavefront, rows per workgroup
@@ -1192,21 +1194,15 @@ __global__ __launch_bounds__(256, NJ <= 1 ? 4 : 2) void k_gemm_t(int64_t M, int 
     load_b(0);
 #pragma unroll
     for (int s = 0; s < 4; ++s) load_a(s, 0);
-    for (int k0 = 0, buf = 0; k0 < K; k0 += 16, buf ^= 1) {
-      double* sb = s_b[buf];
-      const bool in = k0 + bk < K;
+    // 16 k from the registers and sb, which the registers for the next 16 replace; TAIL: the last, partial group
+    const auto group = [&](int k0, double* sb, auto TAIL) __attribute__((always_inline)) {
+      constexpr bool tail = decltype(TAIL)::value;
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) sb[((bk >> 2) * NJ + j) * 64 + (bk & 3) * 16 + bi] = in ? b[j] : 0.0;
+      for (int j = 0; j < NJ; ++j)
+        sb[((bk >> 2) * NJ + j) * 64 + (bk & 3) * 16 + bi] = !tail || k0 + bk < K ? b[j] : 0.0;
       __syncthreads();     // the other buffer's readers passed the previous barrier
-      const int kn = min(k0 + 16, K - 1);      // the last step's reloads are not used
-      load_b(kn);
-      if (k0 + 16 > K) {   // past the end both operands are zero
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-          for (int p = 0; p < MP; ++p)
-            if (k0 + 4 * s + lk >= K) a[s][p] = dbl2u{0.0, 0.0};
-      }
+      const int kn = min(k0 + 16, K - 1);      // with K a multiple of 16 the last reloads are not used
+      if constexpr (!tail) load_b(kn);
       double bf[2][NJ];
 #pragma unroll
       for (int j = 0; j < NJ; ++j) bf[0][j] = sb[j * 64 + lane];
@@ -1221,17 +1217,28 @@ __global__ __launch_bounds__(256, NJ <= 1 ? 4 : 2) void k_gemm_t(int64_t M, int 
 #pragma unroll
           for (int j = 0; j < NJ; ++j)
             acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s][i >> 1][i & 1], bf[s & 1][j], acc[i][j], 0, 0, 0);
-        load_a(s, kn);
+        if constexpr (!tail) load_a(s, kn);
       }
+    };
+    int k0 = 0, buf = 0;
+    for (; k0 + 16 <= K; k0 += 16, buf ^= 1) group(k0, s_b[buf], std::false_type());
+    if (k0 < K) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int p = 0; p < MP; ++p)
+          if (k0 + 4 * s + lk >= K) a[s][p] = dbl2u{0.0, 0.0};   // past the end both operands are zero
+      group(k0, s_b[buf], std::true_type());
+    } else {
+      // keeps the reloads where they are issued: unused after the last step, they would be moved to the
+      // start of the next one, with nothing to hide them
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int p = 0; p < MP; ++p) asm volatile("" ::"v"(a[s][p]));
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) asm volatile("" ::"v"(b[j]));
     }
-    // keeps the reloads where they are issued: unused after the last step, they would be moved to the
-    // start of the next one, with nothing to hide them
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-      for (int p = 0; p < MP; ++p) asm volatile("" ::"v"(a[s][p]));
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) asm volatile("" ::"v"(b[j]));
   };
   if (m0 + ROWS <= M) product(std::true_type());
   else product(std::false_type());

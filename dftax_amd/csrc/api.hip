@@ -294,9 +294,10 @@ void pool_setup() {
 // small, returns every kept block of its device to the pool and tries again.
 // A fresh block first gives back what is kept where it would leave less than
 // kHeadroom of the device free: the runtime allocates too (scratch of a queue's
-// kernels), takes nothing back from the library when that fails, and ends the process. Handles within 85 % of the device, 96 GB kept and the
-// pool's reserve would fill it: 512 requests at twice the load of one after another
-// ended so, and at that load itself 39 GB were left at the lowest.
+// kernels), takes nothing back from the library when that fails, and ends the
+// process. Handles within 85 % of the device, 96 GB kept and the pool's reserve
+// would fill it: 512 requests at twice the load of one after another ended so, and
+// at once that load 27 to 40 GB are left at the lowest.
 struct BigBlock {
   size_t bytes;
   int dev;
@@ -1283,10 +1284,11 @@ void build_all(dfks_ctx* h, hipStream_t st) {
   RBCHK(rocblas_set_stream(rb_eig, s_eig));
   // true: V's inverse Cholesky factor is in mw.Lc (every eigenvalue above the cutoff)
   const auto chol_launch = [&](const double* V, hipStream_t s) {
-    // A handle with 32-bit products keeps the eigenvectors: their fitted functions are sorted by scale, which
-    // 32 bits need (water dimer with recomputed slabs: E off by 5.5e-3 Ha with C^-T, under 1e-3 with U w^-1/2;
-    // (H2O)_8 def2-TZVP with B kept: J off by 4.8e-4 against 2.2e-4). And the Lanczos kernel's partial
-    // sums end at 4 kLzParts.
+    // A handle with 32-bit products keeps the eigenvectors: with C^-T its Fock builds lose more. Largest error of J
+    // and that of E against FP64 with C^-T (with U w^-1/2), fitting shells sorted: B kept, (H2O)_4 def2-TZVP 3.2e-5
+    // (1.5e-5) and 0.9e-4 (1.7e-4) Ha, (H2O)_8 3.7e-5 (2.0e-5) and 2.7e-4 (1.1e-4), a tree of 6 heavy atoms 8.1e-5
+    // (3.7e-5) and 5.3e-4 (2.4e-4); slabs of 128, E of (H2O)_4 5.2e-3 (0.9e-3), of (H2O)_8 1.0e-2 (1.3e-3). An order by
+    // the factor's own pivots has not been tried. And the Lanczos kernel's partial sums end at 4 kLzParts.
     if (h->opt.precision == 1 || naux > 4 * kLzParts || !(h->opt.metric_cutoff >= 0.0)) return false;
     struct Work {
       double* p = nullptr;
@@ -1663,11 +1665,6 @@ void coulomb_recompute(dfks_ctx* h, hipStream_t st) {
   }
 }
 
-// FP64 exchange product T[m,Q,i] = sum_l B[l,m,Q] Cf[l,i], autotuned: the first
-// product of each (device, M, N, K) shape runs both candidates -- the library
-// kernel (128- or 160-wide N tiles, whichever pads less) and rocBLAS -- timed
-// with HIP events on the work stream, and the process keeps the faster one for
-// that shape. Both compute the same T to rounding.
 // Per-shape choice among the variants of a product. Tags and variants:
 //   0  FP64 exchange T = B^T C:      0 rocBLAS, 1 k_gemm, 2 k_gemm_w8, 3 k_gemm_t
 //   3  FP64 exchange K partials:     0 k_gemm, 1 k_gemm_w8, 2 k_gemm_nt (base 1)
@@ -1677,9 +1674,9 @@ void coulomb_recompute(dfks_ctx* h, hipStream_t st) {
 // The first call of a shape on a device times every variant with HIP events
 // and keeps the fastest; the output of that call is recomputed by the kept
 // variant when it is not the one that ran last, so every call of a shape
-// returns the kept variant's result. options.gemm 1, 2 and 3 force variant
+// returns the kept variant's result. options.gemm 1 to 4 force variant
 // gemm - 1 - base, clamped to the variants there are (gemm 2: k_gemm, 3: the
-// 8-wavefront tiles).
+// 8-wavefront tiles, 4: the last of each).
 std::mutex g_tune_mu;
 std::map<std::tuple<int, int, int64_t, int64_t, int64_t>, int> g_tune;
 
@@ -1734,8 +1731,8 @@ int tuned_product(dfks_ctx* h, int tag, int64_t d0, int64_t d1, int64_t d2, int 
 }
 
 // T = B^T C (nao*nfit x nc), FP64
-// Returns whether the gamma row terms of rd were produced with T (the
-// 8-wavefront kernel computes them in its epilogue).
+// Returns whether the gamma row terms of rd were produced with T (k_gemm_w8 and
+// k_gemm_t compute them in their epilogues).
 bool t_product(dfks_ctx* h, const double* C, int nc, const RowDot& rd, hipStream_t st) {
   const int nao = h->nao, nfit = h->nfit;
   const double one = 1.0, zero = 0.0;
@@ -1860,7 +1857,7 @@ void jk_factored(dfks_ctx* h, const double* Cf, const std::vector<double>& sgn, 
     }
     h->mark(kStExchangeGemm + 1, st);
     // gamma += sum_i s_i T_i c_i (timed with the exchange product K below); its row terms come
-    // with T from the 8-wavefront kernels, otherwise from a pass over T
+    // with T from k_gemm_w8, k_gemm_t and k_gemm_b3w8, otherwise from a pass over T
     if (rows_done)
       HIPCHK(launch_colsum(nao, nfit, h->d_gpart, h->d_gamma, 1, st));
     else if (mixed)

@@ -53,6 +53,8 @@ struct PairCls {
   // primitive pairs whose H is held at a time (18 KB where it is more than one), wavefronts per workgroup
   static constexpr int NPC = HSZ > 2304 ? 1 : (2304 / HSZ > 36 ? 36 : 2304 / HSZ);
   static constexpr int NW = NR * 16 > 2600 ? 2 : 4;
+  // wavefronts a SIMD. With two the accumulators, R's ladder and G do not all fit in (3,2,1), which spills 56 words,
+  // (2,1,4) 29, (3,0,4) 25, (3,1,2) 16, (2,2,2) 12, and 2 in (3,2,0) and the two-centre (4,0,3)
   static constexpr int OCC = MT * NM * 8 > 80 ? 1 : 2;
 };
 

@@ -15,6 +15,8 @@
 // def2-SVP: 6.6 ms for the Coulomb and the exchange term, 71 ms with a wavefront per task that
 // differentiated each integral (k_eri_grad in eri.hip, kept for cartesian spans with l >= 2 and for
 // more atoms than the LDS sums hold).
+// One wavefront a SIMD has registers for all but the widest classes: spilled words (3,3,4) 450, (3,3,3) 275, (3,2,4)
+// 199, (3,3,2) 104, (2,2,4) 102, (3,2,3) 85, (3,1,4) 68, (2,2,3) 7.
 // Reference: dftax/ks/forces.py:128-270 (jax.grad through eri3c_bucketed.py:290-426).
 #include <algorithm>
 #include <cstdint>

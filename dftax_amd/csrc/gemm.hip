@@ -845,14 +845,15 @@ static hipError_t launch_gemm_t(const GemmArgs& g, Out* C, int64_t ldc, int nspl
 // 16 bytes of a row: rows start on any 8 bytes
 typedef double dbl2u __attribute__((ext_vector_type(2), aligned(8)));
 
-// Split-K partial tiles of A B^T for K-contiguous operands (the exchange K = T T^T). 128 x 128 a workgroup,
-// 64 x 64 a wavefront, no LDS: a wavefront's fragments of 8 k are 64-byte runs of its rows, loaded from global
-// memory into registers while the 8 k before them multiply; what the wavefronts share comes from L1 and L2.
-// Two wavefronts a SIMD, and groups of 8 k rather than 16, so that sums and groups fit the registers without
-// copies. Workgroup x runs on XCD x % 8: an XCD takes whole splits, all tiles of a split before the next, so
-// their windows of A and B are read from HBM once. Bound by the matrix cores. 144 functions: 0.055 ms (8-wavefront
-// tiles 0.083, k_gemm 0.129); 465: 1.01 (1.42, 2.42); 602: 1.00 (1.03, 1.23); 1032: 8.07 (8.50, 9.25). Where a
-// round is left half empty the 8-wavefront tiles stay ahead (344 functions, 36,800 k: 0.151 against 0.192).
+// Split-K partial tiles of A B^T for K-contiguous operands (the exchange K = T T^T). 64 x 64 a wavefront, four tiles
+// that follow each other in the list (with sym the upper triangle's) a workgroup, no LDS: a wavefront's fragments of
+// 8 k are 64-byte runs of its rows, loaded from global memory into registers while the 8 k before them multiply; what
+// the wavefronts share comes from L1 and L2. Two wavefronts a SIMD, and groups of 8 k rather than 16, so that sums
+// and groups fit the registers without copies. Workgroup x runs on XCD x % 8: an XCD takes whole splits, all tiles of
+// a split before the next, so their windows of A and B are read from HBM once. Bound by the matrix cores. 144
+// functions: 0.055 ms (8-wavefront tiles 0.083, k_gemm 0.129); 465: 1.01 (1.42, 2.42); 602: 1.00 (1.03, 1.23); 1032:
+// 8.07 (8.50, 9.25). Where a round is left half empty the 8-wavefront tiles stay ahead (344 functions, 36,800 k:
+// 0.151 against 0.192).
 __global__ __launch_bounds__(256, 2) void k_gemm_nt(int M, int N, int64_t K, const double* __restrict__ A, int64_t lda,
                                                     const double* __restrict__ B, int64_t ldb, double* __restrict__ C,
                                                     int64_t split_stride, int64_t kchunk, int nsplit, int ntiles,
